@@ -406,17 +406,11 @@ typedef struct pq_contact {
 /* Kernel mapping of the contact path (no counterpart in parry; results are
  * identical for every setting).  Process-wide.
  *   epa_lanes_per_pair: lanes that run one pair's EPA together in the first EPA
- *       tier: 64 (one wave per pair), 32, 16, 8 or 4;
- *   epa_polytope: the first tier's polytope buffers: 0 = 32 vertices / 96 faces
- *       with the ConvexPolyhedra's vertices staged in LDS, 1 = the same without
- *       staging, 2 = 24 vertices / 64 faces, 3 = 32 vertices / 160 faces,
- *       4 = 48 vertices / 224 faces, all three without staging (less LDS per pair
- *       means more pairs resident; a pair whose polytope outgrows the buffers
- *       moves on to the one-wave-per-pair tiers);
- *   epa_schedule: with fewer than 64 lanes per pair, 1 = a wave takes its next
- *       pairs when all its groups are done, 2 = a group of lanes takes its next
- *       pair as soon as it is done with one, 0 = automatic: 1 for the
- *       TriMesh-shape contact (short EPA runs), 2 everywhere else.
+ *       tier: 64 (one wave per pair), 32, 16, 8 or 4, used when epa_schedule is 1
+ *       or 2;
+ *   epa_polytope: 0 to 4; the first tier's polytope has one size now (20
+ *       vertices, 64 faces), and every value selects it;
+ *   epa_schedule: 0 = automatic (8 lanes per pair), 1 and 2 = epa_lanes_per_pair.
  * The default is 16 lanes per pair with polytope 1 and schedule 0. */
 typedef struct pq_contact_tuning {
     uint32_t epa_lanes_per_pair;
@@ -428,7 +422,7 @@ int pq_contact_set_tuning(const pq_contact_tuning *tuning);
 /* Phase timing of the contact path, for measurement (no counterpart in parry).
  * While enabled (process-wide), every contact call records HIP events on its
  * own stream between its phases; pq_contact_phase_ms waits for the last call's
- * events and writes ms[0..4]: the GJK/dispatch kernel, the first EPA tier, the
+ * events and writes ms[0..4]: the GJK/dispatch kernel, the first two EPA tiers, the
  * 768-face tier, the 2048-face tier and the global-memory tier.  Calls that
  * overlap on several streams share the events; leave it off under graph capture. */
 int pq_contact_set_phase_timing(int enable);

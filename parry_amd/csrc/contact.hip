@@ -15,18 +15,19 @@
 //     in registers.  Pairs GJK finds intersecting are appended, with their
 //     final simplex, to an EPA queue (one atomic per wave: ballot + masked
 //     popcount give each lane its slot).
-// Stage 2 (one wave per queued pair): EPA (src/query/epa/epa3.rs:428-651) with
-//   the polytope -- vertices, faces, adjacency, the face heap (the same binary
-//   heap algorithm as Rust's BinaryHeap, so equal-distance faces pop in parry's
-//   order) and the silhouette stack -- in LDS.  The sequential algorithm runs
-//   identically on all 64 lanes; the ConvexPolyhedron support scans are split
-//   across the lanes and merged with a wave reduction that keeps parry's
-//   first-strict-maximum rule.  A pair whose polytope outgrows the LDS
-//   capacity is re-run by stage 3, the same code with large buffers in global
-//   memory.
+// Stage 2 (a group of lanes per queued pair): EPA (src/query/epa/epa3.rs:428-651)
+//   with the polytope in LDS, in three tiers: eight lanes per pair and 64 faces,
+//   sixteen lanes and 192 faces, a wave and 768 faces.  A pair that outgrows a
+//   tier's buffers goes on in the next one where it stopped.  The group's lanes
+//   share the support scans, pick the next face, test every face's visibility
+//   and build the new faces in parallel; the silhouette walk is serial.
+// Stage 3 (one wave per pair): the same with parry's heap of faces (the binary
+//   heap algorithm of Rust's BinaryHeap), 2048 faces in LDS, then 8192 in global
+//   memory, for the few pairs beyond 768 faces or with non-finite face distances.
 // Every contact is finished as contact_support_map_support_map (dist, point2,
 // normal2 in shape 2's frame) and Contact::transform_by_mut (contact.rs:171-176).
 #include <cstring>
+#include <type_traits>
 
 #include "contact_gjk.h"
 
@@ -72,13 +73,13 @@ __device__ __forceinline__ bool feature_map(ShapeRef &g, float &border) {
     }
     return false;
 }
-struct EpaItem {
+struct alignas(16) EpaItem {
     uint32_t pair;
-    uint32_t dim;
-    uint32_t mode;
-    uint32_t pad;
-    float v[4][9];  // point, orig1, orig2
+    uint32_t dim_mode;  // simplex dimension | mode << 8
+    uint32_t i, j;      // the pair's shapes
+    float v[4][9];      // point, orig1, orig2
 };
+__device__ __forceinline__ uint32_t item_mode(const EpaItem *it) { return it->dim_mode >> 8; }
 
 // Writes a contact record straight to its output slot (a local record copied
 // out afterwards would be kept in scratch memory).
@@ -133,10 +134,11 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// counters[0..3]: EPA queue length and the three overflow-list lengths;
-// counters[4..7]: the next list entry each EPA tier hands out;
-// counters[8]: continuation records taken by the first tier.
-constexpr uint32_t kNumCounters = 9;
+// counters[0..4]: EPA queue length and the four overflow-list lengths;
+// counters[5..9]: the next list entry each EPA tier hands out;
+// counters[10..11]: continuation records taken by the first and second tier.
+constexpr uint32_t kNumCounters = 12;
+constexpr uint32_t kTiers = 5;
 __global__ void reset_counters_kernel(uint32_t *counters) {
     if (threadIdx.x < kNumCounters) counters[threadIdx.x] = 0u;
 }
@@ -157,10 +159,12 @@ __global__ __launch_bounds__(kBlock) void contact_gjk_kernel(
     bool need_epa = false;
     uint32_t ball_mode = kPairSupportMaps;
     Simplex s;
-    uint32_t pair_id = 0;
+    uint32_t pair_id = 0, shape_i = 0, shape_j = 0;
     if (k < m) {
         pair_id = (uint32_t)k;
         const uint32_t i = pairs[2 * k], j = pairs[2 * k + 1];
+        shape_i = i;
+        shape_j = j;
         const iso pos1 = load_iso(poses + 7 * (size_t)i), pos2 = load_iso(poses + 7 * (size_t)j);
         const iso pos12 = iso_inv_mul(pos1, pos2);
         ShapeRef g1 = load_shape(rec, verts, i), g2 = load_shape(rec, verts, j);
@@ -315,8 +319,9 @@ __global__ __launch_bounds__(kBlock) void contact_gjk_kernel(
         if (need_epa) {
             EpaItem &it = queue[base + lanes_below(mask)];
             it.pair = pair_id;
-            it.dim = s.dim;
-            it.mode = ball_mode;
+            it.dim_mode = s.dim | (ball_mode << 8);
+            it.i = shape_i;
+            it.j = shape_j;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const Cso &v = s.v[q];
@@ -329,60 +334,8 @@ __global__ __launch_bounds__(kBlock) void contact_gjk_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Stage 2/3: EPA, G lanes per pair
+// Stage 2: EPA, a group of G lanes per pair
 // ---------------------------------------------------------------------------
-// The polytope lives in LDS in compact form: CSO points, faces (vertex and
-// neighbour indices, deleted flag, unit normal), the face heap and the
-// silhouette stacks.  The shape-space points orig1/orig2 of each CSO vertex
-// are only needed for the final witness points, so they go to a per-group
-// global buffer; a face's barycentric coordinates are recomputed (the same
-// projection as Face::new) when its witness points are built.
-// ConvexPolyhedra with at most this many vertices are staged in LDS for the
-// EPA support queries; larger ones are read from global memory.
-constexpr int kStagedVerts = 64;
-
-template <class I> struct EpaFaceT {
-    I pts[3];
-    I adj[3];
-    uint8_t deleted;
-    float n[3];
-};
-
-template <int V, int F, int H, int S, int K, class I, int SV> struct EpaState {
-    static constexpr int kV = V, kF = F, kH = H, kS = S, kK = K, kSV = SV;
-    using Idx = I;
-    using Face = EpaFaceT<I>;
-    float vp[V][3];
-    Face face[F];
-    I heap_id[H];
-    float heap_nd[H];
-    uint32_t sil[S];  // face | opp << 16
-    uint32_t stk[K];  // face | opp << 16
-    I dl[S];          // faces the current iteration deleted (undone if it cannot commit)
-    uint32_t xfer;    // a value one lane passes to its group
-    uint8_t vis[F];   // per face: can_be_seen_by the newest vertex, one bit per opposite vertex
-    float sv[2][SV > 0 ? SV : 1][3];  // both ConvexPolyhedra's vertices (local frames), if SV > 0
-};
-// LDS variant (~4.8 KB per pair) sized for the common case; a pair that
-// outgrows it re-runs with the large buffers in global memory, which have room
-// for parry's 100-iteration cap.
-using EpaSmall = EpaState<32, 96, 96, 32, 96, uint8_t, kStagedVerts>;
-// The same without staged support vertices, and a smaller one: less LDS per pair,
-// more pairs resident per CU (selected by pq_contact_tuning.epa_polytope).
-using EpaSmallUnstaged = EpaState<32, 96, 96, 32, 96, uint8_t, 0>;
-using EpaTiny = EpaState<24, 64, 64, 24, 64, uint8_t, 0>;
-// More faces and heap entries for the same vertices, and a larger polytope
-// still on byte ids: fewer pairs move on to the one-wave-per-pair tiers.
-using EpaSmallWide = EpaState<32, 160, 160, 32, 96, uint8_t, 0>;
-using EpaSmallLarge = EpaState<48, 224, 224, 48, 128, uint8_t, 0>;
-// One wave per pair, room for parry's 100 iterations (the vertex count) and for
-// the faces a long run creates: ~31 KB and ~81 KB of LDS.
-using EpaMedium = EpaState<112, 768, 768, 128, 512, uint16_t, kStagedVerts>;
-using EpaBig = EpaState<112, 2048, 2048, 128, 2048, uint16_t, kStagedVerts>;
-using EpaLarge = EpaState<112, 8192, 8192, 2048, 8192, uint16_t, 0>;
-static_assert(sizeof(EpaFaceT<uint8_t>) == 20, "compact LDS face record");
-constexpr uint32_t kOrigFloats = 6;  // orig1, orig2 per CSO vertex
-
 // The argmax reduction over a group of G consecutive lanes: largest value, then
 // lowest index (a total order, so any pairing of the lanes gives the same
 // winner).  Groups of up to 16 lanes exchange through DPP row permutations --
@@ -518,6 +471,7 @@ template <int G, class W> __device__ const float (*stage_shape(W *w, int slot, c
     return w->sv[slot];
 }
 
+constexpr uint32_t kOrigFloats = 6;  // orig1, orig2 per CSO vertex
 template <class W> __device__ __forceinline__ f3 vpt(const W *w, uint32_t i) {
     return f3{w->vp[i][0], w->vp[i][1], w->vp[i][2]};
 }
@@ -529,6 +483,815 @@ template <class W> __device__ __forceinline__ void vset(W *w, float *orig, uint3
     o[0] = c.o1.x; o[1] = c.o1.y; o[2] = c.o1.z;
     o[3] = c.o2.x; o[4] = c.o2.y; o[5] = c.o2.z;
 }
+
+enum : uint32_t { EPA_OK = 0, EPA_NONE = 1, EPA_OVERFLOW = 2, EPA_RUNNING = 3, EPA_POINT = 4, EPA_RESTART = 5 };
+
+// Barycentric coordinates of Face::new's projection (epa3.rs:96-118,
+// TrianglePointLocation::barycentric_coordinates); returns proj_inside.
+__device__ __forceinline__ bool face_bcoords(f3 pa, f3 pb, f3 pc, float bc[3]) {
+    Loc l;
+    bool inside;
+    const f3 proj = tri_origin(pa, pb, pc, l, inside);
+    bc[0] = bc[1] = bc[2] = 0.0f;
+    const float e = kEps * 100.0f;
+    if (l.kind == LOC_VERTEX) {
+        bc[0] = l.id == 0 ? 1.0f : 0.0f;
+        bc[1] = l.id == 1 ? 1.0f : 0.0f;
+        bc[2] = l.id == 2 ? 1.0f : 0.0f;
+        return inside || norm_sq3(proj) < e * e;
+    }
+    if (l.kind == LOC_EDGE) {  // edges (0,1), (1,2), (0,2)
+        bc[0] = l.id == 1 ? 0.0f : l.b0;
+        bc[1] = l.id == 0 ? l.b1 : (l.id == 1 ? l.b0 : 0.0f);
+        bc[2] = l.id == 0 ? 0.0f : l.b1;
+        return inside || norm_sq3(proj) < e * e;
+    }
+    if (l.kind == LOC_FACE) {
+        bc[0] = l.b0;
+        bc[1] = l.b1;
+        bc[2] = l.b2;
+        return true;
+    }
+    return false;
+}
+
+// ccw_face_normal (utils/ccw_face_normal.rs:19-27), zero if degenerate.
+__device__ __forceinline__ f3 ccw_normal(f3 pa, f3 pb, f3 pc) {
+    const f3 r = cross3(sub3(pb, pa), sub3(pc, pa));
+    const float sq = norm_sq3(r);
+    f3 n = f3{0.0f, 0.0f, 0.0f};
+    if (sq > kEps * kEps) n = div3(r, sqrtf(sq));
+    return n;
+}
+
+// The polytope of one pair in LDS.  A face is three vertex ids (8 bits each) with
+// its visibility bits and, where kMask is false, its deleted flag in one word,
+// and its three neighbours in another, so a step of the silhouette walk reads
+// one face with two loads.  The shape-space points orig1/orig2 of a CSO vertex
+// are only needed for the final witness points: they go to a per-group global
+// buffer, and the face's barycentric coordinates are recomputed there (the same
+// projection as Face::new).
+//
+// There is no heap.  parry's BinaryHeap pops the live face of largest key
+// (-distance); which one only depends on the heap's layout when two live faces
+// share the largest key.  So the next face is the maximum of key[] over the live
+// faces, taken by the group's lanes in parallel, and the heap itself is only
+// rebuilt when that maximum is not unique (lazy_replay): every push and pop so
+// far is known from the face ids, pops[] and nfs[].  On 20,695 mixed pairs the
+// maximum was shared in 0.1% of the iterations.
+template <int V, int F, int S, int K, class I, int SV> struct LazyState {
+    static constexpr int kV = V, kF = F, kS = S, kK = K, kSV = SV;
+    static constexpr bool kMask = F <= 64;  // deleted flags in a 64-bit register mask
+    static constexpr uint32_t kShift = sizeof(I) == 1 ? 8u : 16u;
+    using Idx = I;
+    using Entry = std::conditional_t<sizeof(I) == 1, uint16_t, uint32_t>;
+    alignas(8) I adj[F][4];
+    uint32_t px[F];  // vertices; bits 24-26: can_be_seen_by the newest vertex per opposite vertex; 27: deleted
+    float key[F];    // FaceId's neg_dist, -inf for a face that was not pushed
+    float n[F][3];
+    float vp[V][3];
+    float sv[SV > 0 ? 2 : 1][SV > 0 ? SV : 1][3];  // both ConvexPolyhedra's vertices (local frames), if SV > 0
+    Entry sil[S];              // face | opp << kShift
+    Entry stk[K];              // face | point << kShift
+    I dl[kMask ? 1 : S];       // faces the current iteration deleted (undone if it cannot commit)
+    I hid[F];                  // the heap's face ids, when it is rebuilt
+    I pops[V], nfs[V];         // per iteration: the face it popped, and the number of faces before it
+};
+constexpr uint32_t kDeadBit = 1u << 27;
+
+
+struct LazyRegs {
+    uint32_t nv, nf, best_id, niter;
+    float max_dist, old_dist;
+    uint64_t dead;  // kMask: the deleted faces
+    // the rebuilt heap: its length, the iterations and faces it has taken in
+    uint32_t hlen, hiter, hnf;
+};
+
+template <class W> __device__ __forceinline__ bool face_dead(const W *w, const LazyRegs &r, uint32_t f, uint32_t x) {
+    if constexpr (W::kMask) return ((r.dead >> f) & 1ull) != 0ull;
+    return (x & kDeadBit) != 0u;
+}
+// The three neighbours of a face, kShift bits each.
+template <class W> __device__ __forceinline__ auto face_adj(const W *w, uint32_t f) {
+    if constexpr (sizeof(typename W::Idx) == 1)
+        return *reinterpret_cast<const uint32_t *>(w->adj[f]);
+    else
+        return *reinterpret_cast<const uint64_t *>(w->adj[f]);
+}
+template <class W, class A> __device__ __forceinline__ uint32_t adj_at(A a, uint32_t k) {
+    return (uint32_t)(a >> (W::kShift * k)) & ((1u << W::kShift) - 1u);
+}
+__device__ __forceinline__ uint32_t pt_at(uint32_t x, uint32_t k) { return (x >> (8u * k)) & 0xffu; }
+
+__device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The largest value of a group's lanes (no NaN), in every lane of the group.
+template <int CTRL> __device__ __forceinline__ float max_dpp(float v) {
+    return fmaxf(v, __uint_as_float(dpp_get<CTRL>(__float_as_uint(v))));
+}
+template <int G> __device__ __forceinline__ float group_max(float v) {
+    if constexpr (G >= 16) v = max_dpp<kDppRowMirror>(v);
+    if constexpr (G >= 8) v = max_dpp<kDppRowHalfMirror>(v);
+    v = max_dpp<kDppQuadXor2>(v);
+    v = max_dpp<kDppQuadXor1>(v);
+    if constexpr (G >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
+    if constexpr (G >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+// The bits of a wave ballot that belong to the caller's group.
+template <int G> __device__ __forceinline__ uint64_t group_ballot(bool p) {
+    const uint32_t gbase = __lane_id() & ~(uint32_t)(G - 1);
+    return (__ballot(p) >> gbase) & (G >= 64 ? ~0ull : ((1ull << (G & 63)) - 1ull));
+}
+
+// Face::new (epa3.rs:96-118) by one lane; returns proj_inside.
+template <class W>
+__device__ __forceinline__ bool lazy_face(W *w, uint32_t f, uint32_t a, uint32_t b, uint32_t c, uint32_t j0,
+                                          uint32_t j1, uint32_t j2, f3 &n, f3 &pa) {
+    using I = typename W::Idx;
+    w->px[f] = a | (b << 8) | (c << 16);
+    w->adj[f][0] = (I)j0;
+    w->adj[f][1] = (I)j1;
+    w->adj[f][2] = (I)j2;
+    pa = vpt(w, a);
+    const f3 pb = vpt(w, b), pc = vpt(w, c);
+    float bc[3];
+    const bool in = face_bcoords(pa, pb, pc, bc);
+    n = ccw_normal(pa, pb, pc);
+    w->n[f][0] = n.x;
+    w->n[f][1] = n.y;
+    w->n[f][2] = n.z;
+    return in;
+}
+
+// Face::closest_points (epa3.rs:120-130).
+template <class W> __device__ void lazy_points(const W *w, const float *orig, uint32_t f, f3 &p1, f3 &p2, f3 &n) {
+    const uint32_t x = w->px[f];
+    float bc[3];
+    face_bcoords(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)), bc);
+    f3 o1[3], o2[3];
+    for (int q = 0; q < 3; ++q) {
+        const float *o = orig + kOrigFloats * pt_at(x, q);
+        o1[q] = f3{o[0], o[1], o[2]};
+        o2[q] = f3{o[3], o[4], o[5]};
+    }
+    p1 = add3(add3(mul3(o1[0], bc[0]), mul3(o1[1], bc[1])), mul3(o1[2], bc[2]));
+    p2 = add3(add3(mul3(o2[0], bc[0]), mul3(o2[1], bc[1])), mul3(o2[2], bc[2]));
+    n = f3{w->n[f][0], w->n[f][1], w->n[f][2]};
+}
+
+// BinaryHeap<FaceId> over face ids (max-heap on key[]; equal keys compare Equal),
+// with std's sift_up / sift_down_to_bottom so equal keys pop in parry's order.
+template <class W> __device__ __forceinline__ void heap_sift_up(W *w, uint32_t pos) {
+    const uint32_t id = w->hid[pos];
+    const float nd = w->key[id];
+    while (pos > 0) {
+        const uint32_t parent = (pos - 1) / 2, pid = w->hid[parent];
+        if (nd <= w->key[pid]) break;
+        w->hid[pos] = (typename W::Idx)pid;
+        pos = parent;
+    }
+    w->hid[pos] = (typename W::Idx)id;
+}
+template <class W> __device__ __forceinline__ void heap_pop(W *w, uint32_t &len) {
+    --len;
+    if (len == 0) return;
+    const uint32_t id = w->hid[len];
+    uint32_t pos = 0, child = 1;
+    while (child + 2 <= len) {
+        uint32_t cid = w->hid[child];
+        const uint32_t rid = w->hid[child + 1];
+        if (w->key[cid] <= w->key[rid]) {
+            ++child;
+            cid = rid;
+        }
+        w->hid[pos] = (typename W::Idx)cid;
+        pos = child;
+        child = 2 * pos + 1;
+    }
+    if (child == len - 1) {
+        w->hid[pos] = w->hid[child];
+        pos = child;
+    }
+    w->hid[pos] = (typename W::Idx)id;
+    heap_sift_up(w, pos);
+}
+// The face parry's heap pops next when several live faces share the largest key:
+// brings the heap up to date with every push and pop so far, in parry's order
+// (each iteration pops until its face, deleted faces included, then pushes its
+// new faces by id), then pops the deleted faces at the top.  Run by all lanes of
+// the group with the same values.  Every push and pop is replayed once per pair.
+constexpr uint32_t kNoFace = 0xffffffffu;
+template <class W> __device__ uint32_t lazy_replay(W *w, LazyRegs &r) {
+    for (;;) {
+        const bool now = r.hiter == r.niter;
+        const uint32_t upto = now ? r.nf : w->nfs[r.hiter];
+        for (; r.hnf < upto; ++r.hnf)
+            if (w->key[r.hnf] != -INFINITY) {
+                w->hid[r.hlen] = (typename W::Idx)r.hnf;
+                heap_sift_up(w, r.hlen++);
+            }
+        if (now) break;
+        const uint32_t until = w->pops[r.hiter];
+        uint32_t id = kNoFace;
+        while (r.hlen != 0 && id != until) {
+            id = w->hid[0];
+            heap_pop(w, r.hlen);
+        }
+        ++r.hiter;
+    }
+    while (r.hlen != 0) {
+        const uint32_t id = w->hid[0];
+        if (!face_dead(w, r, id, w->px[id])) return id;
+        heap_pop(w, r.hlen);
+    }
+    return kNoFace;  // not reached: a live pushed face is in the heap
+}
+
+// A polytope at the start of an iteration, handed to the next tier so that the
+// pair continues where it stopped instead of starting over.
+template <int V, int F> struct EpaRec {
+    uint32_t nv, nf, best_id, niter;
+    float max_dist, old_dist;
+    uint32_t pad[2];
+    float vp[V][3];
+    float orig[V][6];
+    uint32_t px[F];   // with kDeadBit
+    uint32_t adj[F];  // 8 bits each
+    float key[F];
+    uint8_t pops[V], nfs[V];
+};
+constexpr uint32_t kNoCont = 0xffffffffu;
+// Where a tier writes the polytopes it hands on.
+template <class R> struct RecSink {
+    R *recs;
+    uint32_t *count;
+    uint32_t cap;
+};
+
+template <int G, class W, class R>
+__device__ uint32_t lazy_export(const W *w, const float *orig, const RecSink<R> &sink, const LazyRegs &r) {
+    static_assert(sizeof(typename W::Idx) == 1, "records hold byte ids");
+    const uint32_t sub = __lane_id() % G;
+    uint32_t ci = 0;
+    if (sub == 0) ci = atomicAdd(sink.count, 1u);
+    ci = (uint32_t)__shfl((int)ci, 0, G);
+    if (ci >= sink.cap) return kNoCont;
+    // orig rows were written to global memory by this wave; the group's lanes
+    // read each other's rows below
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    R *o = sink.recs + ci;
+    if (sub == 0) {
+        o->nv = r.nv;
+        o->nf = r.nf;
+        o->best_id = r.best_id;
+        o->niter = r.niter;
+        o->max_dist = r.max_dist;
+        o->old_dist = r.old_dist;
+    }
+    for (uint32_t k = sub; k < r.nv; k += G) {
+        for (int q = 0; q < 3; ++q) o->vp[k][q] = w->vp[k][q];
+        for (int q = 0; q < 6; ++q) o->orig[k][q] = orig[kOrigFloats * k + q];
+    }
+    for (uint32_t k = sub; k < r.nf; k += G) {
+        const uint32_t x = w->px[k];
+        o->px[k] = (x & 0x00ffffffu) | (face_dead(w, r, k, x) ? kDeadBit : 0u);
+        o->adj[k] = face_adj(w, k);
+        o->key[k] = w->key[k];
+    }
+    for (uint32_t k = sub; k < r.niter; k += G) {
+        o->pops[k] = (uint8_t)w->pops[k];
+        o->nfs[k] = (uint8_t)w->nfs[k];
+    }
+    return ci;
+}
+
+// Loads a record into the group's polytope; face normals are recomputed from the
+// vertices exactly as Face::new computed them.
+template <int G, class W, class R> __device__ void lazy_import(W *w, float *orig, const R *o, LazyRegs &r) {
+    static_assert(!W::kMask, "a tier that continues keeps its deleted flags in LDS");
+    using I = typename W::Idx;
+    const uint32_t sub = __lane_id() % G;
+    r.nv = o->nv;
+    r.nf = o->nf;
+    r.best_id = o->best_id;
+    r.niter = o->niter;
+    r.max_dist = o->max_dist;
+    r.old_dist = o->old_dist;
+    for (uint32_t k = sub; k < r.nv; k += G) {
+        for (int q = 0; q < 3; ++q) w->vp[k][q] = o->vp[k][q];
+        for (int q = 0; q < 6; ++q) orig[kOrigFloats * k + q] = o->orig[k][q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t k = sub; k < r.nf; k += G) {
+        const uint32_t x = o->px[k], a = o->adj[k];
+        w->px[k] = x;
+        for (int q = 0; q < 3; ++q) w->adj[k][q] = (I)((a >> (8 * q)) & 0xffu);
+        w->key[k] = o->key[k];
+        const f3 nn = ccw_normal(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)));
+        w->n[k][0] = nn.x;
+        w->n[k][1] = nn.y;
+        w->n[k][2] = nn.z;
+    }
+    for (uint32_t k = sub; k < r.niter; k += G) {
+        w->pops[k] = (I)o->pops[k];
+        w->nfs[k] = (I)o->nfs[k];
+    }
+    lds_order();
+}
+
+// The EPA problem of a queued pair (contact_support_map_support_map.rs:60-76):
+// its two shapes (their feature maps in kPairFeatureMaps mode) and relative pose,
+// or, for a Ball, the other shape against the ball centre
+// (point_support_map.rs:39-49).
+struct EpaProblem {
+    iso pos;
+    ShapeRef a, b;
+};
+
+__device__ EpaProblem epa_problem(const ShapeRecord *rec, const float4 *verts, const float *poses, const EpaItem *it) {
+    const uint32_t i = it->i, j = it->j;
+    const iso pos1 = load_iso(poses + 7 * (size_t)i), pos2 = load_iso(poses + 7 * (size_t)j);
+    const iso pos12 = iso_inv_mul(pos1, pos2);
+    ShapeRef g1 = load_shape(rec, verts, i), g2 = load_shape(rec, verts, j);
+    const uint32_t mode = item_mode(it);
+    if (mode == kPairFeatureMaps) {
+        float br;
+        (void)feature_map(g1, br);
+        (void)feature_map(g2, br);
+    }
+    if (is_ball_mode(mode)) {
+        if (mode == kBallFirst) return EpaProblem{point_proj_iso(iso_inverse(pos12).t), g2, origin_shape()};
+        return EpaProblem{point_proj_iso(pos12.t), g1, origin_shape()};
+    }
+    return EpaProblem{pos12, g1, g2};
+}
+
+// EPA::closest_points (epa3.rs:428-651) for one pair by a group of G lanes, one
+// iteration at a time: lazy_begin, then lazy_step until it returns a result.
+// Results: EPA_OK (the answer is face r.best_id), EPA_POINT (a simplex of
+// dimension 0), EPA_NONE, EPA_OVERFLOW (the polytope outgrew this tier's buffers
+// and is as it was at the start of the iteration), EPA_RESTART (a face key the
+// maximum cannot order -- NaN or -inf -- which the heap tiers handle).
+template <int G, class W, class R>
+__device__ uint32_t lazy_begin(W *w, float *orig, const EpaProblem &pr, const EpaItem *it, const R *resume, Staged &st,
+                               LazyRegs &r) {
+    st = Staged{stage_shape<G>(w, 0, pr.a), stage_shape<G>(w, 1, pr.b)};
+    lds_order();  // the staged vertices, before any lane reads another lane's entries
+    r = LazyRegs{0, 0, 0, 0, kFltMax, 0.0f, 0ull, 0, 0, 0};
+    if constexpr (!W::kMask) {
+        if (resume) {
+            lazy_import<G>(w, orig, resume, r);
+            return EPA_RUNNING;
+        }
+    }
+    const uint32_t dim = it->dim_mode & 0xffu;
+    if (dim == 0) return EPA_POINT;
+    f3 pv[4];
+    for (int i = 0; i < 4; ++i) pv[i] = f3{it->v[i][0], it->v[i][1], it->v[i][2]};
+    // a tetrahedron of the wrong orientation swaps its vertices 1 and 2
+    const bool swap = dim == 3 && dot3(cross3(sub3(pv[1], pv[0]), sub3(pv[2], pv[0])), sub3(pv[3], pv[0])) > 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        if (i > dim) break;
+        const uint32_t from = swap && i == 1 ? 2u : (swap && i == 2 ? 1u : i);
+        for (int q = 0; q < 3; ++q) w->vp[i][q] = it->v[from][q];
+        for (int q = 0; q < 6; ++q) orig[kOrigFloats * i + q] = it->v[from][3 + q];
+    }
+    r.nv = dim + 1;
+    const uint32_t sub = __lane_id() % G;
+    if (dim == 1) {
+        // orthonormal_subspace_basis([dpt]): first vector a x dpt
+        const f3 dpt = sub3(pv[1], pv[0]);
+        f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.0f, -dpt.x} : f3{0.0f, -dpt.z, dpt.y};
+        a = div3(a, sqrtf(norm_sq3(a)));
+        vset(w, orig, 2, group_cso<G>(pr.pos, pr.a, pr.b, st, cross3(a, dpt)));
+        r.nv = 3;
+    }
+    lds_order();
+    // The first faces, one per lane: (0,1,2) (1,3,2) (0,2,3) (0,3,1) of a
+    // tetrahedron (epa3.rs:459-500), both sides of a triangle otherwise.
+    r.nf = dim == 3 ? 4u : 2u;
+    bool in = false, bad = false, weird = false;
+    if (sub < r.nf) {
+        uint32_t pts, adj;
+        if (dim == 3) {
+            pts = sub == 0 ? 0x020100u : (sub == 1 ? 0x020301u : (sub == 2 ? 0x030200u : 0x010300u));
+            adj = sub == 0 ? 0x020103u : (sub == 1 ? 0x000203u : (sub == 2 ? 0x030100u : 0x000102u));
+        } else {
+            pts = sub == 0 ? 0x020100u : 0x010200u;
+            adj = sub == 0 ? 0x010101u : 0x000000u;
+        }
+        f3 n, pa;
+        in = lazy_face(w, sub, pt_at(pts, 0), pt_at(pts, 1), pt_at(pts, 2), pt_at(adj, 0), pt_at(adj, 1),
+                       pt_at(adj, 2), n, pa);
+        float k = 0.0f;
+        if (dim == 3) {
+            const float dist = dot3(n, vpt(w, sub));  // vertex `sub`, as parry takes it
+            bad = in && -dist > kEpsTol;              // FaceId::new -> None
+            weird = in && !(fabsf(dist) <= kFltMax);
+            k = in ? -dist : -INFINITY;
+        }
+        w->key[sub] = k;
+    }
+    lds_order();
+    if (dim == 3) {
+        if (group_ballot<G>(bad) != 0ull || group_ballot<G>(in) == 0ull) return EPA_NONE;
+        if (group_ballot<G>(weird) != 0ull) return EPA_RESTART;
+    }
+    return EPA_RUNNING;
+}
+
+// One EPA iteration (the body of the loop of epa3.rs:499-647).
+template <int G, class W>
+__device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Staged &st, LazyRegs &r) {
+    using I = typename W::Idx;
+    using E = typename W::Entry;
+    constexpr uint32_t kIdMask = (1u << W::kShift) - 1u;
+    const float eps_tol = kEps * 100.0f;
+    const uint32_t sub = __lane_id() % G;
+    // The live face of largest key.
+    uint32_t fid;
+    float fkey;
+    {
+        float kb = -INFINITY;
+        uint32_t ib = 0;
+        bool dup = false;
+#pragma unroll 4
+        for (uint32_t f = sub; f < r.nf; f += G) {
+            float k = w->key[f];
+            const uint32_t x = W::kMask ? 0u : w->px[f];
+            k = face_dead(w, r, f, x) ? -INFINITY : k;
+            dup = k > kb ? false : (k == kb ? true : dup);
+            ib = k > kb ? f : ib;
+            kb = fmaxf(k, kb);
+        }
+        fkey = group_max<G>(kb);
+        if (fkey == -INFINITY) return EPA_OK;  // parry's heap is empty
+        const uint64_t top = group_ballot<G>(kb == fkey);
+        const uint64_t twice = group_ballot<G>(kb == fkey && dup);
+        fid = (uint32_t)__shfl((int)ib, __builtin_ctzll(top), G);
+        if (twice != 0ull || (top & (top - 1ull)) != 0ull) {
+            fid = lazy_replay(w, r);
+            if (fid == kNoFace) return EPA_RESTART;
+        }
+    }
+    const uint32_t fx = w->px[fid];
+    const auto fadj = face_adj(w, fid);
+    const f3 fn = f3{w->n[fid][0], w->n[fid][1], w->n[fid][2]};
+    const Cso c = group_cso<G>(pr.pos, pr.a, pr.b, st, fn);
+    const float cand = dot3(c.p, fn);
+    uint32_t best_t = r.niter == 0 ? fid : r.best_id;  // the heap's first top is parry's first best face
+    float max_t = r.max_dist;
+    if (cand < max_t) {
+        best_t = fid;
+        max_t = cand;
+    }
+    const float curr_dist = -fkey;
+    if (max_t - curr_dist < eps_tol || (fabsf(curr_dist - r.old_dist) < kEps && cand < max_t)) {
+        r.best_id = best_t;
+        return EPA_OK;
+    }
+    if (r.nv >= (uint32_t)W::kV) return EPA_OVERFLOW;
+    const uint32_t sp = r.nv;  // counted when the iteration commits
+    vset(w, orig, sp, c);
+    const uint64_t dead0 = r.dead;
+    if constexpr (W::kMask)
+        r.dead |= 1ull << fid;
+    else
+        w->px[fid] = fx | kDeadBit;
+    lds_order();
+    // Face::can_be_seen_by (epa3.rs:153-166) of every face from the new vertex,
+    // for each of the three opposite vertices, by the group's lanes in parallel;
+    // the depth-first walk below only reads the bits.  Deleted faces get bits too
+    // (the walk never reads them): with no branch in the body, the loads of
+    // consecutive faces overlap.
+    {
+        const float E2 = kEps * 100.0f;
+#pragma unroll 2
+        for (uint32_t f = sub; f < r.nf; f += G) {
+            const uint32_t x = w->px[f];
+            const f3 q0 = vpt(w, pt_at(x, 0)), q1 = vpt(w, pt_at(x, 1)), q2 = vpt(w, pt_at(x, 2));
+            const f3 fnn = f3{w->n[f][0], w->n[f][1], w->n[f][2]};
+            const f3 qs[3] = {q0, q1, q2};
+            uint32_t bits = 0;
+#pragma unroll
+            for (int opp = 0; opp < 3; ++opp) {
+                const f3 p0 = qs[opp], p1 = qs[(opp + 1) % 3], p2 = qs[(opp + 2) % 3];
+                const bool front = dot3(sub3(c.p, p0), fnn) >= -kEpsTol;
+                const bool flat = norm_sq3(cross3(sub3(p2, p1), sub3(c.p, p1))) <= E2 * E2;  // is_affinely_dependent
+                bits |= (uint32_t)(front | flat) << opp;
+            }
+            reinterpret_cast<uint8_t *>(&w->px[f])[3] = (uint8_t)(bits | ((x >> 24) & (kDeadBit >> 24)));
+        }
+    }
+    lds_order();
+    // compute_silhouette (epa3.rs:653-675) for the three neighbours in order
+    // adj[0], adj[1], adj[2]; a visible face recurses into adj[(opp + 2) % 3],
+    // then adj[opp].  The recursion is an explicit stack of (face, the point its
+    // opposite vertex follows) whose top entry lives in a register.  A step is one
+    // read of the visited face, and both ways on (into a deleted face's first far
+    // neighbour, or back to the stack's top) end in that same read, so the groups
+    // of a wave take their steps together.
+    uint32_t ns = 0, ndel = 0, depth = 2;
+    uint32_t cur = adj_at<W>(fadj, 0) | (pt_at(fx, 0) << W::kShift);
+    uint32_t top = adj_at<W>(fadj, 1) | (pt_at(fx, 1) << W::kShift);
+    w->stk[0] = (E)(adj_at<W>(fadj, 2) | (pt_at(fx, 2) << W::kShift));
+    bool room = true;
+    for (;;) {
+        const uint32_t id = cur & kIdMask, pt = cur >> W::kShift;
+        const uint32_t x = w->px[id];
+        const auto a = face_adj(w, id);
+        const uint32_t below = w->stk[depth > 2u ? depth - 2u : 0u];
+        const uint32_t opp = pt_at(x, 0) == pt ? 1u : (pt_at(x, 1) == pt ? 2u : 0u);  // next_ccw_pt_id
+        const bool live = !face_dead(w, r, id, x);
+        const bool vis = ((x >> (24u + opp)) & 1u) != 0u;
+        const bool del = live && vis;
+        if (live && !vis) {
+            if (ns >= (uint32_t)W::kS) {
+                room = false;
+                break;
+            }
+            w->sil[ns++] = (E)(id | (opp << W::kShift));
+        }
+        if (!del && depth == 0) break;
+        if (del) {
+            if (depth > (uint32_t)W::kK || (!W::kMask && ndel >= (uint32_t)W::kS)) {
+                room = false;
+                break;
+            }
+            if constexpr (W::kMask) {
+                r.dead |= 1ull << id;
+            } else {
+                w->dl[ndel++] = (I)id;
+                w->px[id] = x | kDeadBit;
+            }
+            const uint32_t k1 = opp == 0u ? 2u : opp - 1u;  // (opp + 2) % 3
+            if (depth > 0) w->stk[depth - 1] = (E)top;
+            top = adj_at<W>(a, opp) | (pt_at(x, opp) << W::kShift);
+            ++depth;
+            cur = adj_at<W>(a, k1) | (pt_at(x, k1) << W::kShift);
+        } else {
+            cur = top;
+            top = below;
+            --depth;
+        }
+    }
+    if (room && ns == 0) return EPA_NONE;
+    // Room for the new faces: at most one per silhouette edge.
+    const uint32_t first_new = r.nf;
+    if (!room || first_new + ns > (uint32_t)W::kF) {
+        if constexpr (W::kMask) {
+            r.dead = dead0;
+        } else {
+            for (uint32_t k = 0; k < ndel; ++k) w->px[w->dl[k]] &= ~kDeadBit;
+            w->px[fid] &= ~kDeadBit;
+            lds_order();
+        }
+        return EPA_OVERFLOW;
+    }
+    w->pops[r.niter] = (I)fid;
+    w->nfs[r.niter] = (I)first_new;
+    ++r.nv;
+    r.best_id = best_t;
+    r.max_dist = max_t;
+    r.old_dist = curr_dist;
+    lds_order();
+    // The new faces (epa3.rs:598-626), G silhouette edges at a time, one per
+    // lane.  The edges whose face is still live get consecutive ids in
+    // silhouette order (a ballot gives each its rank), and each lane builds its
+    // edge's face (Face::new reads vertex positions only, and each edge rewrites
+    // its own adjacency slot).  Parry's loop returns at the first new face that
+    // ends EPA, whose heap pushes before that would be discarded anyway.
+    const uint64_t lower = (1ull << sub) - 1ull;
+    uint32_t n_alive = 0;
+    for (uint32_t c0 = 0; c0 < ns; c0 += G) {
+        const uint32_t q = c0 + sub;
+        uint32_t e = 0, ex = 0;
+        bool alive = false;
+        if (q < ns) {
+            e = w->sil[q];
+            ex = w->px[e & kIdMask];
+            alive = !face_dead(w, r, e & kIdMask, ex);
+        }
+        const uint64_t am = group_ballot<G>(alive);
+        const uint32_t new_id = first_new + n_alive + (uint32_t)__popcll(am & lower);
+        bool in = false;
+        float dist = 0.0f;
+        if (alive) {
+            const uint32_t ef = e & kIdMask, opp = e >> W::kShift;
+            const uint32_t k1 = opp == 0u ? 2u : opp - 1u, k2 = opp == 2u ? 0u : opp + 1u;
+            f3 n, pa;
+            in = lazy_face(w, new_id, pt_at(ex, k1), pt_at(ex, k2), sp, ef, new_id + 1, new_id - 1, n, pa);
+            w->adj[ef][k2] = (I)new_id;
+            if (in) dist = dot3(n, pa);
+            w->key[new_id] = in ? -dist : -INFINITY;
+        }
+        n_alive += (uint32_t)__popcll(am);
+        const bool closer = in && dist < curr_dist;
+        const uint64_t stop_m = group_ballot<G>(closer || (in && -dist > kEpsTol));
+        if (stop_m != 0ull) {
+            if ((group_ballot<G>(closer) >> __builtin_ctzll(stop_m)) & 1ull) {
+                r.best_id = fid;  // the popped face is the answer
+                return EPA_OK;
+            }
+            return EPA_NONE;  // FaceId::new -> None
+        }
+        if (group_ballot<G>(in && !(fabsf(dist) <= kFltMax)) != 0ull) return EPA_RESTART;
+    }
+    lds_order();
+    r.nf = first_new + n_alive;
+    if (first_new == r.nf) return EPA_NONE;
+    w->adj[first_new][2] = (I)(r.nf - 1);
+    w->adj[r.nf - 1][1] = (I)first_new;
+    lds_order();
+    ++r.niter;
+    return r.niter > 100 ? EPA_OK : EPA_RUNNING;  // parry's iteration cap
+}
+
+// Writes the result of a queued pair's EPA (one lane per pair): the contact, or
+// the pair's entry in the next tier's list if it moves on.
+__device__ void epa_finish(const ShapeRecord *rec, const float4 *verts, const float *poses, float prediction,
+                           const EpaItem *it, uint32_t st, f3 p1, f3 p2, f3 n, uint32_t ei, uint32_t cont,
+                           DevContact *out, uint32_t *iters, uint32_t *overflow_list, uint32_t *overflow_cont,
+                           uint32_t *overflow_count, uint32_t slot) {
+    const uint32_t k = it->pair;
+    if (st == EPA_OVERFLOW) {
+        if (overflow_list) {
+            const uint32_t pos = atomicAdd(overflow_count, 1u);
+            overflow_list[pos] = slot;
+            if (overflow_cont) overflow_cont[pos] = cont;
+        } else {
+            out[k] = no_contact(kUnsupportedPair);  // cannot happen with the large buffers
+        }
+        return;
+    }
+    const uint32_t i = it->i, j = it->j;
+    const iso pos1 = load_iso(poses + 7 * (size_t)i), pos2 = load_iso(poses + 7 * (size_t)j);
+    const iso pos12 = iso_inv_mul(pos1, pos2);
+    const uint32_t mode = item_mode(it);
+    if (is_ball_mode(mode)) {
+        // the Ball-vs-convex contact from the projection of the ball centre
+        const iso pb = mode == kBallFirst ? iso_inverse(pos12) : pos12;
+        const float radius = rec[mode == kBallFirst ? i : j].param[0];
+        const PointProj proj{true, st == EPA_OK ? p1 : pb.t};
+        finish_ball_contact(pos1, pos2, pb, radius, prediction, proj, false, f3{0.0f, 0.0f, 0.0f}, mode, out + k);
+    } else if (st == EPA_OK) {
+        finish_contact(pos1, pos2, pos12, p1, p2, n, is_local_mode(mode), out + k);
+    } else {
+        out[k] = no_contact(0);  // EPA failed: NoIntersection (contact_support_map_support_map.rs:75-76)
+        if (mode == kPairFeatureMaps) out[k].n1[0] = 1.0f;  // ... of Vector::x_axis()
+    }
+    if (iters) iters[2 * k + 1] = ei;
+}
+
+// One EPA tier: what it reads and where it sends the pairs that outgrow it.
+struct TierArgs {
+    const ShapeRecord *rec;
+    const float4 *verts;
+    const float *poses;
+    float prediction;
+    const EpaItem *queue;
+    const uint32_t *in_list;  // null: the queue itself
+    const uint32_t *in_count;
+    uint32_t *next;
+    const uint32_t *in_cont;
+    DevContact *out;
+    uint32_t *iters;
+    uint32_t *out_list;
+    uint32_t *out_cont;
+    uint32_t *out_count;
+    float *orig;
+};
+
+// Each trip through the loop is one EPA iteration of every running group.  Groups
+// that are done wait until half of the wave's groups are (or none runs): then the
+// wave writes their contacts and sets up their next pairs together, so the
+// memory latency of both (about 14,000 cycles, a third of an iteration's trip
+// when it was paid whenever one group finished) is paid once for all of them.
+// Measured on 2^20 mixed pairs, whole call, with 8 groups per wave: a turn-over
+// at 1 waiting group 4.64 ms, 3 4.46, 4 4.55, 8 4.63; on 262,144 pairs of
+// polyhedra 1.47, 1.38, 1.38 and 1.37 ms.  A wave reserves list entries from the
+// tier's counter in chunks (one atomic's latency per chunk) and hands them to the
+// waiting groups by rank; the turn-over is wave-uniform, so the ballot, lane 0's
+// atomic and the readfirstlane run converged.  Everything else is group-uniform,
+// and the cross-lane operations of the EPA code stay within a group.
+//
+// The first tier is bound by latency: an iteration takes a lone wave about
+// 17,000 cycles (support points 6,000, visibility 2,500, silhouette 4,000, new
+// faces 3,800) and the wave's three companions on a SIMD hide only part of it.
+template <int G, class W, class RI, class RO, int MINW>
+__global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI *recs, RecSink<RO> sink) {
+    constexpr uint32_t kGroups = 64 / G;
+    constexpr uint32_t kTurnover = kGroups > 2 ? kGroups / 2 : 1;
+    __shared__ W w[kGroups];
+    const uint32_t group = threadIdx.x / G;
+    const uint32_t sub = __lane_id() % G;
+    W *const wg = &w[group];
+    float *orig = t.orig + (size_t)(blockIdx.x * kGroups + group) * W::kV * kOrigFloats;
+    const uint32_t count = __hip_atomic_load(t.in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t chunk = count / (gridDim.x * 8u);  // the last chunks are an eighth of a wave's share at most
+    chunk = chunk < 1u ? 1u : (chunk > 32u ? 32u : chunk);
+    uint32_t at = 0, end = 0;  // the wave's reserved entries
+    bool busy = false, drained = false;
+    uint32_t slot = 0, status = EPA_OK;
+    EpaProblem pr{};
+    Staged st{nullptr, nullptr};
+    LazyRegs r{};
+    for (;;) {
+        // group-uniform: running a pair, or waiting for the next turn-over
+        const bool running = status == EPA_RUNNING;
+        const uint64_t wait = __ballot(!running && !drained && sub == 0);
+        const uint32_t n = (uint32_t)__popcll(wait);
+        if (n >= kTurnover || __ballot(running) == 0ull) {  // wave-uniform
+            if (!running && !drained && busy) {
+                uint32_t cont = kNoCont, ei = 0;
+                f3 p1{0.0f, 0.0f, 0.0f}, p2{0.0f, 0.0f, 0.0f}, nn{0.0f, 1.0f, 0.0f};
+                if constexpr (sizeof(typename W::Idx) == 1) {
+                    if (status == EPA_OVERFLOW) cont = lazy_export<G>(wg, orig, sink, r);
+                }
+                if (sub == 0) {
+                    if (status == EPA_OK) {
+                        lazy_points(wg, orig, r.best_id, p1, p2, nn);
+                        ei = r.niter + 1;
+                    }
+                    const uint32_t done = status == EPA_POINT ? EPA_OK : (status == EPA_RESTART ? EPA_OVERFLOW : status);
+                    epa_finish(t.rec, t.verts, t.poses, t.prediction, t.queue + slot, done, p1, p2, nn, ei, cont, t.out,
+                               t.iters, t.out_list, t.out_cont, t.out_count, slot);
+                }
+            }
+            if (n == 0) break;  // nothing runs and every group has seen the end of the list
+            const uint32_t left = end - at;
+            uint32_t more = 0;
+            if (left < n) {
+                const uint32_t take = chunk > n - left ? chunk : n - left;
+                if (__lane_id() == 0) more = atomicAdd(t.next, take);
+                more = __builtin_amdgcn_readfirstlane(more);
+                end = more + take;
+            }
+            const uint32_t rank = (uint32_t)__popcll(wait & ((1ull << (group * G)) - 1ull));
+            const uint32_t q = rank < left ? at + rank : more + (rank - left);
+            at = left < n ? more + (n - left) : at + n;
+            if (!running && !drained) {
+                if (q >= count) {
+                    drained = true;
+                } else {
+                    slot = t.in_list ? t.in_list[q] : q;
+                    const uint32_t ci = t.in_cont ? t.in_cont[q] : kNoCont;
+                    const EpaItem *it = t.queue + slot;
+                    pr = epa_problem(t.rec, t.verts, t.poses, it);
+                    status = lazy_begin<G>(wg, orig, pr, it, ci != kNoCont ? recs + ci : nullptr, st, r);
+                    busy = true;
+                }
+            }
+        }
+        if (status == EPA_RUNNING) status = lazy_step<G>(wg, orig, pr, st, r);
+    }
+}
+
+// First tier: LDS for about eight waves per CU, deleted flags in registers.  Its
+// polytopes move on to the second tier (four pairs per wave), those to the third
+// (one wave per pair, room for parry's 100 iterations).
+using LazySmall = LazyState<20, 64, 20, 24, uint8_t, 0>;
+using LazyWide = LazyState<48, 192, 48, 64, uint8_t, 0>;
+using LazyWave = LazyState<112, 768, 128, 512, uint16_t, 64>;
+using SmallRec = EpaRec<LazySmall::kV, LazySmall::kF>;
+using WideRec = EpaRec<LazyWide::kV, LazyWide::kF>;
+
+// ---------------------------------------------------------------------------
+// Stage 3: EPA with parry's heap, one wave per pair
+// ---------------------------------------------------------------------------
+// For the pairs whose polytope outgrows the third tier (more than 768 faces) and
+// those with a NaN or infinite face key: the heap itself, 2048 faces in LDS, then
+// 8192 in global memory.
+template <class I> struct EpaFaceT {
+    I pts[3];
+    I adj[3];
+    uint8_t deleted;
+    float n[3];
+};
+
+template <int V, int F, int H, int S, int K, class I, int SV> struct EpaState {
+    static constexpr int kV = V, kF = F, kH = H, kS = S, kK = K, kSV = SV;
+    using Idx = I;
+    using Face = EpaFaceT<I>;
+    float vp[V][3];
+    Face face[F];
+    I heap_id[H];
+    float heap_nd[H];
+    uint32_t sil[S];  // face | opp << 16
+    uint32_t stk[K];  // face | opp << 16
+    uint8_t vis[F];   // per face: can_be_seen_by the newest vertex, one bit per opposite vertex
+    float sv[2][SV > 0 ? SV : 1][3];  // both ConvexPolyhedra's vertices (local frames), if SV > 0
+};
+using EpaBig = EpaState<112, 2048, 2048, 128, 2048, uint16_t, 64>;
+using EpaLarge = EpaState<112, 8192, 8192, 2048, 8192, uint16_t, 0>;
 
 // BinaryHeap<FaceId> (max-heap on neg_dist; equal keys compare Equal), with
 // std's sift_up / sift_down_to_bottom so equal keys pop in parry's order.
@@ -606,46 +1369,6 @@ template <class W> struct Heap {
     }
 };
 
-enum : uint32_t { EPA_OK = 0, EPA_NONE = 1, EPA_OVERFLOW = 2, EPA_RUNNING = 3 };
-
-// Barycentric coordinates of Face::new's projection (epa3.rs:96-118,
-// TrianglePointLocation::barycentric_coordinates); returns proj_inside.
-__device__ __forceinline__ bool face_bcoords(f3 pa, f3 pb, f3 pc, float bc[3]) {
-    Loc l;
-    bool inside;
-    const f3 proj = tri_origin(pa, pb, pc, l, inside);
-    bc[0] = bc[1] = bc[2] = 0.0f;
-    const float e = kEps * 100.0f;
-    if (l.kind == LOC_VERTEX) {
-        bc[0] = l.id == 0 ? 1.0f : 0.0f;
-        bc[1] = l.id == 1 ? 1.0f : 0.0f;
-        bc[2] = l.id == 2 ? 1.0f : 0.0f;
-        return inside || norm_sq3(proj) < e * e;
-    }
-    if (l.kind == LOC_EDGE) {  // edges (0,1), (1,2), (0,2)
-        bc[0] = l.id == 1 ? 0.0f : l.b0;
-        bc[1] = l.id == 0 ? l.b1 : (l.id == 1 ? l.b0 : 0.0f);
-        bc[2] = l.id == 0 ? 0.0f : l.b1;
-        return inside || norm_sq3(proj) < e * e;
-    }
-    if (l.kind == LOC_FACE) {
-        bc[0] = l.b0;
-        bc[1] = l.b1;
-        bc[2] = l.b2;
-        return true;
-    }
-    return false;
-}
-
-// ccw_face_normal (utils/ccw_face_normal.rs:19-27), zero if degenerate.
-__device__ __forceinline__ f3 ccw_normal(f3 pa, f3 pb, f3 pc) {
-    const f3 r = cross3(sub3(pb, pa), sub3(pc, pa));
-    const float sq = norm_sq3(r);
-    f3 n = f3{0.0f, 0.0f, 0.0f};
-    if (sq > kEps * kEps) n = div3(r, sqrtf(sq));
-    return n;
-}
-
 // Face::new: fills face f; returns proj_inside.
 template <class W>
 __device__ bool face_new(W *w, uint32_t f, uint32_t a, uint32_t b, uint32_t c, uint32_t j0, uint32_t j1, uint32_t j2) {
@@ -699,159 +1422,18 @@ template <class W> __device__ __forceinline__ uint32_t next_ccw(const W *w, uint
     return 0;
 }
 
-// Face::can_be_seen_by (epa3.rs:147-163).
-template <class W> __device__ bool seen_by(const W *w, uint32_t f, uint32_t point, uint32_t opp) {
-    const typename W::Face &F = w->face[f];
-    const f3 p0 = vpt(w, F.pts[opp]);
-    const f3 p1 = vpt(w, F.pts[(opp + 1) % 3]);
-    const f3 p2 = vpt(w, F.pts[(opp + 2) % 3]);
-    const f3 pt = vpt(w, point);
-    if (dot3(sub3(pt, p0), fnormal(w, f)) >= -kEpsTol) return true;
-    const float E = kEps * 100.0f;
-    return norm_sq3(cross3(sub3(p2, p1), sub3(pt, p1))) <= E * E;  // Triangle::is_affinely_dependent
-}
-
-// A first-tier EPA polytope at the start of an iteration, handed to the
-// wave-per-pair tier so that the pair continues where it stopped instead of
-// starting over (byte ids: at most 48 vertices, 224 faces, 224 heap entries).
-constexpr int kContV = 48, kContF = 224, kContH = 224;
-constexpr uint32_t kNoCont = 0xffffffffu;
-struct EpaCont {
-    uint32_t nv, nf, len, best_id, niter, pad[3];
-    float max_dist, old_dist, padf[2];
-    float vp[kContV][3];
-    float orig[kContV][6];
-    uint32_t face[kContF][2];  // pts | deleted << 24, adj
-    uint32_t heap_id[kContH];
-    float heap_nd[kContH];
-};
-// Where a tier writes the polytopes it hands on (cap 0: it hands on none).
-struct ContSink {
-    EpaCont *recs;
-    uint32_t *count;
-    uint32_t cap;
-};
-struct EpaScalars {
-    uint32_t nv, nf, best_id, niter;
-    float max_dist, old_dist;
-};
-
-// Writes the group's polytope to a continuation record; returns its index or
-// kNoCont (no room, or a polytope type the record cannot hold).
-template <int G, class W>
-__device__ uint32_t epa_export(W *w, const float *orig, const ContSink &sink, const EpaScalars &x, uint32_t len) {
-    if constexpr (sizeof(typename W::Idx) == 1 && W::kV <= kContV && W::kF <= kContF && W::kH <= kContH) {
-        if (sink.cap == 0) return kNoCont;
-        const uint32_t sub = __lane_id() % G;
-        if (sub == 0) w->xfer = atomicAdd(sink.count, 1u);
-        // orig rows were written to global memory by this wave; the group's
-        // lanes read each other's rows below
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t ci = w->xfer;
-        if (ci >= sink.cap) return kNoCont;
-        EpaCont *r = sink.recs + ci;
-        if (sub == 0) {
-            r->nv = x.nv;
-            r->nf = x.nf;
-            r->len = len;
-            r->best_id = x.best_id;
-            r->niter = x.niter;
-            r->max_dist = x.max_dist;
-            r->old_dist = x.old_dist;
-        }
-        for (uint32_t k = sub; k < x.nv; k += G) {
-            for (int q = 0; q < 3; ++q) r->vp[k][q] = w->vp[k][q];
-            for (int q = 0; q < 6; ++q) r->orig[k][q] = orig[kOrigFloats * k + q];
-        }
-        for (uint32_t k = sub; k < x.nf; k += G) {
-            const typename W::Face &F = w->face[k];
-            r->face[k][0] = (uint32_t)F.pts[0] | ((uint32_t)F.pts[1] << 8) | ((uint32_t)F.pts[2] << 16) |
-                            ((uint32_t)F.deleted << 24);
-            r->face[k][1] = (uint32_t)F.adj[0] | ((uint32_t)F.adj[1] << 8) | ((uint32_t)F.adj[2] << 16);
-        }
-        for (uint32_t k = sub; k < len; k += G) {
-            r->heap_id[k] = w->heap_id[k];
-            r->heap_nd[k] = w->heap_nd[k];
-        }
-        return ci;
-    } else {
-        return kNoCont;
-    }
-}
-
-// Loads a continuation record into the group's polytope; face normals are
-// recomputed from the vertices exactly as Face::new computed them.
-template <int G, class W>
-__device__ void epa_import(W *w, float *orig, const EpaCont *r, EpaScalars &x, uint32_t &len) {
-    if constexpr (W::kV >= kContV && W::kF >= kContF && W::kH >= kContH) {
-        const uint32_t sub = __lane_id() % G;
-        x.nv = r->nv;
-        x.nf = r->nf;
-        len = r->len;
-        x.best_id = r->best_id;
-        x.niter = r->niter;
-        x.max_dist = r->max_dist;
-        x.old_dist = r->old_dist;
-        for (uint32_t k = sub; k < x.nv; k += G) {
-            for (int q = 0; q < 3; ++q) w->vp[k][q] = r->vp[k][q];
-            for (int q = 0; q < 6; ++q) orig[kOrigFloats * k + q] = r->orig[k][q];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        using I = typename W::Idx;
-        for (uint32_t k = sub; k < x.nf; k += G) {
-            const uint32_t a = r->face[k][0], b = r->face[k][1];
-            typename W::Face &F = w->face[k];
-            F.pts[0] = (I)(a & 0xffu);
-            F.pts[1] = (I)((a >> 8) & 0xffu);
-            F.pts[2] = (I)((a >> 16) & 0xffu);
-            F.deleted = (uint8_t)(a >> 24);
-            F.adj[0] = (I)(b & 0xffu);
-            F.adj[1] = (I)((b >> 8) & 0xffu);
-            F.adj[2] = (I)((b >> 16) & 0xffu);
-            const f3 nn = ccw_normal(vpt(w, F.pts[0]), vpt(w, F.pts[1]), vpt(w, F.pts[2]));
-            F.n[0] = nn.x;
-            F.n[1] = nn.y;
-            F.n[2] = nn.z;
-        }
-        for (uint32_t k = sub; k < len; k += G) {
-            w->heap_id[k] = (I)r->heap_id[k];
-            w->heap_nd[k] = r->heap_nd[k];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-// EPA::closest_points (epa3.rs:428-651) for one pair, executed by a group of G
-// lanes one iteration at a time: epa_begin, then epa_step until it returns a
-// result (epa_run below runs the whole loop).
-//
-// Every iteration is checkpointable: the heap's top is only peeked, the new
-// vertex goes to the first free slot without being counted, the best face and
-// distances are kept aside, and the faces the iteration deletes are listed.
-// Only when the polytope is known to have room for the iteration's new faces
-// and heap entries is the iteration committed -- the top popped (nothing reads
-// the heap between parry's pop and its pushes, so the heap ends up the same),
-// the vertex counted and the deletions kept.  A polytope that runs out of room
-// is therefore still the one the iteration started with: the deletions are
-// undone and, if `sink` has room, the polytope is written out for the next
-// tier to continue (`cont` gets the record's index).  `resume` starts from such
-// a record instead of the GJK simplex.
 template <class W> struct EpaRegs {
     Heap<W> heap;  // the polytope's face heap (LDS) and its length
     uint32_t nv, nf, best_id, niter;
     float max_dist, old_dist;
 };
 
-// The set-up before EPA's first iteration: the polytope from the GJK simplex, or
-// from a continuation record.  Returns EPA_RUNNING, or the result if EPA ends
-// here.
+// The set-up before EPA's first iteration: the polytope from the GJK simplex.
+// Returns EPA_RUNNING, or the result if EPA ends here.
 template <int G, class W>
 __device__ uint32_t epa_begin(W *w, float *orig, const iso &pos12, const ShapeRef &g1, const ShapeRef &g2,
-                              const EpaItem *it, const EpaCont *resume, Staged &st, EpaRegs<W> &r, f3 &p1, f3 &p2,
-                              f3 &n, uint32_t &epa_iters, uint32_t &cont) {
+                              const EpaItem *it, Staged &st, EpaRegs<W> &r, f3 &p1, f3 &p2, f3 &n,
+                              uint32_t &epa_iters) {
     st = Staged{stage_shape<G>(w, 0, g1), stage_shape<G>(w, 1, g2)};
     // The group's lanes wrote the staged vertices; make them visible to the
     // whole wave before any lane reads another lane's entries.
@@ -859,21 +1441,10 @@ __device__ uint32_t epa_begin(W *w, float *orig, const iso &pos12, const ShapeRe
     __builtin_amdgcn_wave_barrier();
     r = EpaRegs<W>{Heap<W>{w, 0}, 0, 0, 0, 0, kFltMax, 0.0f};
     Heap<W> &heap = r.heap;
-    uint32_t &nv = r.nv, &nf = r.nf, &best_id = r.best_id, &niter = r.niter;
-    float &max_dist = r.max_dist, &old_dist = r.old_dist;
+    uint32_t &nv = r.nv, &nf = r.nf, &best_id = r.best_id;
     epa_iters = 0;
-    cont = kNoCont;
-    if (resume) {
-        EpaScalars x;
-        epa_import<G>(w, orig, resume, x, heap.len);
-        nv = x.nv;
-        nf = x.nf;
-        best_id = x.best_id;
-        niter = x.niter;
-        max_dist = x.max_dist;
-        old_dist = x.old_dist;
-    } else {
-        const uint32_t dim = it->dim;
+    {
+        const uint32_t dim = it->dim_mode & 0xffu;
         for (uint32_t i = 0; i <= dim; ++i) {
             w->vp[i][0] = it->v[i][0];
             w->vp[i][1] = it->v[i][1];
@@ -941,8 +1512,7 @@ __device__ uint32_t epa_begin(W *w, float *orig, const iso &pos12, const ShapeRe
 // EPA_RUNNING while EPA goes on, else the result.
 template <int G, class W>
 __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef &g1, const ShapeRef &g2,
-                             const Staged &st, const ContSink &sink, EpaRegs<W> &r, f3 &p1, f3 &p2, f3 &n,
-                             uint32_t &epa_iters, uint32_t &cont) {
+                             const Staged &st, EpaRegs<W> &r, f3 &p1, f3 &p2, f3 &n, uint32_t &epa_iters) {
     const float eps_tol = kEps * 100.0f;
     Heap<W> &heap = r.heap;
     uint32_t &nv = r.nv, &nf = r.nf, &best_id = r.best_id, &niter = r.niter;
@@ -953,15 +1523,6 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
         face_points(w, orig, best_id, p1, p2);
         n = fnormal(w, best_id);
         return EPA_OK;
-    };
-    // Hands the polytope as it was at the start of this iteration to the next tier.
-    auto overflow = [&](uint32_t ndel, uint32_t fid) -> uint32_t {
-        for (uint32_t k = 0; k < ndel; ++k) w->face[w->dl[k]].deleted = 0;
-        w->face[fid].deleted = 0;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        cont = epa_export<G>(w, orig, sink, EpaScalars{nv, nf, best_id, niter, max_dist, old_dist}, heap.len);
-        return EPA_OVERFLOW;
     };
     // Faces deleted since they were pushed are popped and skipped here, as
     // parry's loop skips them (`continue`), rather than one per call.
@@ -977,7 +1538,7 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
         const typename W::Face face = w->face[fid];
         const f3 fn = f3{face.n[0], face.n[1], face.n[2]};
         const Cso c = group_cso<G>(pos12, g1, g2, st, fn);
-        if (nv >= (uint32_t)W::kV) return overflow(0, fid);
+        if (nv >= (uint32_t)W::kV) return EPA_OVERFLOW;
         const uint32_t sp = nv;  // counted when the iteration commits
         vset(w, orig, sp, c);
         const float cand = dot3(c.p, fn);
@@ -1029,8 +1590,8 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
         // whose top entry lives in a register.  After a visible face, the face
         // visited next (its first far neighbour) is loaded together with the
         // second one's points and carried in registers, so a step costs one
-        // round trip to LDS.  Deleted faces are listed in dl for an undo.
-        uint32_t ns = 0, sk = 0, depth = 0, top = 0, ndel = 0;
+        // round trip to LDS. 
+        uint32_t ns = 0, sk = 0, depth = 0, top = 0;
         typename W::Face cf = w->face[face.adj[0]];
         uint32_t cvis = w->vis[face.adj[0]];
         uint32_t cur = face.adj[0] | (ccw_index(cf, face.pts[0]) << 16);
@@ -1050,14 +1611,12 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
             const uint32_t id = cur & 0xffffu, opp = cur >> 16;
             const bool del = !cf.deleted && ((cvis >> opp) & 1u);
             if (!cf.deleted && !del) {
-                if (ns >= (uint32_t)W::kS) return overflow(ndel, fid);
+                if (ns >= (uint32_t)W::kS) return EPA_OVERFLOW;
                 w->sil[ns++] = cur;
             }
             if (!del && depth == 0) break;
             uint32_t nid, pt1 = 0, popped = 0;
             if (del) {
-                if (ndel >= (uint32_t)W::kS) return overflow(ndel, fid);
-                w->dl[ndel++] = (typename W::Idx)id;
                 w->face[id].deleted = 1;
                 // a1 = (opp + 2) % 3 and a2 = opp, selected by value so the
                 // record stays in registers
@@ -1067,7 +1626,7 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
                 const uint32_t pt2 = pick3(opp, cf.pts[0], cf.pts[1], cf.pts[2]);
                 const uint32_t o2 = next_ccw(w, adj2, pt2);
                 if (depth > 0) {
-                    if (sk >= (uint32_t)W::kK) return overflow(ndel, fid);
+                    if (sk >= (uint32_t)W::kK) return EPA_OVERFLOW;
                     w->stk[sk++] = top;
                 }
                 top = adj2 | (o2 << 16);
@@ -1104,7 +1663,7 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
             n_live += (uint32_t)__popcll((__ballot(alive) >> gbase) & gmask);
         }
         if (first_new + n_live > (uint32_t)W::kF || heap.len - 1 + n_live > (uint32_t)W::kH)
-            return overflow(ndel, fid);
+            return EPA_OVERFLOW;
         // Commit: parry popped this face before all of the above.
         {
             uint32_t pid;
@@ -1178,283 +1737,72 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
     return EPA_RUNNING;
 }
 
-// EPA::closest_points (epa3.rs:428-651) for one pair by a group of G lanes.
-template <int G, class W>
-__device__ uint32_t epa_run(W *w, float *orig, const iso &pos12, const ShapeRef &g1, const ShapeRef &g2,
-                            const EpaItem *it, const EpaCont *resume, const ContSink &sink, f3 &p1, f3 &p2, f3 &n,
-                            uint32_t &epa_iters, uint32_t &cont) {
-    Staged st;
-    EpaRegs<W> r;
-    uint32_t s = epa_begin<G>(w, orig, pos12, g1, g2, it, resume, st, r, p1, p2, n, epa_iters, cont);
-    while (s == EPA_RUNNING) s = epa_step<G>(w, orig, pos12, g1, g2, st, sink, r, p1, p2, n, epa_iters, cont);
-    return s;
-}
 
-
-// The EPA problem of a queued pair (contact_support_map_support_map.rs:60-76):
-// its two shapes (their feature maps in kPairFeatureMaps mode) and relative pose,
-// or, for a Ball, the other shape against the ball centre
-// (point_support_map.rs:39-49).
-struct EpaProblem {
-    iso pos;
-    ShapeRef a, b;
-};
-
-__device__ EpaProblem epa_problem(const ShapeRecord *rec, const float4 *verts, const float *poses,
-                                  const uint32_t *pairs, const EpaItem *it) {
-    const uint32_t k = it->pair;
-    const uint32_t i = pairs[2 * k], j = pairs[2 * k + 1];
-    const iso pos1 = load_iso(poses + 7 * (size_t)i), pos2 = load_iso(poses + 7 * (size_t)j);
-    const iso pos12 = iso_inv_mul(pos1, pos2);
-    ShapeRef g1 = load_shape(rec, verts, i), g2 = load_shape(rec, verts, j);
-    const uint32_t mode = it->mode;
-    if (mode == kPairFeatureMaps) {
-        float br;
-        (void)feature_map(g1, br);
-        (void)feature_map(g2, br);
-    }
-    if (is_ball_mode(mode)) {
-        if (mode == kBallFirst) return EpaProblem{point_proj_iso(iso_inverse(pos12).t), g2, origin_shape()};
-        return EpaProblem{point_proj_iso(pos12.t), g1, origin_shape()};
-    }
-    return EpaProblem{pos12, g1, g2};
-}
-
-// Writes the result of a queued pair's EPA (one lane per pair): the contact, or
-// the pair's entry in the next tier's list if its polytope outgrew this tier's.
-__device__ void epa_finish(const ShapeRecord *rec, const float4 *verts, const float *poses, const uint32_t *pairs,
-                           float prediction, const EpaItem *it, uint32_t st, f3 p1, f3 p2, f3 n, uint32_t ei,
-                           uint32_t cont, DevContact *out, uint32_t *iters, uint32_t *overflow_list,
-                           uint32_t *overflow_cont, uint32_t *overflow_count, uint32_t slot) {
-    const uint32_t k = it->pair;
-    if (st == EPA_OVERFLOW) {
-        if (overflow_list) {
-            const uint32_t pos = atomicAdd(overflow_count, 1u);
-            overflow_list[pos] = slot;
-            if (overflow_cont) overflow_cont[pos] = cont;
-        } else {
-            out[k] = no_contact(kUnsupportedPair);  // cannot happen with the large buffers
-        }
-        return;
-    }
-    const uint32_t i = pairs[2 * k], j = pairs[2 * k + 1];
-    const iso pos1 = load_iso(poses + 7 * (size_t)i), pos2 = load_iso(poses + 7 * (size_t)j);
-    const iso pos12 = iso_inv_mul(pos1, pos2);
-    const uint32_t mode = it->mode;
-    if (is_ball_mode(mode)) {
-        // the Ball-vs-convex contact from the projection of the ball centre
-        const iso pb = mode == kBallFirst ? iso_inverse(pos12) : pos12;
-        const float radius = rec[mode == kBallFirst ? i : j].param[0];
-        const PointProj proj{true, st == EPA_OK ? p1 : pb.t};
-        finish_ball_contact(pos1, pos2, pb, radius, prediction, proj, false, f3{0.0f, 0.0f, 0.0f}, mode, out + k);
-    } else if (st == EPA_OK) {
-        finish_contact(pos1, pos2, pos12, p1, p2, n, is_local_mode(mode), out + k);
-    } else {
-        out[k] = no_contact(0);  // EPA failed: NoIntersection (contact_support_map_support_map.rs:75-76)
-        if (mode == kPairFeatureMaps) out[k].n1[0] = 1.0f;  // ... of Vector::x_axis()
-    }
-    if (iters) iters[2 * k + 1] = ei;
-}
-
-template <int G, class W>
-__device__ void epa_item(W *w, float *orig, const ShapeRecord *rec, const float4 *verts, const float *poses,
-                         const uint32_t *pairs, float prediction, const EpaItem *it, const EpaCont *resume,
-                         const ContSink &sink, DevContact *out, uint32_t *iters, uint32_t *overflow_list,
-                         uint32_t *overflow_cont, uint32_t *overflow_count, uint32_t slot) {
-    const EpaProblem pr = epa_problem(rec, verts, poses, pairs, it);
-    f3 p1, p2, n;
-    uint32_t ei = 0, cont = kNoCont;
-    const uint32_t st = epa_run<G>(w, orig, pr.pos, pr.a, pr.b, it, resume, sink, p1, p2, n, ei, cont);
-    if (__lane_id() % G != 0) return;
-    epa_finish(rec, verts, poses, pairs, prediction, it, st, p1, p2, n, ei, cont, out, iters, overflow_list,
-               overflow_cont, overflow_count, slot);
-}
-
-// EPA tiers.  Each reads a list of queued pairs (the queue itself for the first
-// tier) and sends the pairs whose polytope outgrows its buffers to the next
-// tier's list: G lanes per pair with a small LDS polytope, then one wave per
-// pair with medium and big LDS polytopes, then a global-memory polytope.
-// At most 168 VGPRs (three waves per SIMD) where a wave's polytopes take at
-// most 16 KB of LDS, which leaves room for that many waves: the first tier's
-// latency-bound code needs them.  Larger polytopes are limited by LDS anyway,
-// and a wave per pair (G = 64) keeps its registers.
-template <int G, class W> constexpr int epa_min_waves() { return G < 64 && (64 / G) * sizeof(W) <= 16384 ? 3 : 1; }
-template <int G, class W>
-__global__ __launch_bounds__(64, (epa_min_waves<G, W>())) void epa_tier_kernel(const ShapeRecord *__restrict__ rec,
-                                                      const float4 *__restrict__ verts, const float *__restrict__ poses,
-                                                      const uint32_t *__restrict__ pairs, float prediction,
-                                                      const EpaItem *__restrict__ queue, const uint32_t *in_list,
-                                                      const uint32_t *in_count, uint32_t *next,
-                                                      const uint32_t *in_cont, const EpaCont *cont_recs,
-                                                      ContSink sink, DevContact *__restrict__ out,
-                                                      uint32_t *__restrict__ iters, uint32_t *out_list,
-                                                      uint32_t *out_cont, uint32_t *out_count, float *orig_scratch) {
-    constexpr int kGroups = 64 / G;
-    __shared__ W w[kGroups];
-    const uint32_t group = threadIdx.x / G;
-    const uint32_t gid = blockIdx.x * kGroups + group;
-    float *orig = orig_scratch + (size_t)gid * W::kV * kOrigFloats;
-    const uint32_t count = __hip_atomic_load(in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // The wave takes its next kGroups list entries from the tier's counter
-    // whenever all its groups are done, so no wave is left with a long run of
-    // long pairs.  The fetch happens where the whole wave is converged and the
-    // exit test is wave-uniform: no cross-lane exchange under divergence.
-    for (;;) {
-        uint32_t base = 0;
-        if (__lane_id() == 0) base = atomicAdd(next, (uint32_t)kGroups);
-        base = __builtin_amdgcn_readfirstlane(base);
-        if (base >= count) break;
-        const uint32_t q = base + group;
-        if (q < count) {
-            const uint32_t slot = in_list ? in_list[q] : q;
-            const uint32_t ci = in_cont ? in_cont[q] : kNoCont;
-            epa_item<G>(&w[group], orig, rec, verts, poses, pairs, prediction, queue + slot,
-                        ci != kNoCont ? cont_recs + ci : nullptr, sink, out, iters, out_list, out_cont, out_count,
-                        slot);
-        }
-    }
-}
-
-// The first tier with a refill per group: a group that is done with its pair
-// takes the next list entry at once, while the other groups of its wave go on
-// with theirs, so a wave no longer waits for the longest of its pairs.  Each
-// trip through the loop runs, per group, either the set-up of a new pair or one
-// EPA iteration (the two are executed one after the other by the wave when its
-// groups differ).  The fetch and the loop's exit test are at the top of the
-// loop, where the whole wave is converged: a ballot of the idle groups' first
-// lanes, one atomicAdd by lane 0 for all of them, the base read with
-// readfirstlane, and each idle group's entry at its rank among them (no
-// cross-lane exchange under divergence).  Everything after is group-uniform,
-// and the cross-lane operations of the EPA code stay within a group.
-template <int G, class W>
-__global__ __launch_bounds__(64, (epa_min_waves<G, W>())) void epa_refill_kernel(const ShapeRecord *__restrict__ rec,
-                                                      const float4 *__restrict__ verts, const float *__restrict__ poses,
-                                                      const uint32_t *__restrict__ pairs, float prediction,
-                                                      const EpaItem *__restrict__ queue, const uint32_t *in_list,
-                                                      const uint32_t *in_count, uint32_t *next,
-                                                      const uint32_t *in_cont, const EpaCont *cont_recs,
-                                                      ContSink sink, DevContact *__restrict__ out,
-                                                      uint32_t *__restrict__ iters, uint32_t *out_list,
-                                                      uint32_t *out_cont, uint32_t *out_count, float *orig_scratch) {
-    static_assert(G < 64, "a wave-per-pair tier has nothing to refill");
-    constexpr int kGroups = 64 / G;
-    __shared__ W w[kGroups];
-    const uint32_t group = threadIdx.x / G;
-    const uint32_t sub = __lane_id() % G;
-    const uint32_t gid = blockIdx.x * kGroups + group;
-    W *const wg = &w[group];
-    float *orig = orig_scratch + (size_t)gid * W::kV * kOrigFloats;
-    const uint32_t count = __hip_atomic_load(in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    bool busy = false, drained = false;
-    uint32_t slot = 0, status = EPA_OK, ei = 0, cont = kNoCont;
-    EpaProblem pr{};
-    Staged st{nullptr, nullptr};
-    EpaRegs<W> r{Heap<W>{wg, 0}, 0, 0, 0, 0, kFltMax, 0.0f};
-    f3 p1{0.0f, 0.0f, 0.0f}, p2{0.0f, 0.0f, 0.0f}, n{0.0f, 0.0f, 0.0f};
-    for (;;) {
-        const bool idle = !busy && !drained;  // group-uniform
-        const uint64_t want = __ballot(idle && sub == 0);
-        if (want != 0ull) {  // wave-uniform
-            uint32_t base = 0;
-            if (__lane_id() == 0) base = atomicAdd(next, (uint32_t)__popcll(want));
-            base = __builtin_amdgcn_readfirstlane(base);
-            const uint32_t q = base + (uint32_t)__popcll(want & ((1ull << (group * G)) - 1ull));
-            if (idle && q >= count) {
-                drained = true;
-            } else if (idle) {
-                slot = in_list ? in_list[q] : q;
-                const uint32_t ci = in_cont ? in_cont[q] : kNoCont;
-                pr = epa_problem(rec, verts, poses, pairs, queue + slot);
-                status = epa_begin<G>(wg, orig, pr.pos, pr.a, pr.b, queue + slot,
-                                      ci != kNoCont ? cont_recs + ci : nullptr, st, r, p1, p2, n, ei, cont);
-                busy = true;
-            }
-        }
-        if (__ballot(!drained) == 0ull) break;
-        if (busy) {
-            if (status == EPA_RUNNING)
-                status = epa_step<G>(wg, orig, pr.pos, pr.a, pr.b, st, sink, r, p1, p2, n, ei, cont);
-            if (status != EPA_RUNNING) {
-                if (sub == 0)
-                    epa_finish(rec, verts, poses, pairs, prediction, queue + slot, status, p1, p2, n, ei, cont, out,
-                               iters, out_list, out_cont, out_count, slot);
-                busy = false;
-            }
-        }
-    }
-}
-
-// Last tier: one wave per pair, polytope in global memory.
-__global__ __launch_bounds__(64) void epa_global_kernel(const ShapeRecord *__restrict__ rec,
-                                                        const float4 *__restrict__ verts,
-                                                        const float *__restrict__ poses,
-                                                        const uint32_t *__restrict__ pairs, float prediction,
-                                                        const EpaItem *__restrict__ queue,
-                                                        DevContact *__restrict__ out, uint32_t *__restrict__ iters,
-                                                        const uint32_t *in_list, const uint32_t *in_count,
-                                                        uint32_t *next, EpaLarge *scratch, float *orig_scratch) {
-    EpaLarge *w = scratch + blockIdx.x;
-    float *orig = orig_scratch + (size_t)blockIdx.x * EpaLarge::kV * kOrigFloats;
-    const uint32_t count = __hip_atomic_load(in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A tier of this stage: a wave per pair, the next pair from the tier's counter.
+// P: the wave's polytope, in LDS or global memory.
+template <class W>
+__device__ void epa_wave_loop(const TierArgs &t, W *w, float *orig) {
+    const uint32_t count = __hip_atomic_load(t.in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
         uint32_t q = 0;
-        if (__lane_id() == 0) q = atomicAdd(next, 1u);
+        if (__lane_id() == 0) q = atomicAdd(t.next, 1u);
         q = __builtin_amdgcn_readfirstlane(q);
         if (q >= count) break;
-        epa_item<64>(w, orig, rec, verts, poses, pairs, prediction, queue + in_list[q], nullptr, ContSink{nullptr, nullptr, 0},
-                     out, iters, nullptr, nullptr, nullptr, q);
+        const uint32_t slot = t.in_list[q];
+        const EpaItem *it = t.queue + slot;
+        const EpaProblem pr = epa_problem(t.rec, t.verts, t.poses, it);
+        f3 p1, p2, n;
+        uint32_t ei = 0;
+        Staged st;
+        EpaRegs<W> r;
+        uint32_t s = epa_begin<64>(w, orig, pr.pos, pr.a, pr.b, it, st, r, p1, p2, n, ei);
+        while (s == EPA_RUNNING) s = epa_step<64>(w, orig, pr.pos, pr.a, pr.b, st, r, p1, p2, n, ei);
+        if (__lane_id() == 0)
+            epa_finish(t.rec, t.verts, t.poses, t.prediction, it, s, p1, p2, n, ei, kNoCont, t.out, t.iters, t.out_list,
+                       nullptr, t.out_count, slot);
     }
 }
+__global__ __launch_bounds__(64) void epa_big_kernel(TierArgs t) {
+    __shared__ EpaBig w;
+    epa_wave_loop(t, &w, t.orig + (size_t)blockIdx.x * EpaBig::kV * kOrigFloats);
+}
+__global__ __launch_bounds__(64) void epa_global_kernel(TierArgs t, EpaLarge *scratch) {
+    epa_wave_loop(t, scratch + blockIdx.x, t.orig + (size_t)blockIdx.x * EpaLarge::kV * kOrigFloats);
+}
 
-template <int G, class W>
-hipError_t launch_epa_tier(const DeviceShapes &s, const float *poses, const uint32_t *pairs, float prediction,
-                           uint64_t max_items, const EpaItem *queue, const uint32_t *in_list, const uint32_t *in_count,
-                           uint32_t *next, const uint32_t *in_cont, const EpaCont *cont_recs, ContSink sink,
-                           DevContact *out, uint32_t *iters, uint32_t *out_list, uint32_t *out_cont,
-                           uint32_t *out_count, float *orig, uint64_t max_groups, hipStream_t stream,
-                           bool refill = false) {
+// Waves that fill the current device with a kernel of 64-lane workgroups.
+hipError_t resident_waves(const void *kernel, uint64_t *waves) {
     hipError_t e;
     int dev = 0, cus = 0, per_cu = 0;
     if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-    const void *kernel = (const void *)epa_tier_kernel<G, W>;
-    if constexpr (G < 64) {
-        if (refill) kernel = (const void *)epa_refill_kernel<G, W>;
-    }
     if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0)) != hipSuccess) return e;
-    if (per_cu < 1) per_cu = 1;
+    *waves = (uint64_t)cus * (uint64_t)(per_cu < 1 ? 1 : per_cu);
+    return hipSuccess;
+}
+
+template <int G, class W, class RI, class RO, int MINW>
+hipError_t launch_lazy(const TierArgs &t, const RI *recs, const RecSink<RO> &sink, uint64_t max_items,
+                       uint64_t max_groups, hipStream_t stream) {
     constexpr uint64_t kGroups = 64 / G;
-    uint64_t waves = (uint64_t)cus * (uint64_t)per_cu;
+    uint64_t waves = 0;
+    hipError_t e = resident_waves((const void *)epa_lazy_kernel<G, W, RI, RO, MINW>, &waves);
+    if (e != hipSuccess) return e;
     const uint64_t need = (max_items + kGroups - 1) / kGroups;
     if (waves > need) waves = need;
     if (waves * kGroups > max_groups) waves = max_groups / kGroups;
     if (waves < 1) waves = 1;
-    if constexpr (G < 64) {
-        if (refill) {
-            hipLaunchKernelGGL((epa_refill_kernel<G, W>), dim3((uint32_t)waves), dim3(64), 0, stream, s.rec, s.verts,
-                               poses, pairs, prediction, queue, in_list, in_count, next, in_cont, cont_recs, sink, out,
-                               iters, out_list, out_cont, out_count, orig);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((epa_tier_kernel<G, W>), dim3((uint32_t)waves), dim3(64), 0, stream, s.rec, s.verts, poses,
-                       pairs, prediction, queue, in_list, in_count, next, in_cont, cont_recs, sink, out, iters,
-                       out_list, out_cont, out_count, orig);
+    hipLaunchKernelGGL((epa_lazy_kernel<G, W, RI, RO, MINW>), dim3((uint32_t)waves), dim3(64), 0, stream, t, recs, sink);
     return hipGetLastError();
 }
 
 }  // namespace
 
 // Resident EPA groups the workspace provides orig1/orig2 buffers for, per tier.
-constexpr uint64_t kEpaMaxGroups = 256ull * 16 * 8;
-constexpr uint64_t kEpaMediumWaves = 256ull * 8;
-// orig1/orig2 rows per first-tier group: the most vertices of any first-tier polytope.
-constexpr uint64_t kSmallMaxVertices = 48;
-static_assert(EpaSmall::kV <= kSmallMaxVertices && EpaSmallUnstaged::kV <= kSmallMaxVertices &&
-                  EpaTiny::kV <= kSmallMaxVertices && EpaSmallWide::kV <= kSmallMaxVertices &&
-                  EpaSmallLarge::kV <= kSmallMaxVertices,
-              "first-tier orig buffer too small");
-constexpr uint64_t kEpaBigWaves = 256ull * 2;
+constexpr uint64_t kSmallGroups = 256ull * 12 * 8;
+constexpr uint64_t kWideGroups = 256ull * 8 * 4;
+constexpr uint64_t kWaveGroups = 256ull * 8;
+constexpr uint64_t kBigWaves = 256ull * 2;
 
 int g_epa_lanes_per_pair = 16;
 int g_epa_polytope = 1;
@@ -1466,25 +1814,20 @@ namespace {
 struct ContactWorkspace {
     uint32_t *counters;  // list lengths and the tiers' next entries (reset_counters_kernel)
     EpaItem *queue;
-    uint32_t *lists[3];
-    uint32_t *cont_list;  // per entry of lists[0]: its continuation record or kNoCont
-    EpaCont *conts;
-    uint32_t cont_cap;
+    uint32_t *lists[4];
+    uint32_t *cont_list[2];  // per entry of lists[0] and lists[1]: its continuation record or kNoCont
+    SmallRec *small_recs;
+    WideRec *wide_recs;
+    uint32_t small_cap, wide_cap;
     EpaLarge *large;
-    float *orig_large, *orig_small, *orig_medium, *orig_big;
+    float *orig_small, *orig_wide, *orig_wave, *orig_big, *orig_large;
     size_t bytes;
 };
 
-// Continuation records: one per 48 pairs (overflowing pairs are about 1% of
-// mixed-shape pairs), at least 256 and at most 32768.  A pair that finds them
-// all taken restarts in the next tier instead.
-uint64_t cont_capacity(uint64_t m) {
-    uint64_t c = m / 48;
-    if (c < 256) c = 256;
-    if (c > 32768) c = 32768;
-    return c;
-}
+uint64_t clamp_u64(uint64_t v, uint64_t lo, uint64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
+// Continuation records: the first tier hands on about 3% of mixed-shape pairs,
+// the second 0.3%.  A pair that finds them all taken restarts in the next tier.
 ContactWorkspace carve_workspace(void *base, uint64_t m) {
     const size_t align = 256;
     auto up = [&](size_t b) { return (b + align - 1) / align * align; };
@@ -1498,48 +1841,30 @@ ContactWorkspace carve_workspace(void *base, uint64_t m) {
     };
     w.counters = (uint32_t *)take(kNumCounters * sizeof(uint32_t));
     w.queue = (EpaItem *)take(m * sizeof(EpaItem));
-    for (int k = 0; k < 3; ++k) w.lists[k] = (uint32_t *)take(m * sizeof(uint32_t));
-    w.cont_list = (uint32_t *)take(m * sizeof(uint32_t));
-    w.cont_cap = (uint32_t)cont_capacity(m);
-    w.conts = (EpaCont *)take((size_t)w.cont_cap * sizeof(EpaCont));
+    for (uint32_t *&l : w.lists) l = (uint32_t *)take(m * sizeof(uint32_t));
+    for (uint32_t *&l : w.cont_list) l = (uint32_t *)take(m * sizeof(uint32_t));
+    w.small_cap = (uint32_t)clamp_u64(m / 16, 256, 131072);
+    w.wide_cap = (uint32_t)clamp_u64(m / 128, 256, 16384);
+    w.small_recs = (SmallRec *)take((size_t)w.small_cap * sizeof(SmallRec));
+    w.wide_recs = (WideRec *)take((size_t)w.wide_cap * sizeof(WideRec));
     w.large = (EpaLarge *)take(kEpaGlobalWaves * sizeof(EpaLarge));
-    w.orig_large = (float *)take(kEpaGlobalWaves * EpaLarge::kV * kOrigFloats * sizeof(float));
-    w.orig_small = (float *)take(kEpaMaxGroups * kSmallMaxVertices * kOrigFloats * sizeof(float));
-    w.orig_medium = (float *)take(kEpaMediumWaves * EpaMedium::kV * kOrigFloats * sizeof(float));
-    w.orig_big = (float *)take(kEpaBigWaves * EpaBig::kV * kOrigFloats * sizeof(float));
+    auto orig = [&](uint64_t groups, uint64_t verts) { return (float *)take(groups * verts * kOrigFloats * sizeof(float)); };
+    w.orig_small = orig(kSmallGroups, LazySmall::kV);
+    w.orig_wide = orig(kWideGroups, LazyWide::kV);
+    w.orig_wave = orig(kWaveGroups, LazyWave::kV);
+    w.orig_big = orig(kBigWaves, EpaBig::kV);
+    w.orig_large = orig(kEpaGlobalWaves, EpaLarge::kV);
     w.bytes = off;
     return w;
+}
+
+template <int G>
+hipError_t launch_small(const TierArgs &t, const RecSink<SmallRec> &sink, uint64_t m, hipStream_t stream) {
+    return launch_lazy<G, LazySmall, SmallRec, SmallRec, 3>(t, nullptr, sink, m, kSmallGroups, stream);
 }
 }  // namespace
 
 size_t contact_workspace_bytes(uint64_t num_pairs) { return carve_workspace(nullptr, num_pairs).bytes; }
-
-namespace {
-// First EPA tier: G lanes per pair with the selected small polytope; it hands
-// overflowing pairs on with continuation records.
-template <int G, class W>
-hipError_t launch_first(const DeviceShapes &s, const float *poses, const uint32_t *pairs, float prediction, uint64_t m,
-                        const ContactWorkspace &w, uint32_t *c, DevContact *o, uint32_t *iters, hipStream_t stream,
-                        bool refill) {
-    return launch_epa_tier<G, W>(s, poses, pairs, prediction, m, w.queue, nullptr, c, c + 4, nullptr, nullptr,
-                                 ContSink{w.conts, c + 8, w.cont_cap}, o, iters, w.lists[0], w.cont_list, c + 1,
-                                 w.orig_small, kEpaMaxGroups, stream, refill);
-}
-template <int G>
-hipError_t launch_small(const DeviceShapes &s, const float *poses, const uint32_t *pairs, float prediction, uint64_t m,
-                        const ContactWorkspace &w, uint32_t *c, DevContact *o, uint32_t *iters, hipStream_t stream,
-                        uint32_t flags) {
-    // the first tier's schedule: a refill per group, except for short EPA runs
-    const bool refill = G < 64 && (g_epa_schedule == 2 || (g_epa_schedule == 0 && !(flags & kContactShortEpa)));
-    switch (g_epa_polytope) {
-        case 1: return launch_first<G, EpaSmallUnstaged>(s, poses, pairs, prediction, m, w, c, o, iters, stream, refill);
-        case 2: return launch_first<G, EpaTiny>(s, poses, pairs, prediction, m, w, c, o, iters, stream, refill);
-        case 3: return launch_first<G, EpaSmallWide>(s, poses, pairs, prediction, m, w, c, o, iters, stream, refill);
-        case 4: return launch_first<G, EpaSmallLarge>(s, poses, pairs, prediction, m, w, c, o, iters, stream, refill);
-        default: return launch_first<G, EpaSmall>(s, poses, pairs, prediction, m, w, c, o, iters, stream, refill);
-    }
-}
-}  // namespace
 
 hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint32_t *pairs, uint64_t m,
                            const uint64_t *m_dev, float prediction, const float *seeds, pq_contact *out,
@@ -1559,27 +1884,40 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
     if (e == hipSuccess) e = mark(1);
     if (e != hipSuccess) return e;
     uint32_t *const c = w.counters;
-    switch (g_epa_lanes_per_pair) {
-        case 4: e = launch_small<4>(s, poses, pairs, prediction, m, w, c, o, iters, stream, flags); break;
-        case 8: e = launch_small<8>(s, poses, pairs, prediction, m, w, c, o, iters, stream, flags); break;
-        case 16: e = launch_small<16>(s, poses, pairs, prediction, m, w, c, o, iters, stream, flags); break;
-        case 32: e = launch_small<32>(s, poses, pairs, prediction, m, w, c, o, iters, stream, flags); break;
-        default: e = launch_small<64>(s, poses, pairs, prediction, m, w, c, o, iters, stream, flags); break;
+    // Tier k reads list k - 1 (the queue for the first) and sends the pairs that outgrow it to list k.
+    auto tier = [&](uint32_t k, float *orig) {
+        return TierArgs{s.rec, s.verts, poses, prediction, w.queue, k ? w.lists[k - 1] : nullptr, c + k, c + kTiers + k,
+                        k == 1 ? w.cont_list[0] : (k == 2 ? w.cont_list[1] : nullptr), o, iters,
+                        k < 4 ? w.lists[k] : nullptr, k < 2 ? w.cont_list[k] : nullptr, c + k + 1, orig};
+    };
+    const TierArgs t0 = tier(0, w.orig_small);
+    const RecSink<SmallRec> small_sink{w.small_recs, c + 10, w.small_cap};
+    const int lanes = g_epa_schedule == 0 ? 8 : g_epa_lanes_per_pair;
+    switch (lanes) {
+        case 4: e = launch_small<4>(t0, small_sink, m, stream); break;
+        case 8: e = launch_small<8>(t0, small_sink, m, stream); break;
+        case 16: e = launch_small<16>(t0, small_sink, m, stream); break;
+        case 32: e = launch_small<32>(t0, small_sink, m, stream); break;
+        default: e = launch_small<64>(t0, small_sink, m, stream); break;
     }
+    if (e != hipSuccess) return e;
+    e = launch_lazy<16, LazyWide, SmallRec, WideRec, 2>(tier(1, w.orig_wide), w.small_recs,
+                                                        RecSink<WideRec>{w.wide_recs, c + 11, w.wide_cap}, m,
+                                                        kWideGroups, stream);
     if (e == hipSuccess) e = mark(2);
     if (e != hipSuccess) return e;
-    const ContSink none{nullptr, nullptr, 0};
-    e = launch_epa_tier<64, EpaMedium>(s, poses, pairs, prediction, m, w.queue, w.lists[0], c + 1, c + 5, w.cont_list,
-                                       w.conts, none, o, iters, w.lists[1], nullptr, c + 2, w.orig_medium,
-                                       kEpaMediumWaves, stream);
+    e = launch_lazy<64, LazyWave, WideRec, WideRec, 1>(tier(2, w.orig_wave), w.wide_recs,
+                                                       RecSink<WideRec>{nullptr, nullptr, 0}, m, kWaveGroups, stream);
     if (e == hipSuccess) e = mark(3);
     if (e != hipSuccess) return e;
-    e = launch_epa_tier<64, EpaBig>(s, poses, pairs, prediction, m, w.queue, w.lists[1], c + 2, c + 6, nullptr, nullptr,
-                                    none, o, iters, w.lists[2], nullptr, c + 3, w.orig_big, kEpaBigWaves, stream);
+    uint64_t waves = 0;
+    if ((e = resident_waves((const void *)epa_big_kernel, &waves)) != hipSuccess) return e;
+    waves = clamp_u64(waves, 1, kBigWaves < m ? kBigWaves : m);
+    hipLaunchKernelGGL(epa_big_kernel, dim3((uint32_t)waves), dim3(64), 0, stream, tier(3, w.orig_big));
+    e = hipGetLastError();
     if (e == hipSuccess) e = mark(4);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(epa_global_kernel, dim3(kEpaGlobalWaves), dim3(64), 0, stream, s.rec, s.verts, poses, pairs,
-                       prediction, w.queue, o, iters, w.lists[2], c + 3, c + 7, w.large, w.orig_large);
+    hipLaunchKernelGGL(epa_global_kernel, dim3(kEpaGlobalWaves), dim3(64), 0, stream, tier(4, w.orig_large), w.large);
     e = hipGetLastError();
     if (e == hipSuccess) e = mark(5);
     return e;

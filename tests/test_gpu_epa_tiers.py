@@ -1,0 +1,70 @@
+"""EPA's face choice without a heap, and its polytopes' way through the tiers, against the oracle.
+
+The tiers take the next face as the maximum of the face keys and only rebuild parry's heap when several live
+faces share it: symmetric shapes at aligned poses share it all the time.  Long runs (curved shapes, deep
+overlaps) cross the tiers' vertex and face limits."""
+import numpy as np
+import pytest
+
+from parry_amd import SHAPE_DESC_DTYPE, ShapeSet, contact_pairs
+
+pytestmark = pytest.mark.gpu
+
+# quaternions of quarter turns (i, j, k, w)
+TURNS = np.array([[0, 0, 0, 1], [1, 0, 0, 0], [0, 1, 0, 0], [0.5, 0.5, 0.5, 0.5], [0, 0.70710678, 0, 0.70710678],
+                  [0.70710678, 0, 0, 0.70710678]], np.float64)
+OCTAHEDRON = np.array([[1, 0, 0], [-1, 0, 0], [0, 1, 0], [0, -1, 0], [0, 0, 1], [0, 0, -1]], np.float32)
+
+
+def aligned_case(types, n, seed):
+    """``n`` pairs of unit shapes of the two types at quarter turns, offset by multiples of a quarter."""
+    rng = np.random.default_rng(seed)
+    d = np.zeros(2 * n, SHAPE_DESC_DTYPE)
+    d["type"] = np.tile(types, n)
+    d["params"][:, :3] = 1.0
+    d["params"][d["type"] == 2, 1] = 0.5
+    poly = d["type"] == 4
+    d["num_vertices"][poly] = len(OCTAHEDRON)
+    d["params"][poly] = 0.0
+    poses = np.zeros((2 * n, 7))
+    poses[:, :4] = TURNS[rng.integers(0, len(TURNS), 2 * n)]
+    poses[1::2, 4:] = rng.integers(-5, 6, (n, 3)) * 0.25
+    return d, OCTAHEDRON, poses.astype(np.float32), np.arange(2 * n, dtype=np.uint32).reshape(n, 2)
+
+
+def deep_case(types, n, seed):
+    """``n`` pairs of curved shapes with centres close together: up to parry's 100 iterations."""
+    rng = np.random.default_rng(seed)
+    d = np.zeros(2 * n, SHAPE_DESC_DTYPE)
+    d["type"] = np.tile(types, n)
+    d["params"][:, :2] = rng.uniform(0.3, 1.5, (2 * n, 2))
+    d["params"][:, 2] = 1.0
+    q = rng.standard_normal((2 * n, 4))
+    poses = np.concatenate([q / np.linalg.norm(q, axis=1, keepdims=True), np.zeros((2 * n, 3))], 1)
+    poses[1::2, 4:] = rng.normal(0.0, 0.2, (n, 3))
+    return d, np.zeros((0, 3), np.float32), poses.astype(np.float32), np.arange(2 * n, dtype=np.uint32).reshape(n, 2)
+
+
+CASES = [(aligned_case, t) for t in ((1, 1), (1, 4), (4, 4), (1, 2), (2, 2), (3, 3), (1, 3))]
+CASES += [(deep_case, t) for t in ((2, 2), (2, 3), (3, 3), (1, 2))]
+
+
+@pytest.mark.parametrize("make,types", CASES, ids=lambda v: getattr(v, "__name__", str(v)))
+def test_epa_tiers_match_oracle(orc, make, types):
+    import torch
+
+    for n in (1, 7, 1500):
+        descs, verts, poses, pairs = make(types, n, 7 + n)
+        print(f"case: {make.__name__} {types}, {n} pairs", flush=True)
+        shapes = ShapeSet(descs, verts)
+        out, iters = contact_pairs(shapes, torch.from_numpy(poses).cuda(),
+                                   torch.from_numpy(pairs.view(np.int32)).cuda(), 0.25, with_iters=True)
+        out, iters = out.cpu().numpy(), iters.cpu().numpy()
+        ref = orc.contact_pairs(descs, verts, poses, pairs, 0.25)
+        has = out.view(np.uint32)[:, 13].astype(np.int64)
+        assert np.array_equal(has, ref["status"])
+        hit = has == 1
+        # parry's own sequence of f32 operations: the same bits (+0.0: signed zeros compare equal)
+        assert np.array_equal(out[hit, :13] + 0.0, ref["out"][hit] + 0.0)
+        assert np.array_equal(iters[:, 0], ref["iters"][:, 0].astype(np.int32))
+        print(f"  {hit.sum()} contacts, EPA iterations up to {ref['iters'][:, 1].max()}")
