@@ -77,7 +77,9 @@ int pq_shapes_create(const pq_shape_desc *shapes, uint32_t n, const float *verti
         pq_shapes_destroy(s);
         return hip_fail(e, "pq_shapes_create upload");
     }
-    s->dev = DeviceShapes{(const ShapeRecord *)s->d_rec, (const float4 *)s->d_verts, n, num_vertices};
+    uint32_t types = 0;
+    for (const ShapeRecord &r : rec) types |= 1u << r.type;
+    s->dev = DeviceShapes{(const ShapeRecord *)s->d_rec, (const float4 *)s->d_verts, n, num_vertices, types};
     *out = s;
     return PQ_OK;
 }

@@ -45,7 +45,7 @@ int pq_mesh_contact_create(const pq_trimesh *mesh, const pq_shapes *shapes, pq_m
     mc->mesh = mesh;
     mc->num_shapes = n;
     mc->combined = DeviceShapes{(const ShapeRecord *)mc->d_rec, (const float4 *)mc->d_verts, (uint32_t)nrec,
-                                (uint32_t)nverts};
+                                (uint32_t)nverts, shapes->dev.types};
     *out = mc;
     return PQ_OK;
 }

@@ -139,8 +139,106 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 // counters[10..11]: continuation records taken by the first and second tier.
 constexpr uint32_t kNumCounters = 12;
 constexpr uint32_t kTiers = 5;
-__global__ void reset_counters_kernel(uint32_t *counters) {
-    if (threadIdx.x < kNumCounters) counters[threadIdx.x] = 0u;
+
+// ---------------------------------------------------------------------------
+// The order the pairs are taken in
+// ---------------------------------------------------------------------------
+// A wave of mixed pairs runs the union of its pairs' support functions, vertex
+// scans and iteration counts.  Where it pays (takes_order), a counting sort by
+// the pair's two shape classes (below) puts like pairs side by side for GJK, and
+// so for the EPA queue GJK appends to; the shapes whose EPA runs longest (curved
+// ones) come first, so the tiers do not end on them.  Results go to the pair's own
+// slot, and no result depends on the order.
+constexpr uint32_t kShapeClasses = 16;
+constexpr uint32_t kPairClasses = 2 * kShapeClasses * kShapeClasses;
+constexpr uint32_t kOrderBlock = 256, kOrderRange = 2048;  // lanes and pairs per workgroup
+__device__ __forceinline__ uint32_t shape_class(const ShapeRecord *rec, uint32_t i) {
+    const uint4 r = *reinterpret_cast<const uint4 *>(rec + i);  // type, first vertex, vertices
+    if (r.x == PQ_SHAPE_CAPSULE) return 0;
+    if (r.x == PQ_SHAPE_CONE) return 1;
+    if (r.x == PQ_SHAPE_CONVEX_POLYHEDRON) return 9u - (r.z >= 64u ? 7u : r.z / 8u);  // 2 to 9 by vertex count
+    if (r.x == PQ_SHAPE_CUBOID) return 10;
+    if (r.x == PQ_SHAPE_TRIANGLE) return 11;
+    return 12;
+}
+// The two classes, the earlier one first, and which of the shapes has it.
+__device__ __forceinline__ uint32_t pair_class(const ShapeRecord *rec, uint32_t i, uint32_t j) {
+    const uint32_t a = shape_class(rec, i), b = shape_class(rec, j);
+    const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
+    return (lo * kShapeClasses + hi) * 2u + (a > b ? 1u : 0u);
+}
+__device__ __forceinline__ uint64_t pair_count(uint64_t m, const unsigned long long *m_dev) {
+    if (m_dev && *m_dev < m) m = *m_dev;
+    return m;
+}
+// Pairs per class, and every pair's class.
+__global__ __launch_bounds__(kOrderBlock) void order_count_kernel(const ShapeRecord *__restrict__ rec,
+                                                                  const uint32_t *__restrict__ pairs, uint64_t m,
+                                                                  const unsigned long long *__restrict__ m_dev,
+                                                                  uint16_t *__restrict__ cls,
+                                                                  uint32_t *__restrict__ totals) {
+    __shared__ uint32_t hist[kPairClasses];
+    for (uint32_t c = threadIdx.x; c < kPairClasses; c += kOrderBlock) hist[c] = 0u;
+    __syncthreads();
+    m = pair_count(m, m_dev);
+    const uint64_t first = (uint64_t)blockIdx.x * kOrderRange;
+#pragma unroll 4
+    for (uint32_t q = threadIdx.x; q < kOrderRange; q += kOrderBlock) {
+        const uint64_t k = first + q;
+        if (k < m) {
+            const uint32_t c = pair_class(rec, pairs[2 * k], pairs[2 * k + 1]);
+            cls[k] = (uint16_t)c;
+            atomicAdd(&hist[c], 1u);
+        }
+    }
+    __syncthreads();
+    for (uint32_t c = threadIdx.x; c < kPairClasses; c += kOrderBlock)
+        if (hist[c]) atomicAdd(&totals[c], hist[c]);
+}
+// order[]: the pairs class by class.  A workgroup reserves its part of each class
+// with one atomic; taken[] starts at zero.
+__global__ __launch_bounds__(kOrderBlock) void order_scatter_kernel(uint64_t m,
+                                                                    const unsigned long long *__restrict__ m_dev,
+                                                                    const uint16_t *__restrict__ cls,
+                                                                    const uint32_t *__restrict__ totals,
+                                                                    uint32_t *__restrict__ taken,
+                                                                    uint32_t *__restrict__ order) {
+    static_assert(kPairClasses == 2 * kOrderBlock, "two classes per lane");
+    __shared__ uint32_t hist[kPairClasses], base[kPairClasses], scan[kOrderBlock];
+    const uint32_t l = threadIdx.x;
+    hist[2 * l] = hist[2 * l + 1] = 0u;
+    const uint32_t t0 = totals[2 * l], t1 = totals[2 * l + 1];
+    scan[l] = t0 + t1;
+    __syncthreads();
+    for (uint32_t d = 1; d < kOrderBlock; d *= 2) {
+        const uint32_t v = l >= d ? scan[l - d] : 0u;
+        __syncthreads();
+        scan[l] += v;
+        __syncthreads();
+    }
+    m = pair_count(m, m_dev);
+    const uint64_t first = (uint64_t)blockIdx.x * kOrderRange;
+    uint32_t key[kOrderRange / kOrderBlock], rank[kOrderRange / kOrderBlock];
+#pragma unroll
+    for (uint32_t u = 0; u < kOrderRange / kOrderBlock; ++u) {
+        const uint64_t k = first + u * kOrderBlock + l;
+        key[u] = k < m ? cls[k] : 0u;
+        rank[u] = k < m ? atomicAdd(&hist[key[u]], 1u) : 0u;
+    }
+    __syncthreads();
+    const uint32_t before = scan[l] - t0 - t1, h0 = hist[2 * l], h1 = hist[2 * l + 1];
+    base[2 * l] = before + (h0 ? atomicAdd(&taken[2 * l], h0) : 0u);
+    base[2 * l + 1] = before + t0 + (h1 ? atomicAdd(&taken[2 * l + 1], h1) : 0u);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < kOrderRange / kOrderBlock; ++u) {
+        const uint64_t k = first + u * kOrderBlock + l;
+        if (k < m) order[base[key[u]] + rank[u]] = (uint32_t)k;
+    }
+}
+
+__global__ void reset_counters_kernel(uint32_t *counters, uint32_t n) {
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) counters[k] = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -150,12 +248,14 @@ __global__ __launch_bounds__(kBlock) void contact_gjk_kernel(
     const ShapeRecord *__restrict__ rec, const float4 *__restrict__ verts, const float *__restrict__ poses,
     const uint32_t *__restrict__ pairs, uint64_t m, const unsigned long long *__restrict__ m_dev, float prediction,
     const float *__restrict__ seeds, DevContact *__restrict__ out, uint32_t *__restrict__ iters,
-    EpaItem *__restrict__ queue, uint32_t *__restrict__ counters, uint32_t flags) {
-    const uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    EpaItem *__restrict__ queue, uint32_t *__restrict__ counters, uint32_t flags,
+    const uint32_t *__restrict__ order) {
+    uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (m_dev) {
         const uint64_t md = *m_dev;
         if (md < m) m = md;
     }
+    if (order && k < m) k = order[k];
     bool need_epa = false;
     uint32_t ball_mode = kPairSupportMaps;
     Simplex s;
@@ -380,80 +480,103 @@ template <int G> __device__ __forceinline__ void group_argmax(float &best, uint3
     }
 }
 
-// ConvexPolyhedron support point computed by a group of G consecutive lanes:
+// The bits of a wave ballot that belong to the caller's group.
+template <int G> __device__ __forceinline__ uint64_t group_ballot(bool p) {
+    const uint32_t gbase = __lane_id() & ~(uint32_t)(G - 1);
+    return (__ballot(p) >> gbase) & (G >= 64 ? ~0ull : ((1ull << (G & 63)) - 1ull));
+}
+
+// ConvexPolyhedron support points computed by a group of G consecutive lanes:
 // parry takes the first strict maximum of p.d over the vertex list; if vertex
 // 0's product is NaN nothing ever beats it, otherwise the result is the lowest
 // index among the largest non-NaN products, which is what the group reduction
-// (largest value, then lowest index) returns.
-template <int G> __device__ __forceinline__ f3 group_support(const ShapeRef &s, f3 d) {
-    if (s.type != PQ_SHAPE_CONVEX_POLYHEDRON) return local_support(s, d);
-    const float4 p0 = s.v[0];
-    const float d0 = dot3(f3{p0.x, p0.y, p0.z}, d);
-    if (d0 != d0) return f3{p0.x, p0.y, p0.z};
+// (largest value, then lowest index) returns.  Each lane scans vertices sub,
+// sub + G, ... in order; the coordinates of the best one travel with it.
+struct Scan {
+    float best;
+    uint32_t bi;
+    f3 bp;
+    bool nan0;  // vertex 0's product is NaN (lane 0 of the group)
+};
+constexpr uint32_t kNoVertex = 0xffffffffu;
+__device__ __forceinline__ void scan_step(Scan &s, float4 p, uint32_t k, bool valid, f3 d) {
+    const f3 q = f3{p.x, p.y, p.z};
+    const float dd = dot3(q, d);
+    const bool take = valid && dd == dd && (s.bi == kNoVertex || dd > s.best);
+    s.nan0 = (valid && k == 0u) ? dd != dd : s.nan0;
+    s.best = take ? dd : s.best;
+    s.bi = take ? k : s.bi;
+    s.bp = sel2(take, q, s.bp);
+}
+// Two scans side by side, four vertices of each in flight: one memory latency per
+// 4 G vertices of the longer list (a list of length 0 repeats loads of the
+// other's first vertex and is ignored).  Vertex 0's product is taken from the
+// scan itself, without a load of its own before it.
+template <int G>
+__device__ __forceinline__ void group_scan2(const float4 *v1, uint32_t n1, f3 d1, const float4 *v2, uint32_t n2, f3 d2,
+                                            f3 &r1, f3 &r2) {
     const uint32_t sub = __lane_id() % G;
-    float best = -INFINITY;
-    uint32_t bi = 0xffffffffu;
-    f3 bp = f3{p0.x, p0.y, p0.z};  // the coordinates of vertex bi travel with it
-    // Each lane scans vertices sub, sub + G, ... in order, four loads in flight.
-    for (uint32_t k = sub; k < s.n; k += 4 * G) {
-        float4 p[4];
+    Scan a{-INFINITY, kNoVertex, f3{0.0f, 0.0f, 0.0f}, false}, b = a;
+    const uint32_t n = n1 > n2 ? n1 : n2;
+    const uint32_t last1 = n1 ? n1 - 1u : 0u, last2 = n2 ? n2 - 1u : 0u;
+    for (uint32_t k0 = 0; k0 < n; k0 += 4 * G) {
+        float4 p[4], q[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t kk = k + (uint32_t)j * G;
-            p[j] = kk < s.n ? s.v[kk] : p0;
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t k = k0 + j * G + sub;
+            p[j] = v1[k < last1 ? k : last1];
+            q[j] = v2[k < last2 ? k : last2];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t kk = k + (uint32_t)j * G;
-            const float dd = dot3(f3{p[j].x, p[j].y, p[j].z}, d);
-            if (kk < s.n && dd == dd && (bi == 0xffffffffu || dd > best)) {
-                best = dd;
-                bi = kk;
-                bp = f3{p[j].x, p[j].y, p[j].z};
-            }
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t k = k0 + j * G + sub;
+            scan_step(a, p[j], k, k < n1, d1);
+            scan_step(b, q[j], k, k < n2, d2);
         }
     }
-    // Lane sub = 0 always holds a candidate (vertex 0's product is not NaN), so
-    // the group's reduction ends on a vertex some lane loaded: no reload.
-    group_argmax<G>(best, bi, bp);
-    return bp;
+    const bool nan1 = group_ballot<G>(a.nan0) != 0ull, nan2 = group_ballot<G>(b.nan0) != 0ull;
+    if (nan1 || nan2) {  // vertex 0, whatever the others are
+        if (nan1) a = Scan{0.0f, 0u, f3{v1[0].x, v1[0].y, v1[0].z}, true};
+        if (nan2) b = Scan{0.0f, 0u, f3{v2[0].x, v2[0].y, v2[0].z}, true};
+    }
+    group_argmax<G>(a.best, a.bi, a.bp);
+    group_argmax<G>(b.best, b.bi, b.bp);
+    r1 = a.bp;
+    r2 = b.bp;
 }
 
-// The same reduction over vertices staged in LDS (sv = nullptr: not staged).
-template <int G> __device__ __forceinline__ f3 group_support_staged(const ShapeRef &s, const float (*sv)[3], f3 d) {
-    if (s.type != PQ_SHAPE_CONVEX_POLYHEDRON || sv == nullptr) return group_support<G>(s, d);
-    const f3 p0 = f3{sv[0][0], sv[0][1], sv[0][2]};
-    const float d0 = dot3(p0, d);
-    if (d0 != d0) return p0;
+// One scan over vertices staged in LDS.
+template <int G> __device__ __forceinline__ f3 group_scan_staged(const float (*sv)[3], uint32_t n, f3 d) {
     const uint32_t sub = __lane_id() % G;
-    float best = -INFINITY;
-    uint32_t bi = 0xffffffffu;
-    f3 bp = p0;
-    for (uint32_t k = sub; k < s.n; k += G) {
-        const f3 q = f3{sv[k][0], sv[k][1], sv[k][2]};
-        const float dd = dot3(q, d);
-        if (dd == dd && (bi == 0xffffffffu || dd > best)) {
-            best = dd;
-            bi = k;
-            bp = q;
-        }
-    }
-    group_argmax<G>(best, bi, bp);
-    return bp;
+    Scan a{-INFINITY, kNoVertex, f3{0.0f, 0.0f, 0.0f}, false};
+    for (uint32_t k = sub; k < n; k += G)
+        scan_step(a, make_float4(sv[k][0], sv[k][1], sv[k][2], 0.0f), k, true, d);
+    if (group_ballot<G>(a.nan0) != 0ull) return f3{sv[0][0], sv[0][1], sv[0][2]};
+    group_argmax<G>(a.best, a.bi, a.bp);
+    return a.bp;
 }
 
 struct Staged {
-    const float (*s1)[3];
+    const float (*s1)[3];  // null: not staged
     const float (*s2)[3];
 };
 
-template <int G>
+// CSOPoint::from_shapes (see cso_from_shapes) by a group; STAGED: the
+// ConvexPolyhedra may be staged in LDS.
+template <int G, bool STAGED>
 __device__ __forceinline__ Cso group_cso(const iso &pos12, const ShapeRef &g1, const ShapeRef &g2, const Staged &st,
                                          f3 dir) {
-    const f3 a = group_support_staged<G>(g1, st.s1, dir);
-    const f3 b = g2.type == kShapeOrigin
-                     ? pos12.t
-                     : iso_point(pos12, group_support_staged<G>(g2, st.s2, qrot_inv(pos12.q, neg3(dir))));
+    const f3 d2 = qrot_inv(pos12.q, neg3(dir));
+    const bool poly1 = g1.type == PQ_SHAPE_CONVEX_POLYHEDRON, poly2 = g2.type == PQ_SHAPE_CONVEX_POLYHEDRON;
+    f3 a{0.0f, 0.0f, 0.0f}, b{0.0f, 0.0f, 0.0f};
+    const bool scan1 = poly1 && !(STAGED && st.s1), scan2 = poly2 && !(STAGED && st.s2);
+    if (scan1 || scan2)
+        group_scan2<G>(scan1 ? g1.v : g2.v, scan1 ? g1.n : 0u, dir, scan2 ? g2.v : g1.v, scan2 ? g2.n : 0u, d2, a, b);
+    if (STAGED && poly1 && st.s1) a = group_scan_staged<G>(st.s1, g1.n, dir);
+    if (STAGED && poly2 && st.s2) b = group_scan_staged<G>(st.s2, g2.n, d2);
+    if (!poly1) a = local_support(g1, dir);
+    if (!poly2) b = local_support(g2, d2);
+    b = g2.type == kShapeOrigin ? pos12.t : iso_point(pos12, b);
     return Cso{sub3(a, b), a, b};
 }
 
@@ -545,15 +668,17 @@ template <int V, int F, int S, int K, class I, int SV> struct LazyState {
     static constexpr uint32_t kShift = sizeof(I) == 1 ? 8u : 16u;
     using Idx = I;
     using Entry = std::conditional_t<sizeof(I) == 1, uint16_t, uint32_t>;
-    alignas(8) I adj[F][4];
-    uint32_t px[F];  // vertices; bits 24-26: can_be_seen_by the newest vertex per opposite vertex; 27: deleted
-    float key[F];    // FaceId's neg_dist, -inf for a face that was not pushed
-    float n[F][3];
-    float vp[V][3];
+    struct alignas(sizeof(I) == 1 ? 8 : 4) Face {
+        uint32_t px;  // vertices; bits 24-26: can_be_seen_by the newest vertex per opposite vertex; 27: deleted
+        I adj[4];     // neighbours (three)
+    };
+    alignas(16) float nk[F][4];  // normal, then FaceId's neg_dist (-inf for a face that was not pushed)
+    float vp[V][4];
+    Face face[F];
     float sv[SV > 0 ? 2 : 1][SV > 0 ? SV : 1][3];  // both ConvexPolyhedra's vertices (local frames), if SV > 0
-    Entry sil[S];              // face | opp << kShift
-    Entry stk[K];              // face | point << kShift
-    I dl[kMask ? 1 : S];       // faces the current iteration deleted (undone if it cannot commit)
+    Entry sil[S + 1];          // face | opp << kShift, and a slot for what is not kept
+    Entry stk[K + 1];          // face | point << kShift, likewise
+    I dl[kMask ? 1 : S + 1];   // faces the current iteration deleted (undone if it cannot commit)
     I hid[F];                  // the heap's face ids, when it is rebuilt
     I pops[V], nfs[V];         // per iteration: the face it popped, and the number of faces before it
 };
@@ -573,16 +698,27 @@ template <class W> __device__ __forceinline__ bool face_dead(const W *w, const L
     return (x & kDeadBit) != 0u;
 }
 // The three neighbours of a face, kShift bits each.
-template <class W> __device__ __forceinline__ auto face_adj(const W *w, uint32_t f) {
-    if constexpr (sizeof(typename W::Idx) == 1)
-        return *reinterpret_cast<const uint32_t *>(w->adj[f]);
+template <class F> __device__ __forceinline__ auto face_adj(const F &f) {
+    if constexpr (sizeof(f.adj[0]) == 1)
+        return __builtin_bit_cast(uint32_t, f.adj);
     else
-        return *reinterpret_cast<const uint64_t *>(w->adj[f]);
+        return (uint64_t)f.adj[0] | ((uint64_t)f.adj[1] << 16) | ((uint64_t)f.adj[2] << 32);
+}
+template <class W> __device__ __forceinline__ float &face_key(W *w, uint32_t f) { return w->nk[f][3]; }
+template <class W> __device__ __forceinline__ f3 face_normal(const W *w, uint32_t f) {
+    return f3{w->nk[f][0], w->nk[f][1], w->nk[f][2]};
 }
 template <class W, class A> __device__ __forceinline__ uint32_t adj_at(A a, uint32_t k) {
     return (uint32_t)(a >> (W::kShift * k)) & ((1u << W::kShift) - 1u);
 }
 __device__ __forceinline__ uint32_t pt_at(uint32_t x, uint32_t k) { return (x >> (8u * k)) & 0xffu; }
+// Entry of the silhouette walk: neighbour k of a face and the face's point k.
+template <class W> __device__ __forceinline__ uint32_t walk_entry(const typename W::Face &f, uint32_t k) {
+    if constexpr (sizeof(typename W::Idx) == 1)  // bytes k of adj and px
+        return __builtin_amdgcn_perm(f.px, face_adj(f), 0x0c0c0400u + k * 0x0101u);
+    else
+        return adj_at<W>(face_adj(f), k) | (pt_at(f.px, k) << W::kShift);
+}
 
 __device__ __forceinline__ void lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -602,10 +738,34 @@ template <int G> __device__ __forceinline__ float group_max(float v) {
     if constexpr (G >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
     return v;
 }
-// The bits of a wave ballot that belong to the caller's group.
-template <int G> __device__ __forceinline__ uint64_t group_ballot(bool p) {
-    const uint32_t gbase = __lane_id() & ~(uint32_t)(G - 1);
-    return (__ballot(p) >> gbase) & (G >= 64 ? ~0ull : ((1ull << (G & 63)) - 1ull));
+// proj_inside of Face::new (epa3.rs:96-118): whether the origin projects inside
+// the triangle, or onto a vertex or edge within 100 EPS of the origin.  The
+// comparisons are those of Triangle::project_local_point_and_get_location
+// (point_triangle.rs:54-291) in its order, but the regions are selected instead
+// of branched to: the lanes of a wave build faces of every region, and took all
+// six branches with a division each.
+__device__ __forceinline__ bool face_inside(f3 a, f3 b, f3 c) {
+    const f3 ab = sub3(b, a), ac = sub3(c, a), bc = sub3(c, b);
+    const f3 ap = neg3(a), bp = neg3(b), cp = neg3(c);
+    const float ab_ap = dot3(ab, ap), ac_ap = dot3(ac, ap);
+    const float ab_bp = dot3(ab, bp), ac_bp = dot3(ac, bp);
+    const float ab_cp = dot3(ab, cp), ac_cp = dot3(ac, cp);
+    const f3 n = cross3(ab, ac);
+    const float vc = dot3(n, cross3(ab, ap)), vb = -dot3(n, cross3(ac, cp)), va = dot3(n, cross3(bc, bp));
+    const bool va_ = (ab_ap <= 0.0f) & (ac_ap <= 0.0f);
+    const bool vb_ = !va_ & (ab_bp >= 0.0f) & (ac_bp <= ab_bp);
+    const bool vc_ = !va_ & !vb_ & (ac_cp >= 0.0f) & (ab_cp <= ac_cp);
+    const bool vertex = va_ | vb_ | vc_;
+    const bool eab = !vertex & (vc < 0.0f) & (ab_ap >= 0.0f) & (ab_bp <= 0.0f);
+    const bool eac = !vertex & !eab & (vb < 0.0f) & (ac_ap >= 0.0f) & (ac_cp <= 0.0f);
+    const bool ebc = !vertex & !eab & !eac & (va < 0.0f) & (ac_bp - ab_bp >= 0.0f) & (ab_cp - ac_cp >= 0.0f);
+    const f3 base = sel2(vb_ | ebc, b, sel2(vc_, c, a));
+    const f3 dir = sel2(eab, ab, sel2(eac, ac, bc));
+    const float t = (eab ? ab_ap : (eac ? ac_ap : dot3(bc, bp))) / norm_sq3(dir);
+    const f3 r = sel2(vertex, base, add3(base, mul3(dir, t)));
+    const float e = kEps * 100.0f;
+    const bool near = near_origin(r) || norm_sq3(r) < e * e;
+    return (vertex | eab | eac | ebc) ? near : va + vb + vc != 0.0f;
 }
 
 // Face::new (epa3.rs:96-118) by one lane; returns proj_inside.
@@ -613,24 +773,19 @@ template <class W>
 __device__ __forceinline__ bool lazy_face(W *w, uint32_t f, uint32_t a, uint32_t b, uint32_t c, uint32_t j0,
                                           uint32_t j1, uint32_t j2, f3 &n, f3 &pa) {
     using I = typename W::Idx;
-    w->px[f] = a | (b << 8) | (c << 16);
-    w->adj[f][0] = (I)j0;
-    w->adj[f][1] = (I)j1;
-    w->adj[f][2] = (I)j2;
+    w->face[f] = typename W::Face{a | (b << 8) | (c << 16), {(I)j0, (I)j1, (I)j2, (I)0}};
     pa = vpt(w, a);
     const f3 pb = vpt(w, b), pc = vpt(w, c);
-    float bc[3];
-    const bool in = face_bcoords(pa, pb, pc, bc);
     n = ccw_normal(pa, pb, pc);
-    w->n[f][0] = n.x;
-    w->n[f][1] = n.y;
-    w->n[f][2] = n.z;
-    return in;
+    return face_inside(pa, pb, pc);
+}
+template <class W> __device__ __forceinline__ void set_normal(W *w, uint32_t f, f3 n, float key) {
+    *reinterpret_cast<float4 *>(w->nk[f]) = make_float4(n.x, n.y, n.z, key);
 }
 
 // Face::closest_points (epa3.rs:120-130).
 template <class W> __device__ void lazy_points(const W *w, const float *orig, uint32_t f, f3 &p1, f3 &p2, f3 &n) {
-    const uint32_t x = w->px[f];
+    const uint32_t x = w->face[f].px;
     float bc[3];
     face_bcoords(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)), bc);
     f3 o1[3], o2[3];
@@ -641,17 +796,17 @@ template <class W> __device__ void lazy_points(const W *w, const float *orig, ui
     }
     p1 = add3(add3(mul3(o1[0], bc[0]), mul3(o1[1], bc[1])), mul3(o1[2], bc[2]));
     p2 = add3(add3(mul3(o2[0], bc[0]), mul3(o2[1], bc[1])), mul3(o2[2], bc[2]));
-    n = f3{w->n[f][0], w->n[f][1], w->n[f][2]};
+    n = face_normal(w, f);
 }
 
 // BinaryHeap<FaceId> over face ids (max-heap on key[]; equal keys compare Equal),
 // with std's sift_up / sift_down_to_bottom so equal keys pop in parry's order.
 template <class W> __device__ __forceinline__ void heap_sift_up(W *w, uint32_t pos) {
     const uint32_t id = w->hid[pos];
-    const float nd = w->key[id];
+    const float nd = face_key(w, id);
     while (pos > 0) {
         const uint32_t parent = (pos - 1) / 2, pid = w->hid[parent];
-        if (nd <= w->key[pid]) break;
+        if (nd <= face_key(w, pid)) break;
         w->hid[pos] = (typename W::Idx)pid;
         pos = parent;
     }
@@ -665,7 +820,7 @@ template <class W> __device__ __forceinline__ void heap_pop(W *w, uint32_t &len)
     while (child + 2 <= len) {
         uint32_t cid = w->hid[child];
         const uint32_t rid = w->hid[child + 1];
-        if (w->key[cid] <= w->key[rid]) {
+        if (face_key(w, cid) <= face_key(w, rid)) {
             ++child;
             cid = rid;
         }
@@ -691,7 +846,7 @@ template <class W> __device__ uint32_t lazy_replay(W *w, LazyRegs &r) {
         const bool now = r.hiter == r.niter;
         const uint32_t upto = now ? r.nf : w->nfs[r.hiter];
         for (; r.hnf < upto; ++r.hnf)
-            if (w->key[r.hnf] != -INFINITY) {
+            if (face_key(w, r.hnf) != -INFINITY) {
                 w->hid[r.hlen] = (typename W::Idx)r.hnf;
                 heap_sift_up(w, r.hlen++);
             }
@@ -706,7 +861,7 @@ template <class W> __device__ uint32_t lazy_replay(W *w, LazyRegs &r) {
     }
     while (r.hlen != 0) {
         const uint32_t id = w->hid[0];
-        if (!face_dead(w, r, id, w->px[id])) return id;
+        if (!face_dead(w, r, id, w->face[id].px)) return id;
         heap_pop(w, r.hlen);
     }
     return kNoFace;  // not reached: a live pushed face is in the heap
@@ -759,10 +914,10 @@ __device__ uint32_t lazy_export(const W *w, const float *orig, const RecSink<R> 
         for (int q = 0; q < 6; ++q) o->orig[k][q] = orig[kOrigFloats * k + q];
     }
     for (uint32_t k = sub; k < r.nf; k += G) {
-        const uint32_t x = w->px[k];
-        o->px[k] = (x & 0x00ffffffu) | (face_dead(w, r, k, x) ? kDeadBit : 0u);
-        o->adj[k] = face_adj(w, k);
-        o->key[k] = w->key[k];
+        const typename W::Face f = w->face[k];
+        o->px[k] = (f.px & 0x00ffffffu) | (face_dead(w, r, k, f.px) ? kDeadBit : 0u);
+        o->adj[k] = face_adj(f);
+        o->key[k] = w->nk[k][3];
     }
     for (uint32_t k = sub; k < r.niter; k += G) {
         o->pops[k] = (uint8_t)w->pops[k];
@@ -791,13 +946,8 @@ template <int G, class W, class R> __device__ void lazy_import(W *w, float *orig
     __builtin_amdgcn_wave_barrier();
     for (uint32_t k = sub; k < r.nf; k += G) {
         const uint32_t x = o->px[k], a = o->adj[k];
-        w->px[k] = x;
-        for (int q = 0; q < 3; ++q) w->adj[k][q] = (I)((a >> (8 * q)) & 0xffu);
-        w->key[k] = o->key[k];
-        const f3 nn = ccw_normal(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)));
-        w->n[k][0] = nn.x;
-        w->n[k][1] = nn.y;
-        w->n[k][2] = nn.z;
+        w->face[k] = typename W::Face{x, {(I)(a & 0xffu), (I)((a >> 8) & 0xffu), (I)(a >> 16), (I)0}};
+        set_normal(w, k, ccw_normal(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2))), o->key[k]);
     }
     for (uint32_t k = sub; k < r.niter; k += G) {
         w->pops[k] = (I)o->pops[k];
@@ -871,7 +1021,7 @@ __device__ uint32_t lazy_begin(W *w, float *orig, const EpaProblem &pr, const Ep
         const f3 dpt = sub3(pv[1], pv[0]);
         f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.0f, -dpt.x} : f3{0.0f, -dpt.z, dpt.y};
         a = div3(a, sqrtf(norm_sq3(a)));
-        vset(w, orig, 2, group_cso<G>(pr.pos, pr.a, pr.b, st, cross3(a, dpt)));
+        vset(w, orig, 2, group_cso<G, (W::kSV > 0)>(pr.pos, pr.a, pr.b, st, cross3(a, dpt)));
         r.nv = 3;
     }
     lds_order();
@@ -898,7 +1048,7 @@ __device__ uint32_t lazy_begin(W *w, float *orig, const EpaProblem &pr, const Ep
             weird = in && !(fabsf(dist) <= kFltMax);
             k = in ? -dist : -INFINITY;
         }
-        w->key[sub] = k;
+        set_normal(w, sub, n, k);
     }
     lds_order();
     if (dim == 3) {
@@ -923,14 +1073,23 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
         float kb = -INFINITY;
         uint32_t ib = 0;
         bool dup = false;
-#pragma unroll 4
-        for (uint32_t f = sub; f < r.nf; f += G) {
-            float k = w->key[f];
-            const uint32_t x = W::kMask ? 0u : w->px[f];
-            k = face_dead(w, r, f, x) ? -INFINITY : k;
-            dup = k > kb ? false : (k == kb ? true : dup);
-            ib = k > kb ? f : ib;
-            kb = fmaxf(k, kb);
+        for (uint32_t f0 = sub; f0 < r.nf; f0 += 4 * G) {  // four faces' loads in flight
+            float k[4];
+            uint32_t x[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t f = f0 + u * G < r.nf ? f0 + u * G : f0;
+                k[u] = face_key(w, f);
+                x[u] = W::kMask ? 0u : w->face[f].px;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t f = f0 + u * G;
+                const float kk = f >= r.nf || face_dead(w, r, f & (W::kMask ? 63u : ~0u), x[u]) ? -INFINITY : k[u];
+                dup = kk > kb ? false : (kk == kb ? true : dup);
+                ib = kk > kb ? f : ib;
+                kb = fmaxf(kk, kb);
+            }
         }
         fkey = group_max<G>(kb);
         if (fkey == -INFINITY) return EPA_OK;  // parry's heap is empty
@@ -942,10 +1101,10 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
             if (fid == kNoFace) return EPA_RESTART;
         }
     }
-    const uint32_t fx = w->px[fid];
-    const auto fadj = face_adj(w, fid);
-    const f3 fn = f3{w->n[fid][0], w->n[fid][1], w->n[fid][2]};
-    const Cso c = group_cso<G>(pr.pos, pr.a, pr.b, st, fn);
+    const typename W::Face face = w->face[fid];
+    const uint32_t fx = face.px;
+    const f3 fn = face_normal(w, fid);
+    const Cso c = group_cso<G, (W::kSV > 0)>(pr.pos, pr.a, pr.b, st, fn);
     const float cand = dot3(c.p, fn);
     uint32_t best_t = r.niter == 0 ? fid : r.best_id;  // the heap's first top is parry's first best face
     float max_t = r.max_dist;
@@ -965,7 +1124,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     if constexpr (W::kMask)
         r.dead |= 1ull << fid;
     else
-        w->px[fid] = fx | kDeadBit;
+        w->face[fid].px = fx | kDeadBit;
     lds_order();
     // Face::can_be_seen_by (epa3.rs:153-166) of every face from the new vertex,
     // for each of the three opposite vertices, by the group's lanes in parallel;
@@ -974,75 +1133,78 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     // consecutive faces overlap.
     {
         const float E2 = kEps * 100.0f;
-#pragma unroll 2
-        for (uint32_t f = sub; f < r.nf; f += G) {
-            const uint32_t x = w->px[f];
-            const f3 q0 = vpt(w, pt_at(x, 0)), q1 = vpt(w, pt_at(x, 1)), q2 = vpt(w, pt_at(x, 2));
-            const f3 fnn = f3{w->n[f][0], w->n[f][1], w->n[f][2]};
-            const f3 qs[3] = {q0, q1, q2};
-            uint32_t bits = 0;
+        for (uint32_t f0 = sub; f0 < r.nf; f0 += 2 * G) {  // two faces' loads in flight
+            const uint32_t f[2] = {f0, f0 + G < r.nf ? f0 + G : f0};
+            uint32_t x[2];
+            f3 fnn[2], qs[2][3];
 #pragma unroll
-            for (int opp = 0; opp < 3; ++opp) {
-                const f3 p0 = qs[opp], p1 = qs[(opp + 1) % 3], p2 = qs[(opp + 2) % 3];
-                const bool front = dot3(sub3(c.p, p0), fnn) >= -kEpsTol;
-                const bool flat = norm_sq3(cross3(sub3(p2, p1), sub3(c.p, p1))) <= E2 * E2;  // is_affinely_dependent
-                bits |= (uint32_t)(front | flat) << opp;
+            for (int u = 0; u < 2; ++u) {
+                x[u] = w->face[f[u]].px;
+                fnn[u] = face_normal(w, f[u]);
             }
-            reinterpret_cast<uint8_t *>(&w->px[f])[3] = (uint8_t)(bits | ((x >> 24) & (kDeadBit >> 24)));
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) qs[u][q] = vpt(w, pt_at(x[u], q));
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                uint32_t bits = 0;
+#pragma unroll
+                for (int opp = 0; opp < 3; ++opp) {
+                    const f3 p0 = qs[u][opp], p1 = qs[u][(opp + 1) % 3], p2 = qs[u][(opp + 2) % 3];
+                    const bool front = dot3(sub3(c.p, p0), fnn[u]) >= -kEpsTol;
+                    const bool flat = norm_sq3(cross3(sub3(p2, p1), sub3(c.p, p1))) <= E2 * E2;  // is_affinely_dependent
+                    bits |= (uint32_t)(front | flat) << opp;
+                }
+                reinterpret_cast<uint8_t *>(&w->face[f[u]].px)[3] =
+                    (uint8_t)(bits | ((x[u] >> 24) & (kDeadBit >> 24)));
+            }
         }
     }
     lds_order();
     // compute_silhouette (epa3.rs:653-675) for the three neighbours in order
     // adj[0], adj[1], adj[2]; a visible face recurses into adj[(opp + 2) % 3],
     // then adj[opp].  The recursion is an explicit stack of (face, the point its
-    // opposite vertex follows) whose top entry lives in a register.  A step is one
-    // read of the visited face, and both ways on (into a deleted face's first far
-    // neighbour, or back to the stack's top) end in that same read, so the groups
-    // of a wave take their steps together.
+    // opposite vertex follows) with its top entry kept in a register as well.  A
+    // step is one read of the visited face and no branch: what a step does not do
+    // (record an edge, push) is written to a spare slot, and running out of a
+    // buffer ends the loop.  With branches a step took the wave about 550 cycles.
     uint32_t ns = 0, ndel = 0, depth = 2;
-    uint32_t cur = adj_at<W>(fadj, 0) | (pt_at(fx, 0) << W::kShift);
-    uint32_t top = adj_at<W>(fadj, 1) | (pt_at(fx, 1) << W::kShift);
-    w->stk[0] = (E)(adj_at<W>(fadj, 2) | (pt_at(fx, 2) << W::kShift));
-    bool room = true;
+    uint32_t cur = walk_entry<W>(face, 0), top = walk_entry<W>(face, 1);
+    w->stk[0] = (E)walk_entry<W>(face, 2);
+    w->stk[1] = (E)top;
+    bool ended;
     for (;;) {
         const uint32_t id = cur & kIdMask, pt = cur >> W::kShift;
-        const uint32_t x = w->px[id];
-        const auto a = face_adj(w, id);
+        const typename W::Face f = w->face[id];
         const uint32_t below = w->stk[depth > 2u ? depth - 2u : 0u];
-        const uint32_t opp = pt_at(x, 0) == pt ? 1u : (pt_at(x, 1) == pt ? 2u : 0u);  // next_ccw_pt_id
-        const bool live = !face_dead(w, r, id, x);
-        const bool vis = ((x >> (24u + opp)) & 1u) != 0u;
-        const bool del = live && vis;
-        if (live && !vis) {
-            if (ns >= (uint32_t)W::kS) {
-                room = false;
-                break;
-            }
-            w->sil[ns++] = (E)(id | (opp << W::kShift));
-        }
-        if (!del && depth == 0) break;
-        if (del) {
-            if (depth > (uint32_t)W::kK || (!W::kMask && ndel >= (uint32_t)W::kS)) {
-                room = false;
-                break;
-            }
-            if constexpr (W::kMask) {
-                r.dead |= 1ull << id;
-            } else {
-                w->dl[ndel++] = (I)id;
-                w->px[id] = x | kDeadBit;
-            }
-            const uint32_t k1 = opp == 0u ? 2u : opp - 1u;  // (opp + 2) % 3
-            if (depth > 0) w->stk[depth - 1] = (E)top;
-            top = adj_at<W>(a, opp) | (pt_at(x, opp) << W::kShift);
-            ++depth;
-            cur = adj_at<W>(a, k1) | (pt_at(x, k1) << W::kShift);
+        const bool at0 = pt_at(f.px, 0) == pt, at1 = pt_at(f.px, 1) == pt;
+        const uint32_t opp = at0 ? 1u : (at1 ? 2u : 0u);  // next_ccw_pt_id
+        const uint32_t k1 = at0 ? 0u : (at1 ? 1u : 2u);   // (opp + 2) % 3
+        const bool live = !face_dead(w, r, id, f.px);
+        const bool vis = ((f.px >> (24u + opp)) & 1u) != 0u;
+        const bool del = live & vis, edge = live & !vis;
+        w->sil[edge ? ns : (uint32_t)W::kS] = (E)(id | (opp << W::kShift));
+        ns += edge ? 1u : 0u;
+        if constexpr (W::kMask) {
+            r.dead |= (uint64_t)(del ? 1u : 0u) << id;
         } else {
-            cur = top;
-            top = below;
-            --depth;
+            w->dl[del ? ndel : (uint32_t)W::kS] = (I)id;
+            ndel += del ? 1u : 0u;
+            reinterpret_cast<uint8_t *>(&w->face[id].px)[3] =
+                (uint8_t)((f.px >> 24) | (del ? kDeadBit >> 24 : 0u));
         }
+        ended = !del & (depth == 0u);
+        const uint32_t pushed = walk_entry<W>(f, opp);
+        w->stk[del ? depth : (uint32_t)W::kK] = (E)pushed;
+        cur = del ? walk_entry<W>(f, k1) : top;
+        top = del ? pushed : below;
+        depth += del ? 1u : ~0u;
+        if (ended | (ns >= (uint32_t)W::kS) | (del & (depth >= (uint32_t)W::kK)) |
+            (!W::kMask & (ndel >= (uint32_t)W::kS)))
+            break;
     }
+    const bool room = ended;  // not out of a buffer
     if (room && ns == 0) return EPA_NONE;
     // Room for the new faces: at most one per silhouette edge.
     const uint32_t first_new = r.nf;
@@ -1050,8 +1212,8 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
         if constexpr (W::kMask) {
             r.dead = dead0;
         } else {
-            for (uint32_t k = 0; k < ndel; ++k) w->px[w->dl[k]] &= ~kDeadBit;
-            w->px[fid] &= ~kDeadBit;
+            for (uint32_t k = 0; k < ndel; ++k) w->face[w->dl[k]].px &= ~kDeadBit;
+            w->face[fid].px &= ~kDeadBit;
             lds_order();
         }
         return EPA_OVERFLOW;
@@ -1077,7 +1239,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
         bool alive = false;
         if (q < ns) {
             e = w->sil[q];
-            ex = w->px[e & kIdMask];
+            ex = w->face[e & kIdMask].px;
             alive = !face_dead(w, r, e & kIdMask, ex);
         }
         const uint64_t am = group_ballot<G>(alive);
@@ -1089,9 +1251,9 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
             const uint32_t k1 = opp == 0u ? 2u : opp - 1u, k2 = opp == 2u ? 0u : opp + 1u;
             f3 n, pa;
             in = lazy_face(w, new_id, pt_at(ex, k1), pt_at(ex, k2), sp, ef, new_id + 1, new_id - 1, n, pa);
-            w->adj[ef][k2] = (I)new_id;
+            w->face[ef].adj[k2] = (I)new_id;
             if (in) dist = dot3(n, pa);
-            w->key[new_id] = in ? -dist : -INFINITY;
+            set_normal(w, new_id, n, in ? -dist : -INFINITY);
         }
         n_alive += (uint32_t)__popcll(am);
         const bool closer = in && dist < curr_dist;
@@ -1108,8 +1270,8 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     lds_order();
     r.nf = first_new + n_alive;
     if (first_new == r.nf) return EPA_NONE;
-    w->adj[first_new][2] = (I)(r.nf - 1);
-    w->adj[r.nf - 1][1] = (I)first_new;
+    w->face[first_new].adj[2] = (I)(r.nf - 1);
+    w->face[r.nf - 1].adj[1] = (I)first_new;
     lds_order();
     ++r.niter;
     return r.niter > 100 ? EPA_OK : EPA_RUNNING;  // parry's iteration cap
@@ -1176,20 +1338,24 @@ struct TierArgs {
 // memory latency of both (about 14,000 cycles, a third of an iteration's trip
 // when it was paid whenever one group finished) is paid once for all of them.
 // Measured on 2^20 mixed pairs, whole call, with 8 groups per wave: a turn-over
-// at 1 waiting group 4.64 ms, 3 4.46, 4 4.55, 8 4.63; on 262,144 pairs of
-// polyhedra 1.47, 1.38, 1.38 and 1.37 ms.  A wave reserves list entries from the
-// tier's counter in chunks (one atomic's latency per chunk) and hands them to the
+// at 2 waiting groups 3.82 ms, 3 3.78, 4 3.77, 6 3.81, 8 3.80.  A wave reserves
+// list entries from the tier's counter in chunks (one atomic's latency per chunk)
+// and hands them to the
 // waiting groups by rank; the turn-over is wave-uniform, so the ballot, lane 0's
 // atomic and the readfirstlane run converged.  Everything else is group-uniform,
 // and the cross-lane operations of the EPA code stay within a group.
 //
-// The first tier is bound by latency: an iteration takes a lone wave about
-// 17,000 cycles (support points 6,000, visibility 2,500, silhouette 4,000, new
-// faces 3,800) and the wave's three companions on a SIMD hide only part of it.
+// The first tier is bound by instruction issue (counters on 2^20 mixed pairs: VALU
+// busy 87% of the kernel's SIMD cycles, 1,900 VALU instructions per trip of eight
+// pairs, nine waves per CU), the third by its longest pairs' chains of about 17,000
+// cycles per iteration.  4 lanes per pair in the first tier measured 4.18 ms on
+// the mixed pairs against 3.37 with 8 and 3.9 with 16 (the lanes of a wave take
+// the longest walk of its pairs); the second tier with 8 lanes 3.56 against 3.32
+// with 16.
 template <int G, class W, class RI, class RO, int MINW>
 __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI *recs, RecSink<RO> sink) {
     constexpr uint32_t kGroups = 64 / G;
-    constexpr uint32_t kTurnover = kGroups > 2 ? kGroups / 2 : 1;
+        constexpr uint32_t kTurnover = kGroups > 2 ? kGroups / 2 : 1;
     __shared__ W w[kGroups];
     const uint32_t group = threadIdx.x / G;
     const uint32_t sub = __lane_id() % G;
@@ -1255,12 +1421,14 @@ __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI
     }
 }
 
-// First tier: LDS for about eight waves per CU, deleted flags in registers.  Its
+// First tier: LDS for ten waves per CU, deleted flags in registers.  The odd
+// multiple of 16 bytes per polytope keeps a wave's eight polytopes off each
+// other's LDS banks.  Its
 // polytopes move on to the second tier (four pairs per wave), those to the third
 // (one wave per pair, room for parry's 100 iterations).
-using LazySmall = LazyState<20, 64, 20, 24, uint8_t, 0>;
-using LazyWide = LazyState<48, 192, 48, 64, uint8_t, 0>;
-using LazyWave = LazyState<112, 768, 128, 512, uint16_t, 64>;
+using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0>;
+using LazyWide = LazyState<36, 140, 36, 64, uint8_t, 0>;
+using LazyWave = LazyState<112, 768, 128, 256, uint16_t, 64>;
 using SmallRec = EpaRec<LazySmall::kV, LazySmall::kF>;
 using WideRec = EpaRec<LazyWide::kV, LazyWide::kF>;
 
@@ -1493,7 +1661,7 @@ __device__ uint32_t epa_begin(W *w, float *orig, const iso &pos12, const ShapeRe
                 const f3 dpt = sub3(vpt(w, 1), vpt(w, 0));
                 f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.0f, -dpt.x} : f3{0.0f, -dpt.z, dpt.y};
                 a = div3(a, sqrtf(norm_sq3(a)));
-                vset(w, orig, 2, group_cso<G>(pos12, g1, g2, st, cross3(a, dpt)));
+                vset(w, orig, 2, group_cso<G, (W::kSV > 0)>(pos12, g1, g2, st, cross3(a, dpt)));
                 nv = 3;
             }
             face_new(w, 0, 0, 1, 2, 1, 1, 1);
@@ -1537,7 +1705,7 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
         const float fnd = w->heap_nd[0];
         const typename W::Face face = w->face[fid];
         const f3 fn = f3{face.n[0], face.n[1], face.n[2]};
-        const Cso c = group_cso<G>(pos12, g1, g2, st, fn);
+        const Cso c = group_cso<G, (W::kSV > 0)>(pos12, g1, g2, st, fn);
         if (nv >= (uint32_t)W::kV) return EPA_OVERFLOW;
         const uint32_t sp = nv;  // counted when the iteration commits
         vset(w, orig, sp, c);
@@ -1813,6 +1981,9 @@ hipEvent_t g_contact_phase_events[kContactPhases + 1] = {};
 namespace {
 struct ContactWorkspace {
     uint32_t *counters;  // list lengths and the tiers' next entries (reset_counters_kernel)
+    uint32_t *totals, *taken;  // per class of pairs, after the counters
+    uint32_t *order;
+    uint16_t *cls;
     EpaItem *queue;
     uint32_t *lists[4];
     uint32_t *cont_list[2];  // per entry of lists[0] and lists[1]: its continuation record or kNoCont
@@ -1823,6 +1994,18 @@ struct ContactWorkspace {
     float *orig_small, *orig_wide, *orig_wave, *orig_big, *orig_large;
     size_t bytes;
 };
+
+// Whether the pairs are ordered by class: where there are enough of them to fill
+// the GPU several times over (below that a call lasts as long as its longest
+// pairs, in any order) and the shapes are of several types.  Measured, ordered
+// and not, us a call: mixed types 1,313 and 1,318 at 32,000 pairs, 1,450 and 1,460
+// at 128,000, 3,770 and 4,444 at 2^20; polyhedra alone 480 and 443 at 32,000, 780
+// and 734 at 128,000 (the two ordering kernels take 20 us, and the broadphase's
+// order has its own locality).
+constexpr uint64_t kOrderMinPairs = 1u << 17;
+bool takes_order(const DeviceShapes &s, uint64_t m) {
+    return m >= kOrderMinPairs && (s.types & (s.types - 1u)) != 0u;
+}
 
 uint64_t clamp_u64(uint64_t v, uint64_t lo, uint64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
@@ -1839,7 +2022,12 @@ ContactWorkspace carve_workspace(void *base, uint64_t m) {
         off += up(bytes);
         return p;
     };
-    w.counters = (uint32_t *)take(kNumCounters * sizeof(uint32_t));
+    w.counters = (uint32_t *)take((kNumCounters + 2 * kPairClasses) * sizeof(uint32_t));
+    w.totals = w.counters + kNumCounters;
+    w.taken = w.totals + kPairClasses;
+    const uint64_t ordered = m >= kOrderMinPairs ? m : 0;  // whatever the types: the size depends on m alone
+    w.order = (uint32_t *)take(ordered * sizeof(uint32_t));
+    w.cls = (uint16_t *)take(ordered * sizeof(uint16_t));
     w.queue = (EpaItem *)take(m * sizeof(EpaItem));
     for (uint32_t *&l : w.lists) l = (uint32_t *)take(m * sizeof(uint32_t));
     for (uint32_t *&l : w.cont_list) l = (uint32_t *)take(m * sizeof(uint32_t));
@@ -1874,12 +2062,21 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
     DevContact *o = (DevContact *)out;
     const bool timed = g_contact_phase_timing;
     auto mark = [&](int k) { return timed ? hipEventRecord(g_contact_phase_events[k], stream) : hipSuccess; };
-    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, stream, w.counters);
+    const bool ordered = takes_order(s, m);
+    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(256), 0, stream, w.counters,
+                       kNumCounters + (ordered ? 2 * kPairClasses : 0u));
     hipError_t e = mark(0);
     if (e != hipSuccess) return e;
+    if (ordered) {
+        const dim3 grid((uint32_t)((m + kOrderRange - 1) / kOrderRange));
+        hipLaunchKernelGGL(order_count_kernel, grid, dim3(kOrderBlock), 0, stream, s.rec, pairs, m,
+                           (const unsigned long long *)m_dev, w.cls, w.totals);
+        hipLaunchKernelGGL(order_scatter_kernel, grid, dim3(kOrderBlock), 0, stream, m,
+                           (const unsigned long long *)m_dev, w.cls, w.totals, w.taken, w.order);
+    }
     hipLaunchKernelGGL(contact_gjk_kernel, dim3((uint32_t)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
                        s.rec, s.verts, poses, pairs, m, (const unsigned long long *)m_dev, prediction, seeds, o, iters,
-                       w.queue, w.counters, flags);
+                       w.queue, w.counters, flags, ordered ? w.order : nullptr);
     e = hipGetLastError();
     if (e == hipSuccess) e = mark(1);
     if (e != hipSuccess) return e;
@@ -1901,7 +2098,7 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
         default: e = launch_small<64>(t0, small_sink, m, stream); break;
     }
     if (e != hipSuccess) return e;
-    e = launch_lazy<16, LazyWide, SmallRec, WideRec, 2>(tier(1, w.orig_wide), w.small_recs,
+    e = launch_lazy<16, LazyWide, SmallRec, WideRec, 3>(tier(1, w.orig_wide), w.small_recs,
                                                         RecSink<WideRec>{w.wide_recs, c + 11, w.wide_cap}, m,
                                                         kWideGroups, stream);
     if (e == hipSuccess) e = mark(2);

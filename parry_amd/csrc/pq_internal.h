@@ -172,6 +172,7 @@ struct DeviceShapes {
     const float4 *verts;     // device, xyz + pad
     uint32_t n;
     uint32_t num_vertices;
+    uint32_t types;  // one bit per shape type present
     // ConvexPolyhedron faces (null until pq_shapes_set_polyhedron_faces); a
     // polyhedron's record holds its first face and face count in param[0] and
     // param[1] as uint32 bit patterns.

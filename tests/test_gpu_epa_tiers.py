@@ -68,3 +68,36 @@ def test_epa_tiers_match_oracle(orc, make, types):
         assert np.array_equal(out[hit, :13] + 0.0, ref["out"][hit] + 0.0)
         assert np.array_equal(iters[:, 0], ref["iters"][:, 0].astype(np.int32))
         print(f"  {hit.sum()} contacts, EPA iterations up to {ref['iters'][:, 1].max()}")
+
+
+@pytest.mark.parametrize("m,count", [(131071, None), (131072, None), (131072, 1), (140001, 131000), (135169, 0)])
+def test_ordered_pairs_match_unordered(m, count):
+    """From 131,072 pairs of several shape types on, the pairs are taken class by class: every pair's record is the
+    one a small call writes, and slots at or beyond a device-side count are left alone."""
+    import ctypes
+
+    import torch
+
+    from parry_amd import _native, contact_workspace_bytes, scenes
+
+    print(f"case: {m} mixed pairs, count {count}", flush=True)
+    sc = scenes.mixed_scene(900, seed=5)
+    n = 4000
+    rng = np.random.default_rng(2)
+    base = rng.integers(0, 900, (n, 2)).astype(np.int32)
+    shapes, poses = ShapeSet(sc["descs"], sc["vertices"]), torch.from_numpy(sc["poses"]).cuda()
+    want = contact_pairs(shapes, poses, torch.from_numpy(base).cuda(), 0.5, check_indices=False)
+    pick = torch.from_numpy(rng.integers(0, n, m)).cuda()
+    pairs = torch.from_numpy(base).cuda()[pick].contiguous()
+    out = torch.full((m, 14), -7.0, device="cuda")
+    if count is None:
+        contact_pairs(shapes, poses, pairs, 0.5, out=out, check_indices=False)
+    else:
+        ws = torch.empty(contact_workspace_bytes(m), dtype=torch.uint8, device="cuda")
+        dev_count = torch.tensor([count], dtype=torch.int64, device="cuda")
+        _native.check(_native.lib().pq_contact_pairs_device_count(
+            shapes.handle, poses.data_ptr(), pairs.data_ptr(), m, dev_count.data_ptr(), 0.5, None, out.data_ptr(), None,
+            ws.data_ptr(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    k = m if count is None else count
+    assert torch.equal(out[:k].view(torch.int32), want[pick[:k]].view(torch.int32))
+    assert bool((out[k:] == -7.0).all())
