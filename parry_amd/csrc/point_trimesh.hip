@@ -6,9 +6,17 @@
 // point's distance to a child's AABB as node cost (Aabb::distance_to_local_point,
 // solid = true, point_aabb.rs:135-146) and the distance to the point's
 // projection on the triangle as leaf cost (Triangle::project_local_point,
-// point_triangle.rs:54-291).  One lane per point, the ray kernel's node
-// fetches (four 16-byte loads of the 64-byte wide record) and its LDS stack;
-// the chosen triangle and the projection are bit-identical to parry3d's.
+// point_triangle.rs:54-291).  The chosen triangle and the projection are
+// bit-identical to parry3d's.
+//
+// Two mappings.  One lane per point with the ray kernel's node fetches (four
+// 16-byte loads of the 64-byte wide record) and LDS stack, over points sorted by
+// grid cell so that a wave's lanes walk similar paths.  And one wave per point for
+// small calls and for the points whose walk is long: a point near the middle of a
+// closed mesh has most of the surface at nearly the same distance, and on an
+// 81,920-triangle sphere one of 262,147 points visits 8,100 nodes where the mean
+// is 134, so that the call lasted as long as that one lane's chain of fetches
+// (3.1 ms).  A lane gives up after some nodes and leaves its point to a wave.
 #include <cfloat>
 
 #include "contact_gjk.h"
@@ -31,46 +39,67 @@ __device__ __forceinline__ float aabb_point_dist(float mnx, float mny, float mnz
 struct PtBest {
     float cost;
     f3 p;
-    bool inside;
     uint32_t leaf;
     bool have;
 };
 
-// A leaf of find_best: replaces the best only if strictly closer.
-__device__ __forceinline__ void visit_leaf(const float4 *tri4, uint32_t leaf, f3 pt, bool solid, PtBest &b) {
-    const float4 q0 = tri4[3 * leaf], q1 = tri4[3 * leaf + 1], q2 = tri4[3 * leaf + 2];
-    bool inside = false;
-    const f3 p = tri_project(f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, pt, solid, inside);
-    const float cost = sqrtf(norm_sq3(sub3(pt, p)));  // na::distance
-    if (cost < b.cost) {
-        b.cost = cost;
-        b.p = p;
-        b.inside = inside;
-        b.leaf = leaf;
-        b.have = true;
+// Triangle::project_local_point's point (tri_project's, bit for bit).  The regions
+// are selected, not branched to: the lanes of a wave project onto triangles in
+// every region, and took all of tri_project's branches with a division each.
+__device__ __forceinline__ f3 tri_point(f3 a, f3 b, f3 c, f3 pt, bool solid) {
+    const f3 ab = sub3(b, a), ac = sub3(c, a), bc = sub3(c, b);
+    const f3 ap = sub3(pt, a), bp = sub3(pt, b), cp = sub3(pt, c);
+    const float ab_ap = dot3(ab, ap), ac_ap = dot3(ac, ap);
+    const float ab_bp = dot3(ab, bp), ac_bp = dot3(ac, bp);
+    const float ab_cp = dot3(ab, cp), ac_cp = dot3(ac, cp);
+    const f3 n = cross3(ab, ac);
+    const float vc = dot3(n, cross3(ab, ap)), vb = -dot3(n, cross3(ac, cp)), va = dot3(n, cross3(bc, bp));
+    const bool at_a = (ab_ap <= 0.0f) & (ac_ap <= 0.0f);
+    const bool at_b = !at_a & (ab_bp >= 0.0f) & (ac_bp <= ab_bp);
+    const bool at_c = !at_a & !at_b & (ac_cp >= 0.0f) & (ab_cp <= ac_cp);
+    const bool vertex = at_a | at_b | at_c;
+    const bool on_ab = !vertex & (vc < 0.0f) & (ab_ap >= 0.0f) & (ab_bp <= 0.0f);
+    const bool on_ac = !vertex & !on_ab & (vb < 0.0f) & (ac_ap >= 0.0f) & (ac_cp <= 0.0f);
+    const bool on_bc =
+        !vertex & !on_ab & !on_ac & (va < 0.0f) & (ac_bp - ab_bp >= 0.0f) & (ab_cp - ac_cp >= 0.0f);
+    const bool edge = on_ab | on_ac | on_bc;
+    const float sum = va + vb + vc;
+    const f3 base = sel2(at_b | on_bc, b, sel2(at_c, c, a));
+    const f3 dir = sel2(on_ab, ab, sel2(on_ac, ac, bc));
+    const float t = (on_ab ? ab_ap : (on_ac ? ac_ap : dot3(bc, bp))) / norm_sq3(dir);
+    const float denom = 1.0f / sum;
+    const f3 face = add3(add3(a, mul3(ab, vb * denom)), mul3(ac, vc * denom));
+    f3 r = sel2(vertex, base, sel2(edge, add3(base, mul3(dir, t)), face));
+    if (!(vertex | edge) && !(sum != 0.0f)) {  // a degenerate triangle
+        bool inside;
+        r = tri_project(a, b, c, pt, solid, inside);
     }
+    return r;
 }
 
-// COUNT = true also writes, per point, the wide-node records fetched and the
-// triangles tested (the traffic model of the roofline figure).
-template <bool COUNT>
-__global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_node_wide *__restrict__ nodes,
-                                                                  const TriRecord *__restrict__ tris,
-                                                                  const float *__restrict__ points, uint64_t n,
-                                                                  int solid_flag,
-                                                                  pq_point_projection *__restrict__ out,
-                                                                  uint32_t *__restrict__ counts) {
-    extern __shared__ uint32_t lds_stack[];
-    const uint64_t i = (uint64_t)blockIdx.x * kPtBlock + threadIdx.x;
-    if (i >= n) return;
-    uint32_t *stk = lds_stack + threadIdx.x;
-    const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
-    const float4 *tri4 = reinterpret_cast<const float4 *>(tris);
-    const bool solid = solid_flag != 0;
-    const f3 pt{points[3 * i], points[3 * i + 1], points[3 * i + 2]};
-    PtBest b{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, false, 0u, false};
-    uint32_t n_wide = 0, n_tri = 0;
+// A leaf's projection and its cost (na::distance).
+__device__ __forceinline__ f3 leaf_point(const float4 *tri4, uint32_t leaf, f3 pt, bool solid, float &cost) {
+    const float4 q0 = tri4[3 * (size_t)leaf], q1 = tri4[3 * (size_t)leaf + 1], q2 = tri4[3 * (size_t)leaf + 2];
+    const f3 p = tri_point(f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, pt, solid);
+    cost = sqrtf(norm_sq3(sub3(pt, p)));
+    return p;
+}
 
+// A leaf of find_best: replaces the best only if strictly closer.
+__device__ __forceinline__ void visit_leaf(const float4 *tri4, uint32_t leaf, f3 pt, bool solid, PtBest &b) {
+    float cost;
+    const f3 p = leaf_point(tri4, leaf, pt, solid, cost);
+    const bool closer = cost < b.cost;
+    b.cost = closer ? cost : b.cost;
+    b.p = sel2(closer, p, b.p);
+    b.leaf = closer ? leaf : b.leaf;
+    b.have = b.have | closer;
+}
+
+// find_best from the root, by one lane; `stk` with stride `stride`.
+template <bool COUNT>
+__device__ __forceinline__ void walk(const float4 *node4, const float4 *tri4, f3 pt, bool solid, uint32_t *stk,
+                                     uint32_t stride, PtBest &b, uint32_t &n_wide, uint32_t &n_tri) {
     const float4 root3 = node4[3];
     if ((__float_as_uint(root3.w) & 0x3fffffffu) == 0u) {  // partial root, bvh_traverse.rs:348-359
         const float4 q0 = node4[0], q1 = node4[1];
@@ -79,69 +108,142 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
             ++n_tri;
             visit_leaf(tri4, __float_as_uint(q0.w), pt, solid, b);
         }
-    } else {
-        uint32_t curr = 0, sp = 0;
-        for (;;) {
-            if (COUNT) ++n_wide;
-            const float4 q0 = node4[4 * curr + 0];  // left mins, left children
-            const float4 q1 = node4[4 * curr + 1];  // left maxs, left data
-            const float4 q2 = node4[4 * curr + 2];  // right mins, right children
-            const float4 q3 = node4[4 * curr + 3];  // right maxs, right data
-            float ls = aabb_point_dist(q0.x, q0.y, q0.z, q1.x, q1.y, q1.z, pt);
-            float rs = aabb_point_dist(q2.x, q2.y, q2.z, q3.x, q3.y, q3.z, pt);
-            uint32_t lc = __float_as_uint(q0.w), ld = __float_as_uint(q1.w);
-            uint32_t rc = __float_as_uint(q2.w), rd = __float_as_uint(q3.w);
-            if (ls > rs) {
-                const float tf = ls;
-                ls = rs;
-                rs = tf;
-                const uint32_t tc = lc;
-                lc = rc;
-                rc = tc;
-                const uint32_t td = ld;
-                ld = rd;
-                rd = td;
+        return;
+    }
+    uint32_t curr = 0, sp = 0;
+    for (;;) {
+        if (COUNT) ++n_wide;
+        const float4 q0 = node4[4 * curr + 0];  // left mins, left children
+        const float4 q1 = node4[4 * curr + 1];  // left maxs, left data
+        const float4 q2 = node4[4 * curr + 2];  // right mins, right children
+        const float4 q3 = node4[4 * curr + 3];  // right maxs, right data
+        float ls = aabb_point_dist(q0.x, q0.y, q0.z, q1.x, q1.y, q1.z, pt);
+        float rs = aabb_point_dist(q2.x, q2.y, q2.z, q3.x, q3.y, q3.z, pt);
+        uint32_t lc = __float_as_uint(q0.w), ld = __float_as_uint(q1.w);
+        uint32_t rc = __float_as_uint(q2.w), rd = __float_as_uint(q3.w);
+        if (ls > rs) {
+            const float tf = ls;
+            ls = rs;
+            rs = tf;
+            const uint32_t tc = lc;
+            lc = rc;
+            rc = tc;
+            const uint32_t td = ld;
+            ld = rd;
+            rd = td;
+        }
+        // one latch: into a child, or back to the stack's top, by selects
+        const uint32_t below = stk[(sp != 0u ? sp - 1u : 0u) * stride];
+        const bool near_leaf = (ld & 0x3fffffffu) == 1u, far_leaf = (rd & 0x3fffffffu) == 1u;
+        const bool near_in = ls < b.cost && ls != FLT_MAX;
+        if (near_in && near_leaf) {
+            if (COUNT) ++n_tri;
+            visit_leaf(tri4, lc, pt, solid, b);
+        }
+        const bool far_in = rs < b.cost && rs != FLT_MAX;
+        if (far_in && far_leaf) {
+            if (COUNT) ++n_tri;
+            visit_leaf(tri4, rc, pt, solid, b);
+        }
+        const bool go_near = near_in && !near_leaf, go_far = far_in && !far_leaf;
+        if (go_near && go_far) stk[sp * stride] = rc;
+        const bool pop = !go_near && !go_far;
+        if (pop && sp == 0u) return;
+        curr = go_near ? lc : (go_far ? rc : below);
+        sp = go_near && go_far ? sp + 1u : (pop ? sp - 1u : sp);
+    }
+}
+
+// Whether the projection on a triangle lies in the triangle's box.  Costs are then
+// monotone down the tree: box cost and leaf cost are sums of squares of the same
+// form, and float subtraction, product, sum and root are monotone, so the leaf
+// costs no less than its box, and no less than any box above it (where the boxes
+// are nested, MeshBounds).
+__device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, f3 p) {
+    const float4 q0 = tri4[3 * (size_t)leaf], q1 = tri4[3 * (size_t)leaf + 1], q2 = tri4[3 * (size_t)leaf + 2];
+    const f3 a{q0.x, q0.y, q0.z}, b{q0.w, q1.x, q1.y}, c{q1.z, q1.w, q2.x};
+    const f3 mn = min3(min3(a, b), c), mx = max3(max3(a, b), c);
+    return p.x >= mn.x && p.y >= mn.y && p.z >= mn.z && p.x <= mx.x && p.y <= mx.y && p.z <= mx.z;
+}
+
+// find_best by one lane, with the leaves put aside: a lane reaches a leaf at one
+// node in ten, so some lane of a wave did at nearly every node, and each node cost
+// the wave two projections (2.2 us per node, two thirds of it for them).  Up to four
+// leaves wait in registers, and the wave projects the first of every lane when one
+// lane has more than two.  Returns false if the walk passes `limit` nodes or its
+// answer is not known to be find_best's.
+//
+// The nodes are taken in find_best's order with a best cost that is late, so this
+// walk sees find_best's leaves and a few more, in its order.  If the projection of
+// the first leaf W of smallest cost lies in W's box, find_best takes W too: each
+// leaf before it costs more than W, so no box above W costs as much as the best
+// cost find_best has there, and nothing after W costs less.
+__device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 *tri4, f3 pt, bool solid, uint32_t *stk,
+                                              uint32_t stride, uint32_t limit, PtBest &b) {
+    uint32_t curr = 0, sp = 0, n = 0, steps = 0;
+    uint32_t l0 = 0, l1 = 0, l2 = 0, l3 = 0;
+    bool walking = true;
+    auto put = [&](bool add, uint32_t leaf) {
+        l0 = add && n == 0u ? leaf : l0;
+        l1 = add && n == 1u ? leaf : l1;
+        l2 = add && n == 2u ? leaf : l2;
+        l3 = add && n == 3u ? leaf : l3;
+        n += add ? 1u : 0u;
+    };
+    for (;;) {
+        // A node adds two leaves at most: wave-uniform, so that the lanes keep step.
+        const bool leaves = __any(n > 2u) || !__any(walking);
+        if (!leaves && walking) {
+            const float4 q0 = node4[4 * (size_t)curr + 0];  // left mins, left children
+            const float4 q1 = node4[4 * (size_t)curr + 1];  // left maxs, left data
+            const float4 q2 = node4[4 * (size_t)curr + 2];  // right mins, right children
+            const float4 q3 = node4[4 * (size_t)curr + 3];  // right maxs, right data
+            const uint32_t below = stk[(sp != 0u ? sp - 1u : 0u) * stride];
+            const float cl = aabb_point_dist(q0.x, q0.y, q0.z, q1.x, q1.y, q1.z, pt);
+            const float cr = aabb_point_dist(q2.x, q2.y, q2.z, q3.x, q3.y, q3.z, pt);
+            const bool swap = cl > cr;
+            const float ls = swap ? cr : cl, rs = swap ? cl : cr;
+            const uint32_t lc = __float_as_uint(swap ? q2.w : q0.w), rc = __float_as_uint(swap ? q0.w : q2.w);
+            const uint32_t ld = __float_as_uint(swap ? q3.w : q1.w), rd = __float_as_uint(swap ? q1.w : q3.w);
+            const bool near_leaf = (ld & 0x3fffffffu) == 1u, far_leaf = (rd & 0x3fffffffu) == 1u;
+            const bool near_in = (ls < b.cost) & (ls != FLT_MAX), far_in = (rs < b.cost) & (rs != FLT_MAX);
+            put(near_in & near_leaf, lc);
+            put(far_in & far_leaf, rc);
+            const bool go_near = near_in & !near_leaf, go_far = far_in & !far_leaf;
+            if (go_near & go_far) stk[sp * stride] = rc;
+            const bool pop = !go_near & !go_far;
+            walking = !(pop & (sp == 0u));
+            curr = go_near ? lc : (go_far ? rc : below);
+            sp = (go_near & go_far) ? sp + 1u : (pop ? sp - 1u : sp);
+            if (++steps > limit) return false;
+        }
+        if (leaves) {
+            if (n != 0u) {
+                visit_leaf(tri4, l0, pt, solid, b);
+                l0 = l1;
+                l1 = l2;
+                l2 = l3;
+                --n;
             }
-            bool found_next = false;
-            if (ls < b.cost && ls != FLT_MAX) {
-                if ((ld & 0x3fffffffu) == 1u) {
-                    if (COUNT) ++n_tri;
-                    visit_leaf(tri4, lc, pt, solid, b);
-                } else {
-                    curr = lc;
-                    found_next = true;
-                }
-            }
-            if (rs < b.cost && rs != FLT_MAX) {
-                if ((rd & 0x3fffffffu) == 1u) {
-                    if (COUNT) ++n_tri;
-                    visit_leaf(tri4, rc, pt, solid, b);
-                } else if (found_next) {
-                    stk[sp * kPtBlock] = rc;
-                    ++sp;
-                } else {
-                    curr = rc;
-                    found_next = true;
-                }
-            }
-            if (!found_next) {
-                if (sp == 0) break;
-                --sp;
-                curr = stk[sp * kPtBlock];
-            }
+            if (!walking && n == 0u) break;
         }
     }
-    if (COUNT) {
-        counts[2 * i] = n_wide;
-        counts[2 * i + 1] = n_tri;
-    }
+    return !b.have || point_in_box(tri4, b.leaf, b.p);
+}
+
+// is_inside comes from the winner's triangle, projected again.
+__device__ __forceinline__ void write_projection(pq_point_projection *out, uint64_t i, const float4 *tri4, f3 pt,
+                                                 bool solid, const PtBest &b) {
     pq_point_projection o;
     if (b.have) {
-        o.point[0] = b.p.x;
-        o.point[1] = b.p.y;
-        o.point[2] = b.p.z;
-        o.is_inside = b.inside ? 1u : 0u;
-        o.triangle = __float_as_uint(tri4[3 * b.leaf + 2].y);
+        const float4 q0 = tri4[3 * (size_t)b.leaf], q1 = tri4[3 * (size_t)b.leaf + 1], q2 = tri4[3 * (size_t)b.leaf + 2];
+        bool inside = false;
+        const f3 p = tri_project(f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, pt, solid, inside);
+        o.point[0] = p.x;
+        o.point[1] = p.y;
+        o.point[2] = p.z;
+        o.is_inside = inside ? 1u : 0u;
+        o.triangle = __float_as_uint(q2.y);
     } else {
         o.point[0] = o.point[1] = o.point[2] = 0.0f;
         o.is_inside = 0u;
@@ -149,6 +251,246 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
     }
     out[i] = o;
 }
+__device__ __forceinline__ f3 load_point(const float *points, uint64_t i) {
+    return f3{points[3 * i], points[3 * i + 1], points[3 * i + 2]};
+}
+
+// COUNT = true also writes, per point, the wide-node records fetched and the
+// triangles tested (the traffic model of the roofline figure).  With LIMIT, points
+// whose walk exceeds `limit` nodes go to `heavy` instead (*num_heavy of them).
+template <bool COUNT, bool LIMIT>
+__global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_node_wide *__restrict__ nodes,
+                                                                  const TriRecord *__restrict__ tris,
+                                                                  const float *__restrict__ points, uint64_t n,
+                                                                  int solid_flag,
+                                                                  pq_point_projection *__restrict__ out,
+                                                                  uint32_t *__restrict__ counts,
+                                                                  const uint32_t *__restrict__ order, uint32_t limit,
+                                                                  uint32_t *__restrict__ heavy,
+                                                                  uint32_t *__restrict__ num_heavy) {
+    extern __shared__ uint32_t lds_stack[];
+    const uint64_t j = (uint64_t)blockIdx.x * kPtBlock + threadIdx.x;
+    if (j >= n) return;
+    const uint64_t i = order ? (uint64_t)order[j] : j;
+    const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
+    const float4 *tri4 = reinterpret_cast<const float4 *>(tris);
+    PtBest b{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};
+    uint32_t n_wide = 0, n_tri = 0;
+    const f3 pt = load_point(points, i);
+    bool done = true;
+    if (LIMIT)
+        done = walk_deferred(node4, tri4, pt, solid_flag != 0, lds_stack + threadIdx.x, kPtBlock, limit, b);
+    else
+        walk<COUNT>(node4, tri4, pt, solid_flag != 0, lds_stack + threadIdx.x, kPtBlock, b, n_wide, n_tri);
+    if (LIMIT) {  // one atomic per wave, by the first lane that gave up
+        const uint64_t left = __ballot(!done);
+        if (left != 0ull) {
+            const uint32_t leader = (uint32_t)__builtin_ctzll(left);
+            uint32_t base = 0;
+            if (__lane_id() == leader) base = atomicAdd(num_heavy, (uint32_t)__popcll(left));
+            base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+            if (!done)
+                heavy[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(left >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u))] = (uint32_t)i;
+        }
+        if (!done) return;
+    }
+    if (COUNT) {
+        counts[2 * i] = n_wide;
+        counts[2 * i + 1] = n_tri;
+    }
+    write_projection(out, i, tri4, pt, solid_flag != 0, b);
+}
+
+// ---------------------------------------------------------------------------
+// One wave per point.  The wave takes up to 64 pending nodes at a time, one per
+// lane, and keeps every child whose box is within the best cost so far plus
+// `slack`.  Let W be, of the leaves of smallest cost, the one find_best reaches
+// first.  If W's projection lies in W's box, find_best's answer is W (as for
+// walk_deferred).  The wave finds W if it sees every leaf that can cost so little:
+// those it does not see lie in a box costing more than best + slack, and cost less
+// than that box by at most their projection's distance outside it, which `slack`
+// bounds (MeshBounds).
+// find_best reaches leaves in the order of a path key: at each node a child leaf
+// before a child node, otherwise the nearer child (the left on ties) first.  The
+// key holds one bit per level from the top, then a marker bit.  A winner whose
+// projection is outside its box, a full stack or a point out of the bound's reach
+// falls back to find_best by lane 0.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kDescentNodes = 8;
+constexpr uint32_t kWaveStack = 1024;
+constexpr uint32_t kWaveMaxDepth = 62;  // path key: levels and a marker in 64 bits
+
+template <int CTRL> __device__ __forceinline__ float min_dpp(float v) {
+    return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float wave_min(float v) {  // no NaN
+    v = min_dpp<0x140>(min_dpp<0x141>(min_dpp<0x4E>(min_dpp<0xB1>(v))));  // the rows of 16
+    const float r[4] = {__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)),
+                        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16)),
+                        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32)),
+                        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48))};
+    return fminf(fminf(r[0], r[1]), fminf(r[2], r[3]));
+}
+__device__ __forceinline__ uint64_t wave_min(uint64_t v) {
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = (uint64_t)__shfl_xor((long long)v, d);
+        v = o < v ? o : v;
+    }
+    return v;
+}
+__device__ __forceinline__ uint32_t rank_below(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+__global__ __launch_bounds__(64) void project_points_wave_kernel(const pq_bvh_node_wide *__restrict__ nodes,
+                                                                 const TriRecord *__restrict__ tris,
+                                                                 const float *__restrict__ points, uint32_t n,
+                                                                 const uint32_t *__restrict__ list,
+                                                                 const uint32_t *__restrict__ list_count,
+                                                                 int solid_flag, MeshBounds bounds,
+                                                                 pq_point_projection *__restrict__ out) {
+    __shared__ uint32_t s_node[kWaveStack];
+    __shared__ float s_cost[kWaveStack];
+    __shared__ uint64_t s_key[kWaveStack];
+    const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
+    const float4 *tri4 = reinterpret_cast<const float4 *>(tris);
+    const bool solid = solid_flag != 0;
+    const uint32_t lane = __lane_id();
+    if (list) n = *list_count;
+    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const uint32_t i = list ? list[q] : q;
+        const f3 pt = load_point(points, i);
+        const float d = fabsf(pt.x) + fabsf(pt.y) + fabsf(pt.z) + 3.0f * bounds.extent;
+        const float slack = bounds.foot * d;
+        PtBest b{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};  // the lane's best
+        uint64_t key = ~0ull;
+        uint32_t sp = 1;
+        float bound = FLT_MAX;
+        bool fits = d <= bounds.reach;
+        if (lane == 0) {
+            s_node[0] = 0u;
+            s_cost[0] = 0.0f;
+            s_key[0] = 1ull << 63;
+        }
+        __syncthreads();  // one wave: orders the LDS accesses below
+        while (fits && sp != 0u) {
+            // each node taken leaves at most two
+            const uint32_t room = kWaveStack - sp;
+            // few nodes at a time until a leaf gives a bound to prune by
+            const uint32_t wide = bound < FLT_MAX ? 64u : kDescentNodes;
+            uint32_t take = sp < wide ? sp : wide;
+            take = take < room ? take : room;
+            if (take == 0u) {
+                fits = false;
+                break;
+            }
+            sp -= take;
+            bool active = lane < take;
+            const uint32_t at = sp + (active ? lane : 0u);
+            const uint32_t node = s_node[at];
+            const uint64_t path = s_key[at];
+            active = active && s_cost[at] <= bound;
+            __syncthreads();
+            bool push_near = false, push_far = false;
+            float ls = FLT_MAX, rs = FLT_MAX;
+            uint32_t lc = 0, rc = 0;
+            uint64_t lk = 0, rk = 0;
+            if (active) {
+                const float4 q0 = node4[4 * (size_t)node + 0], q1 = node4[4 * (size_t)node + 1];
+                const float4 q2 = node4[4 * (size_t)node + 2], q3 = node4[4 * (size_t)node + 3];
+                ls = aabb_point_dist(q0.x, q0.y, q0.z, q1.x, q1.y, q1.z, pt);
+                rs = aabb_point_dist(q2.x, q2.y, q2.z, q3.x, q3.y, q3.z, pt);
+                lc = __float_as_uint(q0.w);
+                rc = __float_as_uint(q2.w);
+                uint32_t ld = __float_as_uint(q1.w) & 0x3fffffffu, rd = __float_as_uint(q3.w) & 0x3fffffffu;
+                const bool swap = ls > rs;
+                if (swap) {
+                    const float tf = ls;
+                    ls = rs;
+                    rs = tf;
+                    const uint32_t tc = lc;
+                    lc = rc;
+                    rc = tc;
+                    const uint32_t td = ld;
+                    ld = rd;
+                    rd = td;
+                }
+                const bool near_leaf = ld == 1u, far_leaf = rd == 1u;
+                const bool far_first = far_leaf && !near_leaf;
+                const uint64_t mark = path & (0ull - path), first = (path ^ mark) | (mark >> 1), second = first | mark;
+                lk = far_first ? second : first;
+                rk = far_first ? first : second;
+                const bool near_in = ls <= bound && ls < FLT_MAX, far_in = rs <= bound && rs < FLT_MAX;
+                push_near = near_in && !near_leaf;
+                push_far = far_in && !far_leaf;
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    if (side == 0 ? !(near_in && near_leaf) : !(far_in && far_leaf)) continue;
+                    const uint32_t leaf = side == 0 ? lc : rc;
+                    const uint64_t lkey = side == 0 ? lk : rk;
+                    float cost;
+                    const f3 p = leaf_point(tri4, leaf, pt, solid, cost);
+                    if (cost < b.cost || (cost == b.cost && b.have && lkey < key)) {
+                        b = PtBest{cost, p, leaf, true};
+                        key = lkey;
+                    }
+                }
+            }
+            // far children below near ones, so that near ones are taken first
+            const uint64_t fm = __ballot(push_far), nm = __ballot(push_near);
+            if (push_far) {
+                const uint32_t o = sp + rank_below(fm);
+                s_node[o] = rc;
+                s_cost[o] = rs;
+                s_key[o] = rk;
+            }
+            sp += (uint32_t)__popcll(fm);
+            if (push_near) {
+                const uint32_t o = sp + rank_below(nm);
+                s_node[o] = lc;
+                s_cost[o] = ls;
+                s_key[o] = lk;
+            }
+            sp += (uint32_t)__popcll(nm);
+            if (__any(b.cost + slack < bound)) bound = wave_min(b.cost) + slack;
+            __syncthreads();
+        }
+        if (fits) {
+            const float cost = wave_min(b.cost);
+            const uint64_t none = ~(uint64_t)0;
+            const uint64_t win = wave_min(b.have && b.cost == cost ? key : none);
+            bool ok = true;
+            if (b.have && key == win) {  // the winner's lane (none if no leaf has a cost)
+                ok = point_in_box(tri4, b.leaf, b.p);
+                if (ok) write_projection(out, i, tri4, pt, solid, b);
+            } else if (win == none && lane == 0) {
+                write_projection(out, i, tri4, pt, solid, b);  // none
+            }
+            fits = __ballot(!ok) == 0ull;
+        }
+        if (!fits && lane == 0) {
+            PtBest s{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};
+            uint32_t n_wide = 0, n_tri = 0;
+            walk<false>(node4, tri4, pt, solid, s_node, 1u, s, n_wide, n_tri);
+            write_projection(out, i, tri4, pt, solid, s);
+        }
+        __syncthreads();
+    }
+}
+
+// Up to this many points a call is waves only: they fill the GPU, and lanes would
+// wait for the longest walk and for the sort.  Measured on the 81,920-triangle
+// sphere, us a call (lanes with their waves / waves only): 1,000 points 376 / 76,
+// 8,000 488 / 205, 16,000 433 / 288, 32,000 479 / 540, 65,536 580 / 1,100.
+constexpr uint64_t kWavePoints = 16384;
+// Nodes a lane walks before it leaves its point to a wave.  A wave spends about
+// 16 ns of the whole GPU on a point; a lane's chain costs 1.2 to 1.7 us per node, which
+// the larger calls hide better.  Measured (limit 192 / 256 / 384): 32,000 points
+// 479 / 546 / 718 us, 65,536 671 / 580 / 749, 262,147 1,425 / 786 / 894, 2^20
+// 4,910 / 2,212 / 1,892.
+uint32_t lane_nodes(uint64_t n) { return n < 49152 ? 192u : (n < 524288 ? 256u : 384u); }
+constexpr uint32_t kWaveGrid = 256 * 10;  // resident waves (LDS: ten per CU)
 
 }  // namespace
 
@@ -157,14 +499,42 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
     if (n == 0) return hipSuccess;
     // The traversal stack never holds more than depth - 1 entries (as for rays).
     const size_t lds = (size_t)ray_stack_entries(m.depth) * kPtBlock * sizeof(uint32_t);
-    const uint64_t blocks = (n + kPtBlock - 1) / kPtBlock;
-    if (counts)
-        hipLaunchKernelGGL(project_points_kernel<true>, dim3((uint32_t)blocks), dim3(kPtBlock), lds, stream, m.nodes,
-                           m.tris, points, n, solid, out, counts);
-    else
-        hipLaunchKernelGGL(project_points_kernel<false>, dim3((uint32_t)blocks), dim3(kPtBlock), lds, stream,
-                           m.nodes, m.tris, points, n, solid, out, counts);
-    return hipGetLastError();
+    const auto grid = [](uint64_t k) { return dim3((uint32_t)((k + kPtBlock - 1) / kPtBlock)); };
+    const uint32_t *const none = nullptr;
+    if (counts) {
+        hipLaunchKernelGGL((project_points_kernel<true, false>), grid(n), dim3(kPtBlock), lds, stream, m.nodes, m.tris,
+                           points, n, solid, out, counts, none, 0u, nullptr, nullptr);
+        return hipGetLastError();
+    }
+    // Waves need the mesh's bound on projections, a tree their keys can hold and two leaves.
+    const bool waves = m.bounds.reach >= 0.0f && m.depth <= kWaveMaxDepth && m.num_triangles > 1;
+    if (waves && n <= kWavePoints) {
+        hipLaunchKernelGGL(project_points_wave_kernel, dim3((uint32_t)n), dim3(64), 0, stream, m.nodes, m.tris, points,
+                           (uint32_t)n, none, none, solid, m.bounds, out);
+        return hipGetLastError();
+    }
+    // The sort's buffers may have to grow, which a capture does not allow.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(stream, &capture);
+    if (e != hipSuccess) return e;
+    if (!waves || capture != hipStreamCaptureStatusNone) {
+        hipLaunchKernelGGL((project_points_kernel<false, false>), grid(n), dim3(kPtBlock), lds, stream, m.nodes, m.tris,
+                           points, n, solid, out, nullptr, none, 0u, nullptr, nullptr);
+        return hipGetLastError();
+    }
+    for (uint64_t at = 0; at < n; at += kPointSortMax) {
+        const uint64_t part = n - at < kPointSortMax ? n - at : kPointSortMax;
+        const float *const pts = points + 3 * at;
+        const uint32_t *order = nullptr;
+        uint32_t *heavy = nullptr, *num_heavy = nullptr;
+        if ((e = launch_point_bins(m, pts, part, stream, &order, &heavy, &num_heavy)) != hipSuccess) return e;
+        hipLaunchKernelGGL((project_points_kernel<false, true>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
+                           m.tris, pts, part, solid, out + at, nullptr, order, lane_nodes(part), heavy, num_heavy);
+        hipLaunchKernelGGL(project_points_wave_kernel, dim3(kWaveGrid), dim3(64), 0, stream, m.nodes, m.tris, pts, 0u,
+                           (const uint32_t *)heavy, (const uint32_t *)num_heavy, solid, m.bounds, out + at);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace pq

@@ -59,6 +59,14 @@ struct alignas(16) TriRecord {
 static_assert(sizeof(TriRecord) == 48, "TriRecord is 48 bytes");
 static_assert(sizeof(pq_bvh_node_wide) == 64, "wide node is 64 bytes");
 
+// How far a computed projection on a triangle can lie outside the triangle's box,
+// for points p with |p|_1 + 3 * extent <= reach: foot * (|p|_1 + 3 * extent).
+// reach < 0: no bound (a degenerate triangle, non-finite values, or a tree whose
+// boxes do not enclose their contents).  See mesh_bounds.
+struct MeshBounds {
+    float extent, foot, reach;
+};
+
 struct DeviceMesh {
     const pq_bvh_node_wide *nodes;  // device, leaf children -> TriRecord index
     const TriRecord *tris;          // device
@@ -67,6 +75,7 @@ struct DeviceMesh {
     uint32_t depth;
     uint32_t finite;  // every vertex and every node bound is finite
     pq_ray_tuning tuning;
+    MeshBounds bounds;
 };
 
 // One mesh of a batch, as the batched kernels see it.
@@ -129,6 +138,7 @@ struct RayBinSpace {
     uint32_t *totals;
     uint32_t *keyrank;
     uint32_t *order;
+    uint32_t *count;
 };
 hipError_t ray_bin_workspace(hipStream_t stream, uint64_t num_rays, uint32_t blocks, RayBinSpace *ws);
 
@@ -152,6 +162,12 @@ hipError_t launch_cast_rays_culling(const DeviceMesh &m, const pq_ray *rays, uin
                                     uint32_t culling, pq_ray_hit *hits, uint32_t *counts, hipStream_t stream);
 // Point projections onto the mesh (point_trimesh.hip); solid as in parry.
 // `counts` (nullable, device, 2 per point): wide-node records fetched, triangles tested.
+// Sorts the points by the cell of a grid over the mesh's root box: *order holds the
+// point index at each sorted position, *spare room for n indices and *count a
+// zeroed counter (buffers of the stream, valid until its next sort).
+constexpr uint64_t kPointSortMax = 1ull << 22;  // points of one sort (bounds its buffers)
+hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t n, hipStream_t stream,
+                             const uint32_t **order, uint32_t **spare, uint32_t **count);
 hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint64_t n, int solid,
                                  pq_point_projection *out, uint32_t *counts, hipStream_t stream);
 

@@ -1048,6 +1048,41 @@ __global__ __launch_bounds__(kCountBlock) void bin_count_kernel(const pq_bvh_nod
     for (uint32_t c = threadIdx.x; c < kRayBins; c += kCountBlock) hist[(uint64_t)blockIdx.x * kRayBins + c] = cnt[c];
 }
 
+// Points: the same ranges, the cell on a grid over one and a half times the root
+// box (points farther out take the nearest cell).  Also zeroes *count.
+__global__ __launch_bounds__(kCountBlock) void bin_count_points_kernel(const pq_bvh_node_wide *__restrict__ nodes,
+                                                                       const float *__restrict__ points, uint64_t n,
+                                                                       uint64_t per_block, uint32_t *__restrict__ hist,
+                                                                       uint32_t *__restrict__ keyrank,
+                                                                       uint32_t *__restrict__ count) {
+    __shared__ uint32_t cnt[kRayBins];
+    for (uint32_t c = threadIdx.x; c < kRayBins; c += kCountBlock) cnt[c] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0u;
+    __syncthreads();
+    const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
+    const float4 q0 = node4[0], q1 = node4[1], q2 = node4[2], q3 = node4[3];
+    const bool two = (__float_as_uint(q3.w) & 0x3fffffffu) != 0u;
+    const float mn[3] = {two ? fminf(q0.x, q2.x) : q0.x, two ? fminf(q0.y, q2.y) : q0.y,
+                         two ? fminf(q0.z, q2.z) : q0.z};
+    const float mx[3] = {two ? fmaxf(q1.x, q3.x) : q1.x, two ? fmaxf(q1.y, q3.y) : q1.y,
+                         two ? fmaxf(q1.z, q3.z) : q1.z};
+    const uint64_t begin = (uint64_t)blockIdx.x * per_block;
+    const uint64_t end = begin + per_block < n ? begin + per_block : n;
+    for (uint64_t j = begin + threadIdx.x; j < end; j += kCountBlock) {
+        uint32_t q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float ext = 1.5f * (mx[a] - mn[a]), lo = 0.5f * (mn[a] + mx[a]) - 0.5f * ext;
+            const float u = ext > 0.0f ? (points[3 * j + a] - lo) / ext * (float)(1u << kRayBinBits) : 0.0f;
+            q[a] = (uint32_t)fminf(fmaxf(u, 0.0f), (float)((1u << kRayBinBits) - 1u));  // NaN -> 0
+        }
+        const uint32_t cell = (spread3(q[0]) << 2) | (spread3(q[1]) << 1) | spread3(q[2]);
+        keyrank[j] = cell | (atomicAdd(&cnt[cell], 1u) << kRayBinKeyBits);
+    }
+    __syncthreads();
+    for (uint32_t c = threadIdx.x; c < kRayBins; c += kCountBlock) hist[(uint64_t)blockIdx.x * kRayBins + c] = cnt[c];
+}
+
 // A batch: one workgroup per sort range; range r holds rays of mesh
 // range_mesh[r] only, and the cells are those of that mesh's root box.
 __global__ __launch_bounds__(kCountBlock) void bin_count_batch_kernel(
@@ -1250,6 +1285,26 @@ hipError_t persistent_blocks(const void *kernel, int block, size_t lds, const pq
 }
 
 }  // namespace
+
+hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t n, hipStream_t stream,
+                             const uint32_t **order, uint32_t **spare, uint32_t **count) {
+    if (n > kPointSortMax) return hipErrorInvalidValue;
+    const uint32_t blocks = (uint32_t)((n + kBinRange - 1) / kBinRange);
+    RayBinSpace ws{};
+    hipError_t e = ray_bin_workspace(stream, n, blocks, &ws);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(bin_count_points_kernel, dim3(blocks), dim3(kCountBlock), 0, stream, m.nodes, points, n,
+                       (uint64_t)kBinRange, ws.hist, ws.keyrank, ws.count);
+    hipLaunchKernelGGL(bin_scan_kernel, dim3(kRayBins / 64), dim3(64 * kScanWaves), 0, stream, ws.hist, blocks, nullptr,
+                       ws.totals);
+    hipLaunchKernelGGL(bin_cells_kernel, dim3(1), dim3(kBinBlock), 0, stream, ws.totals, nullptr);
+    hipLaunchKernelGGL(bin_scatter_kernel, dim3((uint32_t)((n + kBinBlock - 1) / kBinBlock)), dim3(kBinBlock), 0,
+                       stream, ws.keyrank, ws.hist, ws.totals, n, (uint64_t)kBinRange, blocks, ws.order);
+    *order = ws.order;
+    *spare = ws.keyrank;  // read by the scatter only
+    *count = ws.count;
+    return hipGetLastError();
+}
 
 uint32_t ray_stack_entries(uint32_t depth) { return depth > 1 ? depth - 1 : 1; }
 
