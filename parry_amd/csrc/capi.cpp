@@ -125,7 +125,30 @@ int upload(void **dptr, const void *src, size_t bytes) {
     return PQ_OK;
 }
 
-// The bound on projections that MeshBounds states.  A projection is a vertex (in
+// Every child box inside its parent's, every triangle inside its leaf's box.
+bool boxes_nested(const pq_bvh_node_wide *nodes, uint32_t num_nodes, const float *vertices, const uint32_t *indices) {
+    auto inside = [](const float *mn, const float *mx, const pq_bvh_node &box) {
+        for (int a = 0; a < 3; ++a)
+            if (!(mn[a] >= box.mins[a] && mx[a] <= box.maxs[a])) return false;
+        return true;
+    };
+    for (uint32_t k = 0; k < num_nodes; ++k)
+        for (const pq_bvh_node *c : {&nodes[k].left, &nodes[k].right}) {
+            const uint32_t leaves = leaf_count(*c);
+            if (leaves == 1) {
+                for (int q = 0; q < 3; ++q) {
+                    const float *p = vertices + 3 * (size_t)indices[3 * (size_t)c->children + q];
+                    if (!inside(p, p, *c)) return false;
+                }
+            } else if (leaves > 1) {
+                const pq_bvh_node_wide &w = nodes[c->children];
+                if (!inside(w.left.mins, w.left.maxs, *c) || !inside(w.right.mins, w.right.maxs, *c)) return false;
+            }
+        }
+    return true;
+}
+
+// The bound on projections that MeshBounds states, for finite vertices.  A projection is a vertex (in
 // the box), a point of an edge, or a + ab * v + ac * w.  With unit roundoff u, the
 // triangle's longest edge e, its normal n and D = |p|_1 + 3 * extent (at least the
 // distance from p to any vertex), rounding leaves v and w each within
@@ -133,14 +156,10 @@ int upload(void **dptr, const void *src, size_t bytes) {
 // within 8 u D / |edge|; either moves the point by at most 90 u D e^4 / |n|^2, if the
 // relative error of va + vb + vc, 30 u D e^3 / |n|^2, is below a quarter.  `foot` has
 // 128 in place of 90.
-MeshBounds mesh_bounds(const pq_bvh_node_wide *nodes, uint32_t num_nodes, const float *vertices,
-                       uint32_t num_vertices, const uint32_t *indices, uint32_t num_triangles) {
-    const MeshBounds none{0.0f, 0.0f, -1.0f};
+constexpr MeshBounds kNoBounds{0.0f, 0.0f, -1.0f};
+MeshBounds mesh_bounds(const float *vertices, uint32_t num_vertices, const uint32_t *indices, uint32_t num_triangles) {
     float extent = 0.0f;
-    for (size_t k = 0; k < 3 * (size_t)num_vertices; ++k) {
-        if (!std::isfinite(vertices[k])) return none;
-        extent = std::fmax(extent, std::fabs(vertices[k]));
-    }
+    for (size_t k = 0; k < 3 * (size_t)num_vertices; ++k) extent = std::fmax(extent, std::fabs(vertices[k]));
     double worst = 0.0, reach = 3.0e38;
     const double u = 1.1920929e-7 / 2;
     for (uint32_t t = 0; t < num_triangles; ++t) {
@@ -160,29 +179,10 @@ MeshBounds mesh_bounds(const pq_bvh_node_wide *nodes, uint32_t num_nodes, const 
             n2 += n[a] * n[a];
         }
         const double q = n2 / (e2 * e2);
-        if (!(q >= 1.0e-3)) return none;  // slivers: the bound would be too wide to use
+        if (!(q >= 1.0e-3)) return kNoBounds;  // slivers: the bound would be too wide to use
         worst = std::fmax(worst, 128.0 * u / q);
         reach = std::fmin(reach, 0.25 * std::sqrt(e2) * q / (30.0 * u));
     }
-    // Every child box inside its parent's, every triangle inside its leaf's box.
-    auto inside = [](const float *mn, const float *mx, const pq_bvh_node &box) {
-        for (int a = 0; a < 3; ++a)
-            if (!(mn[a] >= box.mins[a] && mx[a] <= box.maxs[a])) return false;
-        return true;
-    };
-    for (uint32_t k = 0; k < num_nodes; ++k)
-        for (const pq_bvh_node *c : {&nodes[k].left, &nodes[k].right}) {
-            const uint32_t leaves = leaf_count(*c);
-            if (leaves == 1) {
-                for (int q = 0; q < 3; ++q) {
-                    const float *p = vertices + 3 * (size_t)indices[3 * (size_t)c->children + q];
-                    if (!inside(p, p, *c)) return none;
-                }
-            } else if (leaves > 1) {
-                const pq_bvh_node_wide &w = nodes[c->children];
-                if (!inside(w.left.mins, w.left.maxs, *c) || !inside(w.right.mins, w.right.maxs, *c)) return none;
-            }
-        }
     return MeshBounds{extent, (float)worst, (float)reach};
 }
 
@@ -330,10 +330,11 @@ int pq_trimesh_create(const float *vertices, uint32_t num_vertices, const uint32
     for (const pq_bvh_node_wide &w : dev_nodes)
         for (const pq_bvh_node *c : {&w.left, &w.right})
             for (int d = 0; d < 3; ++d) finite = finite && std::isfinite(c->mins[d]) && std::isfinite(c->maxs[d]);
+    const bool nested =
+        finite && boxes_nested(m->host_nodes.data(), (uint32_t)m->host_nodes.size(), vertices, indices);
     m->dev.finite = finite ? 1u : 0u;
     m->dev.tuning = pq_ray_tuning{PQ_RAY_MAPPING_STATIC, 128, 0, 256, 0, 0};
-    m->dev.bounds = mesh_bounds(m->host_nodes.data(), (uint32_t)m->host_nodes.size(), vertices, num_vertices, indices,
-                                num_triangles);
+    m->dev.bounds = nested ? mesh_bounds(vertices, num_vertices, indices, num_triangles) : kNoBounds;
     *out = m;
     return PQ_OK;
 }

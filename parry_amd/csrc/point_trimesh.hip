@@ -154,6 +154,10 @@ __device__ __forceinline__ void walk(const float4 *node4, const float4 *tri4, f3
     }
 }
 
+__device__ __forceinline__ bool in_box(f3 a, f3 b, f3 c, f3 p) {
+    const f3 mn = min3(min3(a, b), c), mx = max3(max3(a, b), c);
+    return (p.x >= mn.x) & (p.y >= mn.y) & (p.z >= mn.z) & (p.x <= mx.x) & (p.y <= mx.y) & (p.z <= mx.z);
+}
 // Whether the projection on a triangle lies in the triangle's box.  Costs are then
 // monotone down the tree: box cost and leaf cost are sums of squares of the same
 // form, and float subtraction, product, sum and root are monotone, so the leaf
@@ -161,9 +165,7 @@ __device__ __forceinline__ void walk(const float4 *node4, const float4 *tri4, f3
 // are nested, MeshBounds).
 __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, f3 p) {
     const float4 q0 = tri4[3 * (size_t)leaf], q1 = tri4[3 * (size_t)leaf + 1], q2 = tri4[3 * (size_t)leaf + 2];
-    const f3 a{q0.x, q0.y, q0.z}, b{q0.w, q1.x, q1.y}, c{q1.z, q1.w, q2.x};
-    const f3 mn = min3(min3(a, b), c), mx = max3(max3(a, b), c);
-    return p.x >= mn.x && p.y >= mn.y && p.z >= mn.z && p.x <= mx.x && p.y <= mx.y && p.z <= mx.z;
+    return in_box(f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, p);
 }
 
 // find_best by one lane, with the leaves put aside: a lane reaches a leaf at one
@@ -174,15 +176,17 @@ __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, 
 // answer is not known to be find_best's.
 //
 // The nodes are taken in find_best's order with a best cost that is late, so this
-// walk sees find_best's leaves and a few more, in its order.  If the projection of
-// the first leaf W of smallest cost lies in W's box, find_best takes W too: each
-// leaf before it costs more than W, so no box above W costs as much as the best
-// cost find_best has there, and nothing after W costs less.
+// walk sees find_best's leaves and a few more, in its order, as long as the
+// projection of every leaf it takes as the best lies in that leaf's box (a leaf
+// find_best prunes does not then cost less than its best).  So does find_best take
+// the first leaf W of smallest cost: each leaf before it costs more than W, so no box
+// above W costs as much as the best cost find_best has there, and nothing after W
+// costs less.
 __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 *tri4, f3 pt, bool solid, uint32_t *stk,
                                               uint32_t stride, uint32_t limit, PtBest &b) {
     uint32_t curr = 0, sp = 0, n = 0, steps = 0;
     uint32_t l0 = 0, l1 = 0, l2 = 0, l3 = 0;
-    bool walking = true;
+    bool walking = true, known = true;
     auto put = [&](bool add, uint32_t leaf) {
         l0 = add && n == 0u ? leaf : l0;
         l1 = add && n == 1u ? leaf : l1;
@@ -219,7 +223,15 @@ __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 
         }
         if (leaves) {
             if (n != 0u) {
-                visit_leaf(tri4, l0, pt, solid, b);
+                const float4 q0 = tri4[3 * (size_t)l0], q1 = tri4[3 * (size_t)l0 + 1], q2 = tri4[3 * (size_t)l0 + 2];
+                const f3 ta{q0.x, q0.y, q0.z}, tb{q0.w, q1.x, q1.y}, tc{q1.z, q1.w, q2.x};
+                const f3 p = tri_point(ta, tb, tc, pt, solid);
+                const float cost = sqrtf(norm_sq3(sub3(pt, p)));
+                const bool closer = cost < b.cost;
+                known = known & (!closer | in_box(ta, tb, tc, p));
+                b.cost = closer ? cost : b.cost;
+                b.leaf = closer ? l0 : b.leaf;
+                b.have = b.have | closer;
                 l0 = l1;
                 l1 = l2;
                 l2 = l3;
@@ -228,7 +240,7 @@ __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 
             if (!walking && n == 0u) break;
         }
     }
-    return !b.have || point_in_box(tri4, b.leaf, b.p);
+    return known;
 }
 
 // is_inside comes from the winner's triangle, projected again.
