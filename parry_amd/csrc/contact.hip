@@ -685,6 +685,25 @@ template <int V, int F, int S, int K, class I, int SV> struct LazyState {
 constexpr uint32_t kDeadBit = 1u << 27;
 
 
+// With a wave per pair every value of the pair is the same in all lanes: saying so
+// makes the branches on shape types and counts scalar (support points 3,700 ->
+// 2,600 cycles, the next face 3,900 -> 3,100; the walk got slower, 3,600 -> 4,900, and
+// keeps its vector form).
+template <int G> __device__ __forceinline__ uint32_t uni(uint32_t v) {
+    if constexpr (G == 64) return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    return v;
+}
+template <int G> __device__ __forceinline__ float uni(float v) {
+    if constexpr (G == 64) return __uint_as_float(uni<G>(__float_as_uint(v)));
+    return v;
+}
+template <int G> __device__ __forceinline__ f3 uni(f3 v) { return f3{uni<G>(v.x), uni<G>(v.y), uni<G>(v.z)}; }
+template <int G> __device__ __forceinline__ ShapeRef uni(ShapeRef g) {
+    g.type = uni<G>(g.type);
+    g.n = uni<G>(g.n);
+    return g;
+}
+
 struct LazyRegs {
     uint32_t nv, nf, best_id, niter;
     float max_dist, old_dist;
@@ -1066,6 +1085,10 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     constexpr uint32_t kIdMask = (1u << W::kShift) - 1u;
     const float eps_tol = kEps * 100.0f;
     const uint32_t sub = __lane_id() % G;
+    r.nv = uni<G>(r.nv);
+    r.nf = uni<G>(r.nf);
+    r.niter = uni<G>(r.niter);
+    const ShapeRef ga = uni<G>(pr.a), gb = uni<G>(pr.b);
     // The live face of largest key.
     uint32_t fid;
     float fkey;
@@ -1091,7 +1114,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
                 kb = fmaxf(kk, kb);
             }
         }
-        fkey = group_max<G>(kb);
+        fkey = uni<G>(group_max<G>(kb));
         if (fkey == -INFINITY) return EPA_OK;  // parry's heap is empty
         const uint64_t top = group_ballot<G>(kb == fkey);
         const uint64_t twice = group_ballot<G>(kb == fkey && dup);
@@ -1100,11 +1123,12 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
             fid = lazy_replay(w, r);
             if (fid == kNoFace) return EPA_RESTART;
         }
+        fid = uni<G>(fid);
     }
     const typename W::Face face = w->face[fid];
     const uint32_t fx = face.px;
     const f3 fn = face_normal(w, fid);
-    const Cso c = group_cso<G, (W::kSV > 0)>(pr.pos, pr.a, pr.b, st, fn);
+    const Cso c = group_cso<G, (W::kSV > 0)>(pr.pos, ga, gb, st, fn);
     const float cand = dot3(c.p, fn);
     uint32_t best_t = r.niter == 0 ? fid : r.best_id;  // the heap's first top is parry's first best face
     float max_t = r.max_dist;
@@ -1981,7 +2005,7 @@ hipEvent_t g_contact_phase_events[kContactPhases + 1] = {};
 namespace {
 struct ContactWorkspace {
     uint32_t *counters;  // list lengths and the tiers' next entries (reset_counters_kernel)
-    uint32_t *totals, *taken;  // per class of pairs, after the counters
+    uint32_t *bins;  // of the pair order, after the counters
     uint32_t *order;
     uint16_t *cls;
     EpaItem *queue;
@@ -2022,9 +2046,8 @@ ContactWorkspace carve_workspace(void *base, uint64_t m) {
         off += up(bytes);
         return p;
     };
-    w.counters = (uint32_t *)take((kNumCounters + 2 * kPairClasses) * sizeof(uint32_t));
-    w.totals = w.counters + kNumCounters;
-    w.taken = w.totals + kPairClasses;
+    w.counters = (uint32_t *)take((kNumCounters + kPairOrderBins) * sizeof(uint32_t));
+    w.bins = w.counters + kNumCounters;
     const uint64_t ordered = m >= kOrderMinPairs ? m : 0;  // whatever the types: the size depends on m alone
     w.order = (uint32_t *)take(ordered * sizeof(uint32_t));
     w.cls = (uint16_t *)take(ordered * sizeof(uint16_t));
@@ -2046,11 +2069,29 @@ ContactWorkspace carve_workspace(void *base, uint64_t m) {
     return w;
 }
 
+// order_count_kernel and order_scatter_kernel; `bins` zeroed.
+static_assert(kPairOrderBins == 2 * kPairClasses, "totals and positions per class");
+hipError_t order_pairs(const DeviceShapes &s, const uint32_t *pairs, uint64_t m, const uint64_t *m_dev, uint16_t *cls,
+                       uint32_t *bins, uint32_t *order, hipStream_t stream) {
+    const dim3 grid((uint32_t)((m + kOrderRange - 1) / kOrderRange));
+    hipLaunchKernelGGL(order_count_kernel, grid, dim3(kOrderBlock), 0, stream, s.rec, pairs, m,
+                       (const unsigned long long *)m_dev, cls, bins);
+    hipLaunchKernelGGL(order_scatter_kernel, grid, dim3(kOrderBlock), 0, stream, m, (const unsigned long long *)m_dev,
+                       cls, bins, bins + kPairClasses, order);
+    return hipGetLastError();
+}
+
 template <int G>
 hipError_t launch_small(const TierArgs &t, const RecSink<SmallRec> &sink, uint64_t m, hipStream_t stream) {
     return launch_lazy<G, LazySmall, SmallRec, SmallRec, 3>(t, nullptr, sink, m, kSmallGroups, stream);
 }
 }  // namespace
+
+hipError_t launch_pair_order(const DeviceShapes &s, const uint32_t *pairs, uint64_t m, const uint64_t *m_dev,
+                             uint16_t *cls, uint32_t *bins, uint32_t *order, hipStream_t stream) {
+    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(256), 0, stream, bins, kPairOrderBins);
+    return order_pairs(s, pairs, m, m_dev, cls, bins, order, stream);
+}
 
 size_t contact_workspace_bytes(uint64_t num_pairs) { return carve_workspace(nullptr, num_pairs).bytes; }
 
@@ -2062,18 +2103,12 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
     DevContact *o = (DevContact *)out;
     const bool timed = g_contact_phase_timing;
     auto mark = [&](int k) { return timed ? hipEventRecord(g_contact_phase_events[k], stream) : hipSuccess; };
-    const bool ordered = takes_order(s, m);
+    const bool ordered = !(flags & kContactInOrder) && takes_order(s, m);
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(256), 0, stream, w.counters,
-                       kNumCounters + (ordered ? 2 * kPairClasses : 0u));
+                       kNumCounters + (ordered ? kPairOrderBins : 0u));
     hipError_t e = mark(0);
     if (e != hipSuccess) return e;
-    if (ordered) {
-        const dim3 grid((uint32_t)((m + kOrderRange - 1) / kOrderRange));
-        hipLaunchKernelGGL(order_count_kernel, grid, dim3(kOrderBlock), 0, stream, s.rec, pairs, m,
-                           (const unsigned long long *)m_dev, w.cls, w.totals);
-        hipLaunchKernelGGL(order_scatter_kernel, grid, dim3(kOrderBlock), 0, stream, m,
-                           (const unsigned long long *)m_dev, w.cls, w.totals, w.taken, w.order);
-    }
+    if (ordered && (e = order_pairs(s, pairs, m, m_dev, w.cls, w.bins, w.order, stream)) != hipSuccess) return e;
     hipLaunchKernelGGL(contact_gjk_kernel, dim3((uint32_t)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
                        s.rec, s.verts, poses, pairs, m, (const unsigned long long *)m_dev, prediction, seeds, o, iters,
                        w.queue, w.counters, flags, ordered ? w.order : nullptr);

@@ -253,6 +253,13 @@ constexpr uint32_t kContactLocalSupportMaps = 1u;
 // separating direction in normal1 of a pair without contact; a pair without
 // feature maps gets PQ_CONTACT_UNSUPPORTED.
 constexpr uint32_t kContactFeatureMaps = 2u;
+// kContactInOrder: the pairs come class by class already (launch_pair_order).
+constexpr uint32_t kContactInOrder = 4u;
+// The pairs' indices class by class (contact.hip) into `order`, on the stream.
+// Scratch: `cls` one entry per pair, `bins` kPairOrderBins words.
+constexpr uint32_t kPairOrderBins = 1024;
+hipError_t launch_pair_order(const DeviceShapes &s, const uint32_t *pairs, uint64_t m, const uint64_t *m_dev,
+                             uint16_t *cls, uint32_t *bins, uint32_t *order, hipStream_t stream);
 hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint32_t *pairs, uint64_t m,
                            const uint64_t *m_dev, float prediction, const float *seeds, pq_contact *out,
                            uint32_t *iters, void *workspace, hipStream_t stream, uint32_t flags = 0u);
