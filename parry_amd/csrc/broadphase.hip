@@ -98,15 +98,20 @@ __device__ __forceinline__ bool overlaps(const float q[6], float4 mn, float4 mx)
     return (q[0] <= mx.x) & (q[1] <= mx.y) & (q[2] <= mx.z) & (q[3] >= mn.x) & (q[4] >= mn.y) & (q[5] >= mn.z);
 }
 
+// One lane per leaf, the lanes in depth-first leaf order: the lanes of a wave query
+// neighbouring boxes and walk the same nodes.  In leaf-id order (any order in space)
+// a pass over the 262,144-shape scene took 187 us.
 template <bool WRITE>
 __global__ __launch_bounds__(kBlock) void self_pairs_kernel(const pq_bvh_node_wide *__restrict__ nodes,
-                                                            const uint32_t *__restrict__ leaf_slot, uint32_t n,
+                                                            const uint32_t *__restrict__ leaf_slot,
+                                                            const uint32_t *__restrict__ leaf_order, uint32_t n,
                                                             uint32_t *__restrict__ counts,
                                                             const unsigned long long *__restrict__ offsets,
                                                             uint32_t *__restrict__ pairs, uint64_t capacity) {
     extern __shared__ uint32_t lds_stack[];
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= n) return;
+    const uint32_t i = leaf_order[t];
     uint32_t *stk = lds_stack + threadIdx.x;
     const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
     const uint32_t slot = leaf_slot[i];
@@ -213,16 +218,16 @@ hipError_t launch_bvh_self_pairs(const DeviceBvh &b, uint32_t *pairs, uint64_t c
     const uint32_t cap = b.depth > 1 ? b.depth - 1 : 1;
     const size_t lds = (size_t)cap * kBlock * sizeof(uint32_t);
     const dim3 grid((n + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(self_pairs_kernel<false>, grid, dim3(kBlock), lds, stream, b.nodes, b.leaf_slot, n,
-                       b.pair_counts, b.pair_offsets, pairs, capacity);
+    hipLaunchKernelGGL(self_pairs_kernel<false>, grid, dim3(kBlock), lds, stream, b.nodes, b.leaf_slot,
+                       b.leaf_order, n, b.pair_counts, b.pair_offsets, pairs, capacity);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     size_t bytes = b.scan_temp_bytes;
     e = rocprim::exclusive_scan(b.scan_temp, bytes, b.pair_counts, b.pair_offsets, 0ull, (size_t)n + 1,
                                 rocprim::plus<unsigned long long>(), stream);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(self_pairs_kernel<true>, grid, dim3(kBlock), lds, stream, b.nodes, b.leaf_slot, n,
-                       b.pair_counts, b.pair_offsets, pairs, capacity);
+    hipLaunchKernelGGL(self_pairs_kernel<true>, grid, dim3(kBlock), lds, stream, b.nodes, b.leaf_slot,
+                       b.leaf_order, n, b.pair_counts, b.pair_offsets, pairs, capacity);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(copy_total_kernel, dim3(1), dim3(64), 0, stream, b.pair_offsets, n, count);
     return hipGetLastError();

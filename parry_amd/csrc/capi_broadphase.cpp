@@ -163,14 +163,17 @@ int bvh_handle_from_nodes(const std::vector<pq_bvh_node_wide> &nodes, uint32_t n
         return fail(PQ_ERR_UNSUPPORTED, "Bvh depth " + std::to_string(depth) + " exceeds " +
                                             std::to_string(kMaxBroadphaseDepth));
     const uint32_t nn = (uint32_t)nodes.size();
-    std::vector<uint32_t> leaf_slot(n, 0), parent_slot(nn ? nn : 1, UINT32_MAX);
+    std::vector<uint32_t> leaf_slot(n, 0), leaf_order, parent_slot(nn ? nn : 1, UINT32_MAX);
+    leaf_order.reserve(n);
     for (uint32_t w = 0; w < nn; ++w) {
         const pq_bvh_node *side[2] = {&nodes[w].left, &nodes[w].right};
         for (uint32_t s = 0; s < 2; ++s) {
             const pq_bvh_node &c = *side[s];
             const uint32_t lc = leaf_count(c);
-            if (lc == 1) leaf_slot[c.children] = 2 * w + s;
-            else if (lc > 1) parent_slot[c.children] = 2 * w + s;
+            if (lc == 1) {
+                leaf_slot[c.children] = 2 * w + s;
+                leaf_order.push_back(c.children);
+            } else if (lc > 1) parent_slot[c.children] = 2 * w + s;
         }
     }
     // Heights above the leaves: depth-first order puts children after parents, so
@@ -209,6 +212,7 @@ int bvh_handle_from_nodes(const std::vector<pq_bvh_node_wide> &nodes, uint32_t n
     if (e != hipSuccess) rc = hip_fail(e, "rocprim::exclusive_scan (size query)");
     if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.nodes, nn * sizeof(pq_bvh_node_wide));
     if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.leaf_slot, n * sizeof(uint32_t));
+    if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.leaf_order, n * sizeof(uint32_t));
     if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.parent_slot, parent_slot.size() * sizeof(uint32_t));
     if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.pair_counts, ((size_t)n + 1) * sizeof(uint32_t));
     if (rc == PQ_OK) rc = dev_alloc(b, (void **)&d.pair_offsets, ((size_t)n + 1) * sizeof(unsigned long long));
@@ -221,6 +225,8 @@ int bvh_handle_from_nodes(const std::vector<pq_bvh_node_wide> &nodes, uint32_t n
         if (nn) e = hipMemcpy(d.nodes, nodes.data(), nn * sizeof(pq_bvh_node_wide), hipMemcpyHostToDevice);
         if (e == hipSuccess && n)
             e = hipMemcpy(d.leaf_slot, leaf_slot.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice);
+        if (e == hipSuccess && n)  // one entry per leaf: callers check that each leaf is in the tree once
+            e = hipMemcpy(d.leaf_order, leaf_order.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(d.parent_slot, parent_slot.data(), parent_slot.size() * sizeof(uint32_t),
                           hipMemcpyHostToDevice);

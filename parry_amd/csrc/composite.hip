@@ -57,6 +57,8 @@ __global__ __launch_bounds__(kBlock) void combined_poses_kernel(const float *__r
     for (int k = 0; k < 7; ++k) out[7 * i + k] = src[k];
 }
 
+constexpr uint64_t kKeepMax = 256;  // triangles per shape the counting pass keeps at most
+
 // BvhNode::intersects with a box (closed intervals, bvh_tree.rs:954-957).
 __device__ __forceinline__ bool node_meets(float4 mn, float4 mx, f3 lo, f3 hi) {
     return (mn.x <= hi.x) & (mn.y <= hi.y) & (mn.z <= hi.z) & (mx.x >= lo.x) & (mx.y >= lo.y) & (mx.z >= lo.z);
@@ -64,16 +66,30 @@ __device__ __forceinline__ bool node_meets(float4 mn, float4 mx, f3 lo, f3 hi) {
 
 // Step 1.  A node is named by (wide index << 1) | side; `stk` is this lane's
 // LDS stack (stride kBlock), at most `depth` entries (one pending right sibling
-// per level of the walk).
+// per level of the walk).  The counting pass keeps each shape's first `keep`
+// triangles (kept[k * n + q], in the memory the candidates' contacts go to later), so
+// that the writing pass walks again only for shapes with more; a second walk for all
+// took as long as the first (200 us for 32,768 shapes on 81,920 triangles).
 template <bool WRITE>
 __global__ __launch_bounds__(kBlock) void mesh_candidates_kernel(
     const pq_bvh_node_wide *__restrict__ nodes, const ShapeRecord *__restrict__ rec, const float4 *__restrict__ verts,
     const float *__restrict__ mesh_pose, const float *__restrict__ poses, uint32_t ntri, uint32_t n, float prediction,
     uint32_t *__restrict__ counts, const unsigned long long *__restrict__ offsets, uint32_t *__restrict__ pairs,
-    uint64_t capacity) {
+    uint64_t capacity, uint32_t *__restrict__ kept, uint32_t keep) {
     extern __shared__ uint32_t lds_stack[];
     const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
     if (q >= n) return;
+    if (WRITE) {
+        const uint64_t first = offsets[q];
+        const uint32_t have = (uint32_t)(offsets[q + 1] - first);
+        if (have <= keep) {
+            for (uint32_t k = 0; k < have && first + k < capacity; ++k) {
+                pairs[2 * (first + k)] = kept[(size_t)k * n + q];
+                pairs[2 * (first + k) + 1] = ntri + q;
+            }
+            return;
+        }
+    }
     uint32_t *stk = lds_stack + threadIdx.x;
     const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
     const iso pos12 = iso_inv_mul(load_iso(mesh_pose), load_iso(poses + 7 * (size_t)q));
@@ -115,6 +131,7 @@ __global__ __launch_bounds__(kBlock) void mesh_candidates_kernel(
                 }
                 ++out;
             } else {
+                if (found < keep) kept[(size_t)found * n + q] = children;
                 ++found;
             }
         } else {
@@ -235,8 +252,11 @@ hipError_t launch_mesh_contacts(const DeviceMesh &m, const DeviceShapes &combine
     const size_t lds = ((size_t)m.depth + 1) * kBlock * sizeof(uint32_t);
     hipLaunchKernelGGL(combined_poses_kernel, dim3((uint32_t)(((uint64_t)ntri + n + kBlock - 1) / kBlock)), block, 0,
                        stream, mesh_pose, poses, ntri, n, w.poses);
+    const uint64_t room = capacity * (sizeof(pq_contact) / sizeof(uint32_t)) / n;  // triangles per shape in w.cand
+    const uint32_t keep = (uint32_t)(room < kKeepMax ? room : kKeepMax);
+    uint32_t *const kept = (uint32_t *)w.cand;
     hipLaunchKernelGGL(mesh_candidates_kernel<false>, grid, block, lds, stream, m.nodes, combined.rec, combined.verts,
-                       mesh_pose, poses, ntri, n, prediction, w.counts, nullptr, nullptr, 0ull);
+                       mesh_pose, poses, ntri, n, prediction, w.counts, nullptr, nullptr, 0ull, kept, keep);
     hipLaunchKernelGGL(set_last_zero_kernel, dim3(1), dim3(64), 0, stream, w.counts, n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -245,7 +265,7 @@ hipError_t launch_mesh_contacts(const DeviceMesh &m, const DeviceShapes &combine
                                 rocprim::plus<unsigned long long>(), stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(mesh_candidates_kernel<true>, grid, block, lds, stream, m.nodes, combined.rec, combined.verts,
-                       mesh_pose, poses, ntri, n, prediction, nullptr, w.offsets, w.pairs, capacity);
+                       mesh_pose, poses, ntri, n, prediction, nullptr, w.offsets, w.pairs, capacity, kept, keep);
     hipLaunchKernelGGL(copy_count_kernel, dim3(1), dim3(64), 0, stream, w.offsets, n, w.total);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (capacity) {

@@ -203,6 +203,7 @@ hipError_t launch_shape_aabbs(const DeviceShapes &s, const float *poses, float *
 struct DeviceBvh {
     pq_bvh_node_wide *nodes;  // device, depth-first
     uint32_t *leaf_slot;      // device, per leaf: wide * 2 + (1 if right)
+    uint32_t *leaf_order;     // device: the leaves in depth-first order
     uint32_t *parent_slot;    // device, per wide node: parent wide * 2 + side (root: UINT32_MAX)
     uint32_t *pair_counts;    // device, n + 1
     unsigned long long *pair_offsets;  // device, n + 1
