@@ -80,8 +80,7 @@ def _check_pairs(fn: str, pairs, num_shapes: int, check_indices: bool) -> None:
             or pairs.shape[1] != 2:
         raise ValueError(f"{fn}: pairs must be an (m, 2) int32/uint32 tensor, got {tuple(pairs.shape)} {pairs.dtype}")
     if check_indices and pairs.numel():
-        v = pairs.view(torch.int32)
-        lo, hi = int(v.min()), int(v.max())
+        lo, hi = torch.stack(torch.aminmax(pairs.view(torch.int32))).tolist()
         if lo < 0 or hi >= num_shapes:
             raise ValueError(f"{fn}: pair indices must lie in [0, {num_shapes}), got [{lo}, {hi}]")
 
