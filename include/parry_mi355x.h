@@ -423,7 +423,7 @@ int pq_contact_set_tuning(const pq_contact_tuning *tuning);
  * While enabled (process-wide), every contact call records HIP events on its
  * own stream between its phases; pq_contact_phase_ms waits for the last call's
  * events and writes ms[0..4]: the GJK/dispatch kernel, the first two EPA tiers, the
- * 768-face tier, the 2048-face tier and the global-memory tier.  Calls that
+ * 760-face tier, the 2048-face tier and the global-memory tier.  Calls that
  * overlap on several streams share the events; leave it off under graph capture. */
 int pq_contact_set_phase_timing(int enable);
 int pq_contact_phase_ms(float *ms, uint32_t n);

@@ -17,13 +17,13 @@
 //     popcount give each lane its slot).
 // Stage 2 (a group of lanes per queued pair): EPA (src/query/epa/epa3.rs:428-651)
 //   with the polytope in LDS, in three tiers: eight lanes per pair and 64 faces,
-//   sixteen lanes and 192 faces, a wave and 768 faces.  A pair that outgrows a
+//   sixteen lanes and 132 faces, a wave and 760 faces.  A pair that outgrows a
 //   tier's buffers goes on in the next one where it stopped.  The group's lanes
 //   share the support scans, pick the next face, test every face's visibility
 //   and build the new faces in parallel; the silhouette walk is serial.
 // Stage 3 (one wave per pair): the same with parry's heap of faces (the binary
 //   heap algorithm of Rust's BinaryHeap), 2048 faces in LDS, then 8192 in global
-//   memory, for the few pairs beyond 768 faces or with non-finite face distances.
+//   memory, for the few pairs beyond 760 faces or with non-finite face distances.
 // Every contact is finished as contact_support_map_support_map (dist, point2,
 // normal2 in shape 2's frame) and Contact::transform_by_mut (contact.rs:171-176).
 #include <cstring>
@@ -667,7 +667,9 @@ __device__ __forceinline__ f3 ccw_normal(f3 pa, f3 pb, f3 pc) {
 // the faces not deleted, in any order: a new face takes the list place of a face
 // the iteration deleted.  Of a polytope's faces half are deleted after eight
 // iterations and four fifths after sixty.  Scanning them all, 2^20 mixed pairs took
-// 3.31 ms (now 3.14) and 300 pairs 405 us (now 368).
+// 3.31 ms (3.14 with the list) and 300 pairs 405 us (368).  Normals are kept by list
+// place too, not by face, which a deleted face does not need: three waves per CU more
+// in the third tier, 2^20 mixed pairs 3.14 -> 3.07 ms.
 template <int V, int F, int S, int K, class I, int SV, int L> struct LazyState {
     static constexpr int kV = V, kF = F, kS = S, kK = K, kSV = SV, kL = L;
     static constexpr bool kMask = F <= 64;  // deleted flags in a 64-bit register mask
@@ -678,7 +680,9 @@ template <int V, int F, int S, int K, class I, int SV, int L> struct LazyState {
         uint32_t px;  // vertices; bits 24-26: can_be_seen_by the newest vertex per opposite vertex; 27: deleted
         I adj[4];     // the three neighbours, and the face's place in live[]
     };
-    alignas(16) float nk[F][4];  // normal, then FaceId's neg_dist (-inf for a face that was not pushed)
+    alignas(16) float nk[L][4];  // by place in live[]: normal, then FaceId's neg_dist (-inf for a face that was
+                                 // not pushed, or a place whose face was deleted)
+    float key[F];                // neg_dist of every face, for the rebuilt heap
     float vp[V][4];
     Face face[F];
     float sv[SV > 0 ? 2 : 1][SV > 0 ? SV : 1][3];  // both ConvexPolyhedra's vertices (local frames), if SV > 0
@@ -731,9 +735,9 @@ template <class F> __device__ __forceinline__ auto face_adj(const F &f) {
     else
         return (uint64_t)f.adj[0] | ((uint64_t)f.adj[1] << 16) | ((uint64_t)f.adj[2] << 32);
 }
-template <class W> __device__ __forceinline__ float &face_key(W *w, uint32_t f) { return w->nk[f][3]; }
-template <class W> __device__ __forceinline__ f3 face_normal(const W *w, uint32_t f) {
-    return f3{w->nk[f][0], w->nk[f][1], w->nk[f][2]};
+template <class W> __device__ __forceinline__ float face_key(const W *w, uint32_t f) { return w->key[f]; }
+template <class W> __device__ __forceinline__ f3 place_normal(const W *w, uint32_t place) {
+    return f3{w->nk[place][0], w->nk[place][1], w->nk[place][2]};
 }
 template <class W, class A> __device__ __forceinline__ uint32_t adj_at(A a, uint32_t k) {
     return (uint32_t)(a >> (W::kShift * k)) & ((1u << W::kShift) - 1u);
@@ -807,15 +811,17 @@ __device__ __forceinline__ bool lazy_face(W *w, uint32_t f, uint32_t a, uint32_t
     n = ccw_normal(pa, pb, pc);
     return face_inside(pa, pb, pc);
 }
-template <class W> __device__ __forceinline__ void set_normal(W *w, uint32_t f, f3 n, float key) {
-    *reinterpret_cast<float4 *>(w->nk[f]) = make_float4(n.x, n.y, n.z, key);
+template <class W> __device__ __forceinline__ void set_normal(W *w, uint32_t f, uint32_t place, f3 n, float key) {
+    *reinterpret_cast<float4 *>(w->nk[place]) = make_float4(n.x, n.y, n.z, key);
+    w->key[f] = key;
 }
 
 // Face::closest_points (epa3.rs:120-130).
 template <class W> __device__ void lazy_points(const W *w, const float *orig, uint32_t f, f3 &p1, f3 &p2, f3 &n) {
     const uint32_t x = w->face[f].px;
+    const f3 a = vpt(w, pt_at(x, 0)), b = vpt(w, pt_at(x, 1)), c = vpt(w, pt_at(x, 2));
     float bc[3];
-    face_bcoords(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)), bc);
+    face_bcoords(a, b, c, bc);
     f3 o1[3], o2[3];
     for (int q = 0; q < 3; ++q) {
         const float *o = orig + kOrigFloats * pt_at(x, q);
@@ -824,7 +830,7 @@ template <class W> __device__ void lazy_points(const W *w, const float *orig, ui
     }
     p1 = add3(add3(mul3(o1[0], bc[0]), mul3(o1[1], bc[1])), mul3(o1[2], bc[2]));
     p2 = add3(add3(mul3(o2[0], bc[0]), mul3(o2[1], bc[1])), mul3(o2[2], bc[2]));
-    n = face_normal(w, f);
+    n = ccw_normal(a, b, c);  // as lazy_face computed it
 }
 
 // BinaryHeap<FaceId> over face ids (max-heap on key[]; equal keys compare Equal),
@@ -945,7 +951,7 @@ __device__ uint32_t lazy_export(const W *w, const float *orig, const RecSink<R> 
         const typename W::Face f = w->face[k];
         o->px[k] = (f.px & 0x00ffffffu) | (face_dead(w, r, k, f.px) ? kDeadBit : 0u);
         o->adj[k] = face_adj(f);
-        o->key[k] = w->nk[k][3];
+        o->key[k] = w->key[k];
     }
     for (uint32_t k = sub; k < r.niter; k += G) {
         o->pops[k] = (uint8_t)w->pops[k];
@@ -982,8 +988,13 @@ template <int G, class W, class R> __device__ void lazy_import(W *w, float *orig
         if (k < r.nf) {
             const uint32_t a = o->adj[k];
             w->face[k] = typename W::Face{x, {(I)(a & 0xffu), (I)((a >> 8) & 0xffu), (I)((a >> 16) & 0xffu), (I)place}};
-            if ((x & kDeadBit) == 0u) w->live[place] = (I)k;
-            set_normal(w, k, ccw_normal(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2))), o->key[k]);
+            if ((x & kDeadBit) == 0u) {
+                w->live[place] = (I)k;
+                const f3 n = ccw_normal(vpt(w, pt_at(x, 0)), vpt(w, pt_at(x, 1)), vpt(w, pt_at(x, 2)));
+                set_normal(w, k, place, n, o->key[k]);
+            } else {
+                w->key[k] = o->key[k];
+            }
         }
     }
     for (uint32_t k = sub; k < r.niter; k += G) {
@@ -1086,7 +1097,7 @@ __device__ uint32_t lazy_begin(W *w, float *orig, const EpaProblem &pr, const Ep
             weird = in && !(fabsf(dist) <= kFltMax);
             k = in ? -dist : -INFINITY;
         }
-        set_normal(w, sub, n, k);
+        set_normal(w, sub, sub, n, k);
     }
     lds_order();
     if (dim == 3) {
@@ -1110,28 +1121,21 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     r.nl = uni<G>(r.nl);
     const ShapeRef ga = uni<G>(pr.a), gb = uni<G>(pr.b);
     // The live face of largest key.
-    uint32_t fid;
+    uint32_t fid, fplace;
     float fkey;
     {
         float kb = -INFINITY;
         uint32_t ib = 0;
         bool dup = false;
-        for (uint32_t i0 = sub; i0 < r.nl; i0 += 4 * G) {  // four faces' loads in flight
-            uint32_t f[4];
+        for (uint32_t i0 = sub; i0 < r.nl; i0 += 4 * G) {  // four keys' loads in flight
             float k[4];
-            uint32_t x[4];
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) f[u] = w->live[i0 + u * G < r.nl ? i0 + u * G : i0];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                k[u] = face_key(w, f[u]);
-                x[u] = W::kMask ? 0u : w->face[f[u]].px;
-            }
+            for (uint32_t u = 0; u < 4; ++u) k[u] = w->nk[i0 + u * G < r.nl ? i0 + u * G : i0][3];
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
-                const float kk = i0 + u * G >= r.nl || face_dead(w, r, f[u], x[u]) ? -INFINITY : k[u];
+                const float kk = i0 + u * G < r.nl ? k[u] : -INFINITY;
                 dup = kk > kb ? false : (kk == kb ? true : dup);
-                ib = kk > kb ? f[u] : ib;
+                ib = kk > kb ? i0 + u * G : ib;
                 kb = fmaxf(kk, kb);
             }
         }
@@ -1139,16 +1143,18 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
         if (fkey == -INFINITY) return EPA_OK;  // parry's heap is empty
         const uint64_t top = group_ballot<G>(kb == fkey);
         const uint64_t twice = group_ballot<G>(kb == fkey && dup);
-        fid = (uint32_t)__shfl((int)ib, __builtin_ctzll(top), G);
+        fplace = (uint32_t)__shfl((int)ib, __builtin_ctzll(top), G);
         if (twice != 0ull || (top & (top - 1ull)) != 0ull) {
             fid = lazy_replay(w, r);
             if (fid == kNoFace) return EPA_RESTART;
+            fplace = w->face[fid].adj[3];
         }
-        fid = uni<G>(fid);
+        fplace = uni<G>(fplace);
+        fid = uni<G>((uint32_t)w->live[fplace]);
     }
     const typename W::Face face = w->face[fid];
     const uint32_t fx = face.px;
-    const f3 fn = face_normal(w, fid);
+    const f3 fn = place_normal(w, fplace);
     const Cso c = group_cso<G, (W::kSV > 0)>(pr.pos, ga, gb, st, fn);
     const float cand = dot3(c.p, fn);
     uint32_t best_t = r.niter == 0 ? fid : r.best_id;  // the heap's first top is parry's first best face
@@ -1184,7 +1190,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 x[u] = w->face[f[u]].px;
-                fnn[u] = face_normal(w, f[u]);
+                fnn[u] = place_normal(w, u == 0 || i0 + G >= r.nl ? i0 : i0 + G);
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -1214,7 +1220,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     // (record an edge, push) is written to a spare slot, and running out of a
     // buffer ends the loop.  With branches a step took the wave about 550 cycles.
     uint32_t ns = 0, ndel = 1, depth = 2;
-    w->dl[0] = face.adj[3];
+    w->dl[0] = (I)fplace;
     uint32_t cur = walk_entry<W>(face, 0), top = walk_entry<W>(face, 1);
     w->stk[0] = (E)walk_entry<W>(face, 2);
     w->stk[1] = (E)top;
@@ -1299,7 +1305,7 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
             in = lazy_face(w, new_id, pt_at(ex, k1), pt_at(ex, k2), sp, ef, new_id + 1, new_id - 1, place, n, pa);
             w->face[ef].adj[k2] = (I)new_id;
             if (in) dist = dot3(n, pa);
-            set_normal(w, new_id, n, in ? -dist : -INFINITY);
+            set_normal(w, new_id, place, n, in ? -dist : -INFINITY);
         }
         n_alive += (uint32_t)__popcll(am);
         const bool closer = in && dist < curr_dist;
@@ -1315,7 +1321,8 @@ __device__ uint32_t lazy_step(W *w, float *orig, const EpaProblem &pr, const Sta
     }
     lds_order();
     r.nf = first_new + n_alive;
-    r.nl += n_alive > ndel ? n_alive - ndel : 0u;  // places left over keep their deleted face
+    r.nl += n_alive > ndel ? n_alive - ndel : 0u;
+    for (uint32_t k = n_alive; k < ndel; ++k) w->nk[w->dl[k]][3] = -INFINITY;  // places no new face took
     if (first_new == r.nf) return EPA_NONE;
     w->face[first_new].adj[2] = (I)(r.nf - 1);
     w->face[r.nf - 1].adj[1] = (I)first_new;
@@ -1468,21 +1475,22 @@ __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI
     }
 }
 
-// First tier: LDS for ten waves per CU, deleted flags in registers.  The odd
-// multiple of 16 bytes per polytope keeps a wave's eight polytopes off each
-// other's LDS banks.  Its
-// polytopes move on to the second tier (four pairs per wave), those to the third
-// (one wave per pair, room for parry's 100 iterations).
-using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0, 60>;
-using LazyWide = LazyState<36, 140, 36, 64, uint8_t, 0, 80>;
-using LazyWave = LazyState<112, 768, 128, 256, uint16_t, 64, 256>;
+// First tier: LDS for ten waves per CU, deleted flags in registers.  1,920 bytes per
+// polytope, no multiple of a power of two that would put a wave's eight polytopes on
+// the same LDS banks.  Its polytopes move on to the second tier (four pairs per wave,
+// ten waves per CU), those to the third (one wave per pair, seven waves per CU, room
+// for parry's 100 iterations).  A closed polytope of V vertices has 2 V - 4 faces:
+// that many places and a few more; one that needs more moves on as well.
+using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0, 39>;
+using LazyWide = LazyState<36, 132, 36, 64, uint8_t, 0, 70>;
+using LazyWave = LazyState<112, 760, 128, 256, uint16_t, 64, 208>;
 using SmallRec = EpaRec<LazySmall::kV, LazySmall::kF>;
 using WideRec = EpaRec<LazyWide::kV, LazyWide::kF>;
 
 // ---------------------------------------------------------------------------
 // Stage 3: EPA with parry's heap, one wave per pair
 // ---------------------------------------------------------------------------
-// For the pairs whose polytope outgrows the third tier (more than 768 faces) and
+// For the pairs whose polytope outgrows the third tier (more than 760 faces) and
 // those with a NaN or infinite face key: the heap itself, 2048 faces in LDS, then
 // 8192 in global memory.
 template <class I> struct EpaFaceT {
