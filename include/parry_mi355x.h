@@ -409,8 +409,9 @@ typedef struct pq_contact {
  *       tier: 64 (one wave per pair), 32, 16, 8 or 4, used when epa_schedule is 1
  *       or 2;
  *   epa_polytope: 0 to 4; the first tier's polytope has one size now (20
- *       vertices, 64 faces), and every value selects it;
- *   epa_schedule: 0 = automatic (8 lanes per pair), 1 and 2 = epa_lanes_per_pair.
+ *       vertices, 60 faces), and every value selects it;
+ *   epa_schedule: 0 = automatic (16 lanes per pair in calls of at most 16,384
+ *       pairs, else 8), 1 and 2 = epa_lanes_per_pair.
  * The default is 16 lanes per pair with polytope 1 and schedule 0. */
 typedef struct pq_contact_tuning {
     uint32_t epa_lanes_per_pair;

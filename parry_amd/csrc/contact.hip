@@ -16,8 +16,8 @@
 //     final simplex, to an EPA queue (one atomic per wave: ballot + masked
 //     popcount give each lane its slot).
 // Stage 2 (a group of lanes per queued pair): EPA (src/query/epa/epa3.rs:428-651)
-//   with the polytope in LDS, in three tiers: eight lanes per pair and 64 faces,
-//   sixteen lanes and 132 faces, a wave and 760 faces.  A pair that outgrows a
+//   with the polytope in LDS, in three tiers: eight lanes per pair and 60 faces,
+//   sixteen lanes and 132 faces, a wave and 760 faces (more lanes in small calls).  A pair that outgrows a
 //   tier's buffers goes on in the next one where it stopped.  The group's lanes
 //   share the support scans, pick the next face, test every face's visibility
 //   and build the new faces in parallel; the silhouette walk is serial.
@@ -2027,6 +2027,14 @@ constexpr uint64_t kWideGroups = 256ull * 8 * 4;
 constexpr uint64_t kWaveGroups = 256ull * 8;
 constexpr uint64_t kBigWaves = 256ull * 2;
 
+// Calls of at most this many pairs are bound by the longest chain of iterations, not
+// by instruction issue: more lanes per pair make an iteration shorter.  First tier
+// with 8 lanes and second with 16, against 16 and 64: 100 mixed pairs 212 and 188 us,
+// 500 497 and 433, 2,000 633 and 602, 10,000 857 and 818, 20,000 768 and 734, 80,000
+// 1,076 and 1,149; polyhedra 500 262 and 247, 10,000 380 and 381, 20,000 419 and 427,
+// 40,000 465 and 512.
+constexpr uint64_t kFewPairs = 16384;
+
 int g_epa_lanes_per_pair = 16;
 int g_epa_polytope = 1;
 int g_epa_schedule = 0;
@@ -2155,7 +2163,8 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
     };
     const TierArgs t0 = tier(0, w.orig_small);
     const RecSink<SmallRec> small_sink{w.small_recs, c + 10, w.small_cap};
-    const int lanes = g_epa_schedule == 0 ? 8 : g_epa_lanes_per_pair;
+    const bool few = m <= kFewPairs;
+    const int lanes = g_epa_schedule == 0 ? (few ? 16 : 8) : g_epa_lanes_per_pair;
     switch (lanes) {
         case 4: e = launch_small<4>(t0, small_sink, m, stream); break;
         case 8: e = launch_small<8>(t0, small_sink, m, stream); break;
@@ -2164,9 +2173,13 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
         default: e = launch_small<64>(t0, small_sink, m, stream); break;
     }
     if (e != hipSuccess) return e;
-    e = launch_lazy<16, LazyWide, SmallRec, WideRec, 3>(tier(1, w.orig_wide), w.small_recs,
-                                                        RecSink<WideRec>{w.wide_recs, c + 11, w.wide_cap}, m,
-                                                        kWideGroups, stream);
+    const RecSink<WideRec> wide_sink{w.wide_recs, c + 11, w.wide_cap};
+    if (few)
+        e = launch_lazy<64, LazyWide, SmallRec, WideRec, 3>(tier(1, w.orig_wide), w.small_recs, wide_sink, m,
+                                                            kWideGroups, stream);
+    else
+        e = launch_lazy<16, LazyWide, SmallRec, WideRec, 3>(tier(1, w.orig_wide), w.small_recs, wide_sink, m,
+                                                            kWideGroups, stream);
     if (e == hipSuccess) e = mark(2);
     if (e != hipSuccess) return e;
     e = launch_lazy<64, LazyWave, WideRec, WideRec, 1>(tier(2, w.orig_wave), w.wide_recs,

@@ -70,6 +70,24 @@ def test_epa_tiers_match_oracle(orc, make, types):
         print(f"  {hit.sum()} contacts, EPA iterations up to {ref['iters'][:, 1].max()}")
 
 
+@pytest.mark.parametrize("m", [16384, 16385])
+@pytest.mark.parametrize("make,types", CASES, ids=lambda v: getattr(v, "__name__", str(v)))
+def test_many_pairs_match_few(make, types, m):
+    """Up to 16,384 pairs take more lanes per pair in the first two tiers: the same records on both sides."""
+    import torch
+
+    print(f"case: {make.__name__} {types}, {m} pairs", flush=True)
+    n = 700
+    descs, verts, poses, pairs = make(types, n, 3)
+    shapes, poses = ShapeSet(descs, verts), torch.from_numpy(poses).cuda()
+    few = torch.from_numpy(pairs.view(np.int32)).cuda()
+    want, wi = contact_pairs(shapes, poses, few, 0.25, with_iters=True)
+    pick = torch.from_numpy(np.random.default_rng(4).integers(0, n, m)).cuda()
+    out, it = contact_pairs(shapes, poses, few[pick].contiguous(), 0.25, with_iters=True)
+    assert torch.equal(out.view(torch.int32), want[pick].view(torch.int32))
+    assert torch.equal(it, wi[pick])
+
+
 @pytest.mark.parametrize("m,count", [(131071, None), (131072, None), (131072, 1), (140001, 131000), (135169, 0)])
 def test_ordered_pairs_match_unordered(m, count):
     """From 131,072 pairs of several shape types on, the pairs are taken class by class: every pair's record is the
