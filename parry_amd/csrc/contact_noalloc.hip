@@ -18,7 +18,7 @@
 
 namespace {
 
-// 124.7 MiB of contact workspace covers 262,144 pairs.
+// 111.7 MiB of contact workspace covers 262,144 pairs.
 constexpr uint64_t kNoAllocMaxPairs = PQ_CONTACT_NOALLOC_MAX_PAIRS;
 constexpr size_t kScratchBytes = 128ull << 20;
 constexpr int kMaxDevices = 64;
