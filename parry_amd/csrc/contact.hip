@@ -1475,13 +1475,13 @@ __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI
     }
 }
 
-// First tier: LDS for ten waves per CU, deleted flags in registers.  1,920 bytes per
-// polytope, no multiple of a power of two that would put a wave's eight polytopes on
-// the same LDS banks.  Its polytopes move on to the second tier (four pairs per wave,
+// First tier: LDS for ten waves per CU, deleted flags in registers.  1,888 bytes per
+// polytope: an odd multiple of 32 puts a wave's eight polytopes on different LDS banks
+// (with 1,920 bytes 2^20 mixed pairs took 3.07 ms, with 1,888 3.05).  Its polytopes move on to the second tier (four pairs per wave,
 // ten waves per CU), those to the third (one wave per pair, seven waves per CU, room
 // for parry's 100 iterations).  A closed polytope of V vertices has 2 V - 4 faces:
 // that many places and a few more; one that needs more moves on as well.
-using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0, 39>;
+using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0, 37>;
 using LazyWide = LazyState<36, 132, 36, 64, uint8_t, 0, 70>;
 using LazyWave = LazyState<112, 760, 128, 256, uint16_t, 64, 208>;
 using SmallRec = EpaRec<LazySmall::kV, LazySmall::kF>;
