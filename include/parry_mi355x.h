@@ -187,6 +187,8 @@ int pq_trimesh_export_bvh(const pq_trimesh *mesh, pq_bvh_node_wide *out_host, ui
  *                              mapping is first set or tuned (at most 65535
  *                              meshes and 65536 sort ranges).
  * block_size (static, persistent, binned): lanes per workgroup, 64, 128 or 256.
+ * In small calls (static up to 65536 rays, binned up to 20480) a wave casts fewer
+ * than 64 rays.
  * stack_regs (static, persistent, binned): find_best's pending-node stack keeps
  * its top 0, 1, 2 or 4 entries in registers and the rest in LDS.
  * The queue (persistent and wave) and the sort's buffers (binned, grown to the
