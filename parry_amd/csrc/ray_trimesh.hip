@@ -394,20 +394,25 @@ __device__ __forceinline__ void write_hit(pq_ray_hit *hits, uint64_t i, const Tr
     hits[i] = make_hit(t.have, h, tri_id, ntri);
 }
 
-// Static mapping; also serves trees whose root holds a single leaf
+// Static mapping, `lanes` rays per wave if FEW, else 64; also serves trees whose root holds a single leaf
 // (bvh_traverse.rs:348-359).  COUNT = true additionally writes, per ray, the
 // number of wide-node records fetched and of triangles tested (the traffic
 // model of the roofline figure).  CULL selects the culling variant
 // (TriMesh::cast_local_ray_with_culling, ray_trimesh.rs:152-178).
-template <bool COUNT, int CULL, int BLOCK, int REG>
+template <bool COUNT, int CULL, int BLOCK, int REG, bool FEW>
 __global__ __launch_bounds__(BLOCK) void cast_rays_kernel(const pq_bvh_node_wide *__restrict__ nodes,
                                                           const TriRecord *__restrict__ tris, uint32_t ntri,
                                                           const pq_ray *__restrict__ rays, uint64_t n, float max_toi,
                                                           pq_ray_hit *__restrict__ hits,
                                                           uint32_t *__restrict__ counts,
-                                                          const uint32_t *__restrict__ order, uint32_t finite) {
+                                                          const uint32_t *__restrict__ order, uint32_t finite,
+                                                          uint32_t lanes) {
     extern __shared__ uint32_t lds_stack[];
-    const uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+    uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if constexpr (FEW) {  // a wave's first `lanes` lanes cast a ray each
+        const uint32_t lane = threadIdx.x % 64u;
+        j = lane < lanes ? j / 64u * lanes + lane : n;
+    }
     if (j >= n) return;
     const uint64_t i = order ? (uint64_t)order[j] : j;  // the binned mapping's j-th ray in sorted order
     LaneStack<BLOCK, REG> stk;
@@ -1306,6 +1311,29 @@ hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t 
     return hipGetLastError();
 }
 
+// Rays per wave of the static and binned mappings.  A wave runs a leaf test whenever
+// one of its lanes has one, so rays that share a wave slow each other down; a call too
+// small to fill the chip is faster with fewer rays in more waves.  Measured, static,
+// us a call on 5,120 and 81,920 triangles: 1,000 rays 64 a wave 54 and 93, 4 a wave 42 and
+// 68, 2 38 and 58, 1 37 and 52; 4,096 rays 48 and 96, 2 31 and 58, 1 31 and 57; 16,384
+// rays 52 and 110, 8 45 and 86, 4 40 and 78, 2 51 and 87; 40,000 rays on 1,280 and 81,920
+// triangles 41 and 116, 8 43 and 103; 65,536 rays 57 and 121, 32 54 and 110, 16 52 and
+// 112, 8 65 and 120; 131,072 rays 58 and 130, 32 61 and 130.
+// Sorted rays share their paths: 32,768 on 81,920 triangles 110 with 64 and 115 with 8.
+static uint32_t wave_rays(uint64_t n, bool sorted) {
+    if (n <= 1024) return 1;
+    if (n <= 8192) return 2;
+    if (n <= 20480) return 4;
+    if (sorted) return 64;
+    if (n <= 32768) return 8;
+    return n <= 65536 ? 32 : 64;
+}
+// Blocks of `block` lanes whose waves cast `lanes` rays each.
+static dim3 lane_grid(uint64_t n, uint32_t lanes, uint32_t block) {
+    const uint64_t waves = (n + lanes - 1) / lanes, per_block = block / 64u;
+    return dim3((uint32_t)((waves + per_block - 1) / per_block));
+}
+
 uint32_t ray_stack_entries(uint32_t depth) { return depth > 1 ? depth - 1 : 1; }
 
 // The wave mapping's stack is one VGPR (64 entries).
@@ -1316,7 +1344,6 @@ hipError_t launch_cast_rays_culling(const DeviceMesh &m, const pq_ray *rays, uin
     if (n == 0) return hipSuccess;
     constexpr int B = 256;
     const size_t lds = stack_lds_bytes(m.depth, B, 0);
-    const dim3 grid((uint32_t)((n + B - 1) / B)), block(B);
     // the mesh's binned mapping sorts these rays too; any other mapping runs static lanes
     const bool single_leaf = m.num_nodes == 1 && m.num_triangles == 1;
     const uint32_t *order = nullptr;
@@ -1324,18 +1351,29 @@ hipError_t launch_cast_rays_culling(const DeviceMesh &m, const pq_ray *rays, uin
         const hipError_t e = launch_ray_bins(m, rays, n, stream, &order);
         if (e != hipSuccess) return e;
     }
-    if (culling == 1 && counts)
-        hipLaunchKernelGGL((cast_rays_kernel<true, 1, B, 0>), grid, block, lds, stream, m.nodes, m.tris,
-                           m.num_triangles, rays, n, max_toi, hits, counts, order, m.finite);
-    else if (culling == 1)
-        hipLaunchKernelGGL((cast_rays_kernel<false, 1, B, 0>), grid, block, lds, stream, m.nodes, m.tris,
-                           m.num_triangles, rays, n, max_toi, hits, counts, order, m.finite);
-    else if (counts)
-        hipLaunchKernelGGL((cast_rays_kernel<true, 2, B, 0>), grid, block, lds, stream, m.nodes, m.tris,
-                           m.num_triangles, rays, n, max_toi, hits, counts, order, m.finite);
+    const uint32_t lanes = wave_rays(n, order != nullptr);
+    const dim3 grid = lane_grid(n, lanes, B), block(B);
+    const auto launch = [&](auto count, auto cull, auto few) {
+        hipLaunchKernelGGL((cast_rays_kernel<decltype(count)::value, decltype(cull)::value, B, 0, decltype(few)::value>),
+                           grid, block, lds, stream, m.nodes, m.tris, m.num_triangles, rays, n, max_toi, hits, counts,
+                           order, m.finite, lanes);
+    };
+    const auto pick = [&](auto cull, auto few) {
+        if (counts)
+            launch(std::true_type{}, cull, few);
+        else
+            launch(std::false_type{}, cull, few);
+    };
+    const auto cast = [&](auto cull) {
+        if (lanes < 64)
+            pick(cull, std::true_type{});
+        else
+            pick(cull, std::false_type{});
+    };
+    if (culling == 1)
+        cast(std::integral_constant<int, 1>{});
     else
-        hipLaunchKernelGGL((cast_rays_kernel<false, 2, B, 0>), grid, block, lds, stream, m.nodes, m.tris,
-                           m.num_triangles, rays, n, max_toi, hits, counts, order, m.finite);
+        cast(std::integral_constant<int, 2>{});
     return hipGetLastError();
 }
 
@@ -1383,9 +1421,15 @@ hipError_t launch_single(const DeviceMesh &m, const pq_ray *rays, uint64_t n, fl
                 const hipError_t e = launch_ray_bins(m, rays, n, stream, &order);
                 if (e != hipSuccess) return e;
             }
-            hipLaunchKernelGGL((cast_rays_kernel<COUNT, 0, B, R>), dim3((uint32_t)((n + B - 1) / B)), dim3(B), lds,
-                               stream, m.nodes, m.tris, m.num_triangles, rays, n, max_toi, hits, counts, order,
-                               m.finite);
+            const uint32_t lanes = wave_rays(n, order != nullptr);
+            if (lanes < 64)
+                hipLaunchKernelGGL((cast_rays_kernel<COUNT, 0, B, R, true>), lane_grid(n, lanes, B), dim3(B), lds,
+                                   stream, m.nodes, m.tris, m.num_triangles, rays, n, max_toi, hits, counts, order,
+                                   m.finite, lanes);
+            else
+                hipLaunchKernelGGL((cast_rays_kernel<COUNT, 0, B, R, false>), lane_grid(n, lanes, B), dim3(B), lds,
+                                   stream, m.nodes, m.tris, m.num_triangles, rays, n, max_toi, hits, counts, order,
+                                   m.finite, lanes);
         }
         return hipGetLastError();
     });
