@@ -156,11 +156,18 @@ bool boxes_nested(const pq_bvh_node_wide *nodes, uint32_t num_nodes, const float
 // within 8 u D / |edge|; either moves the point by at most 90 u D e^4 / |n|^2, if the
 // relative error of va + vb + vc, 30 u D e^3 / |n|^2, is below a quarter.  `foot` has
 // 128 in place of 90.
+// Rounding is relative to a result only where nothing under- or overflows.  A product
+// that underflows is off by 2^-149 at most: with e >= kMinEdge (D is no less than
+// 0.8 e) that moves va, vb, vc and an edge's parameter by less than a thousandth of
+// the terms above, and |n|^2 >= 2^-122 has a finite reciprocal.  Below it a mesh of
+// radius 1e-10 got wrong triangles.  No sum passes 16 D e^3, no square D^2: `reach`
+// keeps both in range.
+constexpr double kMinEdge = 0x1p-28;
 constexpr MeshBounds kNoBounds{0.0f, 0.0f, -1.0f};
 MeshBounds mesh_bounds(const float *vertices, uint32_t num_vertices, const uint32_t *indices, uint32_t num_triangles) {
     float extent = 0.0f;
     for (size_t k = 0; k < 3 * (size_t)num_vertices; ++k) extent = std::fmax(extent, std::fabs(vertices[k]));
-    double worst = 0.0, reach = 3.0e38;
+    double worst = 0.0, reach = 0x1p60;
     const double u = 1.1920929e-7 / 2;
     for (uint32_t t = 0; t < num_triangles; ++t) {
         double v[3][3], e2 = 0.0, n2 = 0.0, d[3][3], n[3];
@@ -178,10 +185,12 @@ MeshBounds mesh_bounds(const float *vertices, uint32_t num_vertices, const uint3
             n[a] = d[0][(a + 1) % 3] * d[1][(a + 2) % 3] - d[0][(a + 2) % 3] * d[1][(a + 1) % 3];
             n2 += n[a] * n[a];
         }
-        const double q = n2 / (e2 * e2);
-        if (!(q >= 1.0e-3)) return kNoBounds;  // slivers: the bound would be too wide to use
+        const double q = n2 / (e2 * e2), e = std::sqrt(e2);
+        // slivers, for which the bound would be too wide to use, and edges too short for it to hold
+        if (!(q >= 1.0e-3 && e >= kMinEdge)) return kNoBounds;
         worst = std::fmax(worst, 128.0 * u / q);
-        reach = std::fmin(reach, 0.25 * std::sqrt(e2) * q / (30.0 * u));
+        reach = std::fmin(reach, 0.25 * e * q / (30.0 * u));
+        reach = std::fmin(reach, 0x1p122 / (e * e2));
     }
     return MeshBounds{extent, (float)worst, (float)reach};
 }

@@ -68,3 +68,27 @@ def test_projection_mappings_match_oracle(orc, make, level, n):
         hit = ref["triangle"] != 0xFFFFFFFF
         assert np.array_equal(pt[hit].view(np.uint32), ref["point"][hit].view(np.uint32))
         assert np.array_equal(inside[hit].astype(np.uint32), ref["is_inside"][hit])
+
+
+def check_against_oracle(orc, v, f, p, solid=False):
+    import torch
+
+    out = TriMesh(v, f).project_local_points(torch.from_numpy(p).cuda(), solid)
+    pt, inside, tri = (x.cpu().numpy() for x in split_projections(out))
+    ref = orc.OracleTriMesh(v, f).project_points(p, solid)
+    assert np.array_equal(tri.view(np.uint32), ref["triangle"])
+    hit = ref["triangle"] != 0xFFFFFFFF
+    assert np.array_equal(pt[hit].view(np.uint32), ref["point"][hit].view(np.uint32))
+    assert np.array_equal(inside[hit].astype(np.uint32), ref["is_inside"][hit])
+
+
+@pytest.mark.parametrize("n", [16384, 17000])
+@pytest.mark.parametrize("scale", [1e-15, 1e-11, 1e-10, 3e-8, 1e-7, 1e8, 1e10, 1e15])
+def test_projection_scales_match_oracle(orc, scale, n):
+    """Edges from far below to just above the length that the projections' bound needs (products of
+    four edges underflow), and meshes whose products overflow."""
+    v, f = sphere(4)
+    v = (v.astype(np.float64) * scale).astype(np.float32)
+    p = (np.random.default_rng(n).uniform(-1.5, 1.5, (n, 3)) * scale).astype(np.float32)
+    print(f"case: scale {scale}, {n} points", flush=True)
+    check_against_oracle(orc, v, f, p)
