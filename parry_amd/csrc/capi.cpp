@@ -4,6 +4,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -60,14 +61,23 @@ hipError_t stream_queue(hipStream_t stream, unsigned long long **queue) {
     return hipSuccess;
 }
 
+namespace {
+size_t bin_words(uint64_t n, uint32_t blocks) { return (size_t)kRayBins * blocks + kRayBins + 2 * (size_t)n; }
+void carve_bins(uint32_t *base, uint64_t n, uint32_t blocks, RayBinSpace *ws) {
+    ws->hist = base;
+    ws->totals = base + (size_t)kRayBins * blocks;
+    ws->keyrank = ws->totals + kRayBins;
+    ws->order = ws->keyrank + n;
+}
+}  // namespace
+
 hipError_t ray_bin_workspace(hipStream_t stream, uint64_t num_rays, uint32_t blocks, RayBinSpace *ws) {
     static std::mutex mu;
     static std::map<std::pair<int, hipStream_t>, std::pair<uint32_t *, size_t>> spaces;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    const size_t hist_words = (size_t)kRayBins * blocks + kRayBins;
-    const size_t words = hist_words + 2 * (size_t)num_rays + 1;
+    const size_t words = bin_words(num_rays, blocks);
     std::lock_guard<std::mutex> lock(mu);
     auto &slot = spaces[std::make_pair(dev, stream)];
     if (slot.second < words) {
@@ -80,11 +90,50 @@ hipError_t ray_bin_workspace(hipStream_t stream, uint64_t num_rays, uint32_t blo
         if ((e = hipMalloc(&p, words * sizeof(uint32_t))) != hipSuccess) return e;
         slot = {(uint32_t *)p, words};
     }
-    ws->hist = slot.first;
-    ws->totals = slot.first + (size_t)kRayBins * blocks;
-    ws->keyrank = slot.first + hist_words;
-    ws->order = ws->keyrank + num_rays;
-    ws->count = ws->order + num_rays;
+    carve_bins(slot.first, num_rays, blocks, ws);
+    return hipSuccess;
+}
+
+hipError_t point_bin_workspace(hipStream_t stream, uint64_t num_points, uint32_t blocks, PointBinSpace *ws) {
+    struct Slot {
+        std::mutex mu;
+        uint32_t *base = nullptr;
+        size_t words = 0;
+    };
+    static std::mutex mu;
+    static std::map<std::pair<int, hipStream_t>, Slot> slots;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    Slot *slot = nullptr;
+    try {
+        std::lock_guard<std::mutex> lock(mu);
+        slot = &slots[std::make_pair(dev, stream)];  // stays where it is
+    } catch (const std::bad_alloc &) {
+        return hipErrorOutOfMemory;
+    }
+    std::unique_lock<std::mutex> hold(slot->mu);
+    const size_t words = bin_words(num_points, blocks) + 1;
+    if (slot->words < words) {
+        // Another stream may be in a capture, which allocating must not end.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if ((e = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return e;
+        void *p = nullptr;
+        if (slot->base) e = hipStreamSynchronize(stream);
+        if (e == hipSuccess) {
+            (void)hipFree(slot->base);
+            slot->base = nullptr;
+            slot->words = 0;
+            e = hipMalloc(&p, words * sizeof(uint32_t));
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) return e;
+        slot->base = (uint32_t *)p;
+        slot->words = words;
+    }
+    carve_bins(slot->base, num_points, blocks, ws);
+    ws->count = ws->order + num_points;
+    ws->hold = std::move(hold);
     return hipSuccess;
 }
 

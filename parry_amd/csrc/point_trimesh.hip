@@ -525,26 +525,31 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
                            (uint32_t)n, none, none, solid, m.bounds, out);
         return hipGetLastError();
     }
-    // The sort's buffers may have to grow, which a capture does not allow.
+    // The sort's buffers may have to grow, which a capture does not allow, and a
+    // per-thread stream is another stream in each thread.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(stream, &capture);
     if (e != hipSuccess) return e;
-    if (!waves || capture != hipStreamCaptureStatusNone) {
-        hipLaunchKernelGGL((project_points_kernel<false, false>), grid(n), dim3(kPtBlock), lds, stream, m.nodes, m.tris,
-                           points, n, solid, out, nullptr, none, 0u, nullptr, nullptr);
-        return hipGetLastError();
-    }
+    const bool sorted = waves && capture == hipStreamCaptureStatusNone && stream != hipStreamPerThread;
     for (uint64_t at = 0; at < n; at += kPointSortMax) {
-        const uint64_t part = n - at < kPointSortMax ? n - at : kPointSortMax;
+        const uint64_t part = sorted && n - at > kPointSortMax ? kPointSortMax : n - at;
         const float *const pts = points + 3 * at;
-        const uint32_t *order = nullptr;
-        uint32_t *heavy = nullptr, *num_heavy = nullptr;
-        if ((e = launch_point_bins(m, pts, part, stream, &order, &heavy, &num_heavy)) != hipSuccess) return e;
-        hipLaunchKernelGGL((project_points_kernel<false, true>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
-                           m.tris, pts, part, solid, out + at, nullptr, order, lane_nodes(part), heavy, num_heavy);
-        hipLaunchKernelGGL(project_points_wave_kernel, dim3(kWaveGrid), dim3(64), 0, stream, m.nodes, m.tris, pts, 0u,
-                           (const uint32_t *)heavy, (const uint32_t *)num_heavy, solid, m.bounds, out + at);
+        PointBinSpace ws{};
+        if (sorted && point_bin_workspace(stream, part, point_bin_blocks(part), &ws) == hipSuccess) {
+            if ((e = launch_point_bins(m, pts, part, stream, ws)) != hipSuccess) return e;
+            uint32_t *const heavy = ws.keyrank;  // read by the sort's last kernel only
+            hipLaunchKernelGGL((project_points_kernel<false, true>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
+                               m.tris, pts, part, solid, out + at, nullptr, ws.order, lane_nodes(part), heavy,
+                               ws.count);
+            hipLaunchKernelGGL(project_points_wave_kernel, dim3(kWaveGrid), dim3(64), 0, stream, m.nodes, m.tris, pts,
+                               0u, heavy, ws.count, solid, m.bounds, out + at);
+        } else {
+            if (sorted) (void)hipGetLastError();  // no room for the buffers: the plain walk needs none
+            hipLaunchKernelGGL((project_points_kernel<false, false>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
+                               m.tris, pts, part, solid, out + at, nullptr, none, 0u, nullptr, nullptr);
+        }
         if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (!sorted) break;
     }
     return hipSuccess;
 }

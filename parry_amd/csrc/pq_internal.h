@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -138,9 +139,18 @@ struct RayBinSpace {
     uint32_t *totals;
     uint32_t *keyrank;
     uint32_t *order;
-    uint32_t *count;
 };
 hipError_t ray_bin_workspace(hipStream_t stream, uint64_t num_rays, uint32_t blocks, RayBinSpace *ws);
+// The same for the point projections' sort, in buffers of their own: a captured graph
+// holds the rays' buffers, and a larger projection would free them under it (no graph
+// holds these: captured projections use none).  `hold` locks them until the caller
+// has queued what reads them, so calls from several threads on one stream come one
+// after the other.
+struct PointBinSpace : RayBinSpace {
+    uint32_t *count;  // a counter, zeroed by the sort
+    std::unique_lock<std::mutex> hold;
+};
+hipError_t point_bin_workspace(hipStream_t stream, uint64_t num_points, uint32_t blocks, PointBinSpace *ws);
 
 // LDS stack entries the ray kernels need for a tree of `depth` wide levels.
 uint32_t ray_stack_entries(uint32_t depth);
@@ -162,12 +172,13 @@ hipError_t launch_cast_rays_culling(const DeviceMesh &m, const pq_ray *rays, uin
                                     uint32_t culling, pq_ray_hit *hits, uint32_t *counts, hipStream_t stream);
 // Point projections onto the mesh (point_trimesh.hip); solid as in parry.
 // `counts` (nullable, device, 2 per point): wide-node records fetched, triangles tested.
-// Sorts the points by the cell of a grid over the mesh's root box: *order holds the
-// point index at each sorted position, *spare room for n indices and *count a
-// zeroed counter (buffers of the stream, valid until its next sort).
+// launch_point_bins sorts the points by the cell of a grid over the mesh's root box:
+// ws.order holds the point index at each sorted position, ws.keyrank is free for n
+// indices and *ws.count is zero.  `ws` for point_bin_blocks(n) blocks.
 constexpr uint64_t kPointSortMax = 1ull << 22;  // points of one sort (bounds its buffers)
+constexpr uint32_t point_bin_blocks(uint64_t n) { return (uint32_t)((n + kRayBinRange - 1) / kRayBinRange); }
 hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t n, hipStream_t stream,
-                             const uint32_t **order, uint32_t **spare, uint32_t **count);
+                             const PointBinSpace &ws);
 hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint64_t n, int solid,
                                  pq_point_projection *out, uint32_t *counts, hipStream_t stream);
 

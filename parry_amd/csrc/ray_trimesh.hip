@@ -1292,12 +1292,9 @@ hipError_t persistent_blocks(const void *kernel, int block, size_t lds, const pq
 }  // namespace
 
 hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t n, hipStream_t stream,
-                             const uint32_t **order, uint32_t **spare, uint32_t **count) {
+                             const PointBinSpace &ws) {
     if (n > kPointSortMax) return hipErrorInvalidValue;
-    const uint32_t blocks = (uint32_t)((n + kBinRange - 1) / kBinRange);
-    RayBinSpace ws{};
-    hipError_t e = ray_bin_workspace(stream, n, blocks, &ws);
-    if (e != hipSuccess) return e;
+    const uint32_t blocks = point_bin_blocks(n);
     hipLaunchKernelGGL(bin_count_points_kernel, dim3(blocks), dim3(kCountBlock), 0, stream, m.nodes, points, n,
                        (uint64_t)kBinRange, ws.hist, ws.keyrank, ws.count);
     hipLaunchKernelGGL(bin_scan_kernel, dim3(kRayBins / 64), dim3(64 * kScanWaves), 0, stream, ws.hist, blocks, nullptr,
@@ -1305,9 +1302,6 @@ hipError_t launch_point_bins(const DeviceMesh &m, const float *points, uint64_t 
     hipLaunchKernelGGL(bin_cells_kernel, dim3(1), dim3(kBinBlock), 0, stream, ws.totals, nullptr);
     hipLaunchKernelGGL(bin_scatter_kernel, dim3((uint32_t)((n + kBinBlock - 1) / kBinBlock)), dim3(kBinBlock), 0,
                        stream, ws.keyrank, ws.hist, ws.totals, n, (uint64_t)kBinRange, blocks, ws.order);
-    *order = ws.order;
-    *spare = ws.keyrank;  // read by the scatter only
-    *count = ws.count;
     return hipGetLastError();
 }
 
