@@ -16,7 +16,9 @@
 // closed mesh has most of the surface at nearly the same distance, and on an
 // 81,920-triangle sphere one of 262,147 points visits 8,100 nodes where the mean
 // is 134, so that the call lasted as long as that one lane's chain of fetches
-// (3.1 ms).  A lane gives up after some nodes and leaves its point to a wave.
+// (3.1 ms).  A lane leaves its point to a wave after some nodes, later where the point
+// is outside the mesh's box; if too many points are left for waves to be the faster
+// way, lanes walk them again.
 #include <cfloat>
 
 #include "contact_gjk.h"
@@ -172,8 +174,9 @@ __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, 
 // node in ten, so some lane of a wave did at nearly every node, and each node cost
 // the wave two projections (2.2 us per node, two thirds of it for them).  Up to four
 // leaves wait in registers, and the wave projects the first of every lane when one
-// lane has more than two.  Returns false if the walk passes `limit` nodes or its
-// answer is not known to be find_best's.
+// lane has more than two.  After `limit` nodes, or four times as many where `far`, a
+// lane that may leaves its point to the wave kernel: `leave` puts it in the list (and
+// returns its argument).
 //
 // The nodes are taken in find_best's order with a best cost that is late, so this
 // walk sees find_best's leaves and a few more, in its order, as long as the
@@ -182,8 +185,11 @@ __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, 
 // the first leaf W of smallest cost: each leaf before it costs more than W, so no box
 // above W costs as much as the best cost find_best has there, and nothing after W
 // costs less.
-__device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 *tri4, f3 pt, bool solid, uint32_t *stk,
-                                              uint32_t stride, uint32_t limit, PtBest &b) {
+enum : uint32_t { WALK_DONE, WALK_UNKNOWN, WALK_LEFT };  // unknown: the answer may not be find_best's
+template <class Leave>
+__device__ __forceinline__ uint32_t walk_deferred(const float4 *node4, const float4 *tri4, f3 pt, bool solid,
+                                                  uint32_t *stk, uint32_t stride, uint32_t limit, bool may, bool far,
+                                                  const Leave &leave, PtBest &b) {
     uint32_t curr = 0, sp = 0, n = 0, steps = 0;
     uint32_t l0 = 0, l1 = 0, l2 = 0, l3 = 0;
     bool walking = true, known = true;
@@ -197,6 +203,10 @@ __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 
     for (;;) {
         // A node adds two leaves at most: wave-uniform, so that the lanes keep step.
         const bool leaves = __any(n > 2u) || !__any(walking);
+        if (!leaves && (steps == limit || steps == 4u * limit)) {  // all walking lanes at once: they keep step
+            if (leave(walking && may && (!far || steps != limit))) return WALK_LEFT;
+        }
+        steps += leaves ? 0u : 1u;
         if (!leaves && walking) {
             const float4 q0 = node4[4 * (size_t)curr + 0];  // left mins, left children
             const float4 q1 = node4[4 * (size_t)curr + 1];  // left maxs, left data
@@ -219,7 +229,6 @@ __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 
             walking = !(pop & (sp == 0u));
             curr = go_near ? lc : (go_far ? rc : below);
             sp = (go_near & go_far) ? sp + 1u : (pop ? sp - 1u : sp);
-            if (++steps > limit) return false;
         }
         if (leaves) {
             if (n != 0u) {
@@ -240,7 +249,7 @@ __device__ __forceinline__ bool walk_deferred(const float4 *node4, const float4 
             if (!walking && n == 0u) break;
         }
     }
-    return known;
+    return known ? WALK_DONE : WALK_UNKNOWN;
 }
 
 // is_inside comes from the winner's triangle, projected again.
@@ -267,9 +276,35 @@ __device__ __forceinline__ f3 load_point(const float *points, uint64_t i) {
     return f3{points[3 * i], points[3 * i + 1], points[3 * i + 2]};
 }
 
+// No leaf has a cost for a point with a NaN (find_best visits the whole tree to no end).
+__device__ __forceinline__ bool any_nan(f3 p) { return p.x != p.x || p.y != p.y || p.z != p.z; }
+__device__ __forceinline__ float bound_dist(const MeshBounds &bounds, f3 p) {  // MeshBounds' |p|_1 + 3 * extent
+    return fabsf(p.x) + fabsf(p.y) + fabsf(p.z) + 3.0f * bounds.extent;
+}
+__device__ __forceinline__ bool in_root_box(const float4 *node4, f3 p) {
+    const float4 a = node4[0], b = node4[1], c = node4[2], d = node4[3];
+    const auto in = [](float l0, float l1, float h0, float h1, float v) {
+        return v >= fminf(l0, l1) && v <= fmaxf(h0, h1);
+    };
+    return in(a.x, c.x, b.x, d.x, p.x) && in(a.y, c.y, b.y, d.y, p.y) && in(a.z, c.z, b.z, d.z, p.z);
+}
+
+// The points that lanes leave to waves: a long walk ends sooner there, but takes 16 to
+// 240 ns of the whole GPU.  Beyond kHeavyMax of them lanes walk them again, without a
+// limit.  Measured with all points in a ball of radius 0.02 / 0.1 / 0.3 at the middle of
+// the 81,920-triangle unit sphere, ms a call: 130,000 points by waves 32 / 11.5 / 6.4, by
+// lanes 34 / 16.2 / 10.9; 260,000 by waves 63 / 22.4 / 12.3, by lanes 34.6 / 16.3 / 11.4; 10^6
+// 244 / 86 / 47 and 94 / 39 / 22.
+constexpr uint32_t kHeavyMax = 131072;
+struct HeavyList {
+    uint32_t *at;
+    uint32_t *count;
+};
+
 // COUNT = true also writes, per point, the wide-node records fetched and the
-// triangles tested (the traffic model of the roofline figure).  With LIMIT, points
-// whose walk exceeds `limit` nodes go to `heavy` instead (*num_heavy of them).
+// triangles tested (the traffic model of the roofline figure).  With LIMIT, long walks
+// go to `heavy` (walk_deferred), and so do points whose answer is not known to be
+// find_best's; without it, a list is walked plainly if it is too long for waves.
 template <bool COUNT, bool LIMIT>
 __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_node_wide *__restrict__ nodes,
                                                                   const TriRecord *__restrict__ tris,
@@ -277,11 +312,15 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
                                                                   int solid_flag,
                                                                   pq_point_projection *__restrict__ out,
                                                                   uint32_t *__restrict__ counts,
-                                                                  const uint32_t *__restrict__ order, uint32_t limit,
-                                                                  uint32_t *__restrict__ heavy,
-                                                                  uint32_t *__restrict__ num_heavy) {
+                                                                  const uint32_t *order, uint32_t limit,
+                                                                  MeshBounds bounds, HeavyList heavy) {
     extern __shared__ uint32_t lds_stack[];
     const uint64_t j = (uint64_t)blockIdx.x * kPtBlock + threadIdx.x;
+    if (!LIMIT && heavy.at) {
+        n = *heavy.count;
+        if (n <= kHeavyMax) return;  // the wave kernel's
+        order = heavy.at;
+    }
     if (j >= n) return;
     const uint64_t i = order ? (uint64_t)order[j] : j;
     const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
@@ -289,29 +328,36 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
     PtBest b{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};
     uint32_t n_wide = 0, n_tri = 0;
     const f3 pt = load_point(points, i);
-    bool done = true;
-    if (LIMIT)
-        done = walk_deferred(node4, tri4, pt, solid_flag != 0, lds_stack + threadIdx.x, kPtBlock, limit, b);
-    else
-        walk<COUNT>(node4, tri4, pt, solid_flag != 0, lds_stack + threadIdx.x, kPtBlock, b, n_wide, n_tri);
-    if (LIMIT) {  // one atomic per wave, by the first lane that gave up
-        const uint64_t left = __ballot(!done);
-        if (left != 0ull) {
-            const uint32_t leader = (uint32_t)__builtin_ctzll(left);
-            uint32_t base = 0;
-            if (__lane_id() == leader) base = atomicAdd(num_heavy, (uint32_t)__popcll(left));
-            base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
-            if (!done)
-                heavy[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(left >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u))] = (uint32_t)i;
+    const bool solid = solid_flag != 0;
+    uint32_t *const stk = lds_stack + threadIdx.x;
+    if constexpr (LIMIT) {
+        if (!any_nan(pt)) {
+            const auto leave = [&](bool left) {  // one atomic per wave, by the first lane that leaves
+                const uint64_t mask = __ballot(left);
+                if (mask == 0ull) return false;
+                const uint32_t leader = (uint32_t)__builtin_ctzll(mask);
+                uint32_t base = 0;
+                if (__lane_id() == leader) base = atomicAdd(heavy.count, (uint32_t)__popcll(mask));
+                base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+                if (left)
+                    heavy.at[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] =
+                        (uint32_t)i;
+                return left;
+            };
+            const bool may = bound_dist(bounds, pt) <= bounds.reach;  // a wave's lane 0 is no faster
+            const uint32_t r = walk_deferred(node4, tri4, pt, solid, stk, kPtBlock, limit, may,
+                                             !in_root_box(node4, pt), leave, b);
+            if (r == WALK_LEFT || leave(r == WALK_UNKNOWN)) return;
         }
-        if (!done) return;
+    } else {
+        walk<COUNT>(node4, tri4, pt, solid, stk, kPtBlock, b, n_wide, n_tri);
     }
     if (COUNT) {
         counts[2 * i] = n_wide;
         counts[2 * i + 1] = n_tri;
     }
-    write_projection(out, i, tri4, pt, solid_flag != 0, b);
+    write_projection(out, i, tri4, pt, solid, b);
 }
 
 // ---------------------------------------------------------------------------
@@ -326,8 +372,9 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
 // find_best reaches leaves in the order of a path key: at each node a child leaf
 // before a child node, otherwise the nearer child (the left on ties) first.  The
 // key holds one bit per level from the top, then a marker bit.  A winner whose
-// projection is outside its box, a full stack or a point out of the bound's reach
-// falls back to find_best by lane 0.
+// projection is outside its box or a full stack falls back to find_best by lane 0,
+// and so does a point out of the bound's reach unless `shared` is set: then the first
+// blocks take `shared` points each and walk those out of reach, a lane for each.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kDescentNodes = 8;
 constexpr uint32_t kWaveStack = 1024;
@@ -358,23 +405,49 @@ __device__ __forceinline__ uint32_t rank_below(uint64_t mask) {
 __global__ __launch_bounds__(64) void project_points_wave_kernel(const pq_bvh_node_wide *__restrict__ nodes,
                                                                  const TriRecord *__restrict__ tris,
                                                                  const float *__restrict__ points, uint32_t n,
-                                                                 const uint32_t *__restrict__ list,
-                                                                 const uint32_t *__restrict__ list_count,
-                                                                 int solid_flag, MeshBounds bounds,
+                                                                 HeavyList list, uint32_t shared, int solid_flag,
+                                                                 MeshBounds bounds,
                                                                  pq_point_projection *__restrict__ out) {
-    __shared__ uint32_t s_node[kWaveStack];
-    __shared__ float s_cost[kWaveStack];
-    __shared__ uint64_t s_key[kWaveStack];
+    __shared__ alignas(8) uint32_t lds[4 * kWaveStack];
+    uint32_t *const s_node = lds;
+    float *const s_cost = reinterpret_cast<float *>(lds + kWaveStack);
+    uint64_t *const s_key = reinterpret_cast<uint64_t *>(lds + 2 * kWaveStack);
     const float4 *node4 = reinterpret_cast<const float4 *>(nodes);
     const float4 *tri4 = reinterpret_cast<const float4 *>(tris);
     const bool solid = solid_flag != 0;
     const uint32_t lane = __lane_id();
-    if (list) n = *list_count;
-    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
-        const uint32_t i = list ? list[q] : q;
+    const auto plain = [&](uint32_t i, f3 pt, uint32_t lanes) {  // by one of `lanes` lanes
+        PtBest s{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};
+        uint32_t n_wide = 0, n_tri = 0;
+        walk<false>(node4, tri4, pt, solid, lds + (lanes > 1u ? lane : 0u), lanes, s, n_wide, n_tri);
+        write_projection(out, i, tri4, pt, solid, s);
+    };
+    uint32_t first = blockIdx.x;
+    if (list.at) {
+        n = *list.count;
+        if (n > kHeavyMax) return;  // project_points_kernel's
+    } else if (shared != 0u) {
+        const uint32_t blocks = (n + shared - 1u) / shared;
+        if (first < blocks) {
+            const uint32_t i = first * shared + lane;
+            if (lane < shared && i < n) {
+                const f3 pt = load_point(points, i);
+                if (!any_nan(pt) && !(bound_dist(bounds, pt) <= bounds.reach)) plain(i, pt, shared);
+            }
+            return;
+        }
+        first -= blocks;
+    }
+    for (uint32_t q = first; q < n; q += gridDim.x) {
+        const uint32_t i = list.at ? list.at[q] : q;
         const f3 pt = load_point(points, i);
-        const float d = fabsf(pt.x) + fabsf(pt.y) + fabsf(pt.z) + 3.0f * bounds.extent;
+        const float d = bound_dist(bounds, pt);
         const float slack = bounds.foot * d;
+        if (any_nan(pt)) {
+            if (lane == 0) write_projection(out, i, tri4, pt, solid, PtBest{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false});
+            continue;
+        }
+        if (shared != 0u && !(d <= bounds.reach)) continue;
         PtBest b{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};  // the lane's best
         uint64_t key = ~0ull;
         uint32_t sp = 1;
@@ -481,12 +554,7 @@ __global__ __launch_bounds__(64) void project_points_wave_kernel(const pq_bvh_no
             }
             fits = __ballot(!ok) == 0ull;
         }
-        if (!fits && lane == 0) {
-            PtBest s{FLT_MAX, f3{0.0f, 0.0f, 0.0f}, 0u, false};
-            uint32_t n_wide = 0, n_tri = 0;
-            walk<false>(node4, tri4, pt, solid, s_node, 1u, s, n_wide, n_tri);
-            write_projection(out, i, tri4, pt, solid, s);
-        }
+        if (!fits && lane == 0) plain(i, pt, 1u);
         __syncthreads();
     }
 }
@@ -499,10 +567,23 @@ constexpr uint64_t kWavePoints = 16384;
 // Nodes a lane walks before it leaves its point to a wave.  A wave spends about
 // 16 ns of the whole GPU on a point; a lane's chain costs 1.2 to 1.7 us per node, which
 // the larger calls hide better.  Measured (limit 192 / 256 / 384): 32,000 points
-// 479 / 546 / 718 us, 65,536 671 / 580 / 749, 262,147 1,425 / 786 / 894, 2^20
-// 4,910 / 2,212 / 1,892.
+// 480 / 553 / 736 us, 65,536 534 / 587 / 763, 262,147 815 / 801 / 936, 2^20
+// 2,553 / 2,203 / 1,927.
+// Points outside the mesh's box have walks of even lengths that no wave needs to cut
+// short (463 nodes at most on that sphere, from any distance): with one limit for all,
+// 260,000 points at 20 radii took 6,240 us, with four times the limit outside 704 (1,290
+// before there were waves).  Above rough ground the even limit is better: 260,000 points
+// up to ten widths high 576 and 746 (843 before).
 uint32_t lane_nodes(uint64_t n) { return n < 49152 ? 192u : (n < 524288 ? 256u : 384u); }
 constexpr uint32_t kWaveGrid = 256 * 10;  // resident waves (LDS: ten per CU)
+// Points out of reach that share a wave in a small call (0: a wave each; so many fit the
+// GPU at once).  16,000 points at 200 radii: 1,376 us with a wave each, 657 with eight to
+// a wave; 1,209 before there were waves.
+uint32_t shared_lanes(uint32_t n) {
+    if (n <= kWaveGrid) return 0u;
+    return n <= 2 * kWaveGrid ? 2u : (n <= 4 * kWaveGrid ? 4u : 8u);
+}
+static_assert(8 * kWaveMaxDepth <= 4 * kWaveStack, "the shared walks' stacks");
 
 }  // namespace
 
@@ -513,16 +594,19 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
     const size_t lds = (size_t)ray_stack_entries(m.depth) * kPtBlock * sizeof(uint32_t);
     const auto grid = [](uint64_t k) { return dim3((uint32_t)((k + kPtBlock - 1) / kPtBlock)); };
     const uint32_t *const none = nullptr;
+    const HeavyList no_list{nullptr, nullptr};
     if (counts) {
         hipLaunchKernelGGL((project_points_kernel<true, false>), grid(n), dim3(kPtBlock), lds, stream, m.nodes, m.tris,
-                           points, n, solid, out, counts, none, 0u, nullptr, nullptr);
+                           points, n, solid, out, counts, none, 0u, m.bounds, no_list);
         return hipGetLastError();
     }
     // Waves need the mesh's bound on projections, a tree their keys can hold and two leaves.
     const bool waves = m.bounds.reach >= 0.0f && m.depth <= kWaveMaxDepth && m.num_triangles > 1;
     if (waves && n <= kWavePoints) {
-        hipLaunchKernelGGL(project_points_wave_kernel, dim3((uint32_t)n), dim3(64), 0, stream, m.nodes, m.tris, points,
-                           (uint32_t)n, none, none, solid, m.bounds, out);
+        const uint32_t shared = shared_lanes((uint32_t)n);
+        const uint32_t blocks = (uint32_t)n + (shared ? ((uint32_t)n + shared - 1u) / shared : 0u);
+        hipLaunchKernelGGL(project_points_wave_kernel, dim3(blocks), dim3(64), 0, stream, m.nodes, m.tris, points,
+                           (uint32_t)n, no_list, shared, solid, m.bounds, out);
         return hipGetLastError();
     }
     // The sort's buffers may have to grow, which a capture does not allow, and a
@@ -537,16 +621,19 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
         PointBinSpace ws{};
         if (sorted && point_bin_workspace(stream, part, point_bin_blocks(part), &ws) == hipSuccess) {
             if ((e = launch_point_bins(m, pts, part, stream, ws)) != hipSuccess) return e;
-            uint32_t *const heavy = ws.keyrank;  // read by the sort's last kernel only
+            const HeavyList heavy{ws.keyrank, ws.count};  // keyrank: the sort's last kernel has read it
             hipLaunchKernelGGL((project_points_kernel<false, true>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
-                               m.tris, pts, part, solid, out + at, nullptr, ws.order, lane_nodes(part), heavy,
-                               ws.count);
+                               m.tris, pts, part, solid, out + at, nullptr, ws.order, lane_nodes(part),
+                               m.bounds, heavy);
             hipLaunchKernelGGL(project_points_wave_kernel, dim3(kWaveGrid), dim3(64), 0, stream, m.nodes, m.tris, pts,
-                               0u, heavy, ws.count, solid, m.bounds, out + at);
+                               0u, heavy, 0u, solid, m.bounds, out + at);
+            if (part > kHeavyMax)
+                hipLaunchKernelGGL((project_points_kernel<false, false>), grid(part), dim3(kPtBlock), lds, stream,
+                                   m.nodes, m.tris, pts, 0ull, solid, out + at, nullptr, none, 0u, m.bounds, heavy);
         } else {
             if (sorted) (void)hipGetLastError();  // no room for the buffers: the plain walk needs none
             hipLaunchKernelGGL((project_points_kernel<false, false>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
-                               m.tris, pts, part, solid, out + at, nullptr, none, 0u, nullptr, nullptr);
+                               m.tris, pts, part, solid, out + at, nullptr, none, 0u, m.bounds, no_list);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (!sorted) break;

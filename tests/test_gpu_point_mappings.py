@@ -92,3 +92,36 @@ def test_projection_scales_match_oracle(orc, scale, n):
     p = (np.random.default_rng(n).uniform(-1.5, 1.5, (n, 3)) * scale).astype(np.float32)
     print(f"case: scale {scale}, {n} points", flush=True)
     check_against_oracle(orc, v, f, p)
+
+
+@pytest.mark.parametrize("n", [64, 2561, 5121, 10241, 16384, 16385, 60001])
+def test_far_and_nan_points_match_oracle(orc, n):
+    """Points up to and beyond the distance that the bound on projections holds for, and points with a NaN: by a wave
+    each, several to a wave and by sorted lanes."""
+    v, f = sphere(4)
+    rng = np.random.default_rng(n)
+    p = rng.normal(size=(n, 3))
+    p *= (10.0 ** rng.choice([0.0, 0.1, 0.5, 1.0, 1.7, 2.0, 2.3, 3.0, 5.0, 10.0, 17.0], n) /
+          np.linalg.norm(p, axis=1))[:, None]
+    p = p.astype(np.float32)
+    p[rng.integers(0, n, n // 30), rng.integers(0, 3, n // 30)] = np.nan
+    print(f"case: {n} points", flush=True)
+    check_against_oracle(orc, v, f, p)
+
+
+def test_more_long_walks_than_waves_take(orc):
+    """140,000 points at the middle, all of whose walks are long: the plain walk's records (which the counted call
+    gives), and the oracle's for some of them."""
+    import torch
+
+    v, f = sphere(5)
+    p = np.random.default_rng(1).normal(0.0, 0.01, (140000, 3)).astype(np.float32)
+    d = torch.from_numpy(p).cuda()
+    mesh, counts = TriMesh(v, f), torch.zeros(140000, 2, dtype=torch.int32, device="cuda")
+    print("case: 140,000 points", flush=True)
+    got = mesh.project_local_points(d, False).view(torch.int32)
+    want = mesh.project_local_points(d, False, counts=counts).view(torch.int32)
+    assert int((counts[:, 0] > 256).sum()) > 131072
+    assert torch.equal(got, want)
+    ref = orc.OracleTriMesh(v, f).project_points(p[:2000], False)
+    assert np.array_equal(got[:2000, 4].cpu().numpy().view(np.uint32), ref["triangle"])
