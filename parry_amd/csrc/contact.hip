@@ -1416,6 +1416,9 @@ __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI
     W *const wg = &w[group];
     float *orig = t.orig + (size_t)(blockIdx.x * kGroups + group) * W::kV * kOrigFloats;
     const uint32_t count = __hip_atomic_load(t.in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // As many waves as pairs are enough; the others, and an empty tier, would wait for an
+    // atomic: updates of 60 manifolds without an overlap 46.5 us (42 without this wait).
+    if (blockIdx.x >= count) return;
     uint32_t chunk = count / (gridDim.x * 8u);  // the last chunks are an eighth of a wave's share at most
     chunk = chunk < 1u ? 1u : (chunk > 32u ? 32u : chunk);
     uint32_t at = 0, end = 0;  // the wave's reserved entries
@@ -1966,6 +1969,7 @@ __device__ uint32_t epa_step(W *w, float *orig, const iso &pos12, const ShapeRef
 template <class W>
 __device__ void epa_wave_loop(const TierArgs &t, W *w, float *orig) {
     const uint32_t count = __hip_atomic_load(t.in_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (blockIdx.x >= count) return;
     for (;;) {
         uint32_t q = 0;
         if (__lane_id() == 0) q = atomicAdd(t.next, 1u);

@@ -119,3 +119,25 @@ def test_ordered_pairs_match_unordered(m, count):
     k = m if count is None else count
     assert torch.equal(out[:k].view(torch.int32), want[pick[:k]].view(torch.int32))
     assert bool((out[k:] == -7.0).all())
+
+
+@pytest.mark.parametrize("k", [0, 1, 2, 5, 9, 33])
+def test_few_overlaps_match_oracle(orc, k):
+    """Lists shorter than a tier's waves, down to empty ones: k overlapping pairs of 40, and of 16,400."""
+    import torch
+
+    print(f"case: {k} overlapping pairs", flush=True)
+    descs, verts, poses, pairs = deep_case((2, 3), 40, 11)
+    poses[2 * k + 1::2, 4] += 50.0
+    ref = orc.contact_pairs(descs, verts, poses, pairs, 0.25)
+    shapes, d = ShapeSet(descs, verts), torch.from_numpy(poses).cuda()
+    few = torch.from_numpy(pairs.view(np.int32)).cuda()
+    out, iters = contact_pairs(shapes, d, few, 0.25, with_iters=True)
+    hit = ref["status"] == 1
+    assert hit.sum() == k and np.array_equal(out.cpu().numpy().view(np.uint32)[:, 13], ref["status"])
+    assert np.array_equal(out.cpu().numpy()[hit, :13] + 0.0, ref["out"][hit] + 0.0)
+    pick = torch.full((16400,), 39, device="cuda")
+    pick[torch.arange(40, device="cuda") * 400] = torch.arange(40, device="cuda")
+    many, it = contact_pairs(shapes, d, few[pick].contiguous(), 0.25, with_iters=True)
+    assert torch.equal(many.view(torch.int32), out.view(torch.int32)[pick])
+    assert torch.equal(it, iters[pick])
