@@ -408,12 +408,11 @@ typedef struct pq_contact {
 /* Kernel mapping of the contact path (no counterpart in parry; results are
  * identical for every setting).  Process-wide.
  *   epa_lanes_per_pair: lanes that run one pair's EPA together in the first EPA
- *       tier: 64 (one wave per pair), 32, 16, 8 or 4, used when epa_schedule is 1
- *       or 2;
- *   epa_polytope: 0 to 4; the first tier's polytope has one size now (20
- *       vertices, 60 faces), and every value selects it;
- *   epa_schedule: 0 = automatic (16 lanes per pair in calls of at most 16,384
- *       pairs, else 8), 1 and 2 = epa_lanes_per_pair.
+ *       tier: 64 (one wave per pair), 32, 16, 8 or 4;
+ *   epa_polytope: 0 to 4; the first tier's polytope has one size (20 vertices,
+ *       60 faces), and every value selects it;
+ *   epa_schedule: 0, 1 or 2; the first tier has one schedule.  0 with 16 lanes
+ *       per pair is automatic: 16 in calls of at most 16,384 pairs, else 8.
  * The default is 16 lanes per pair with polytope 1 and schedule 0. */
 typedef struct pq_contact_tuning {
     uint32_t epa_lanes_per_pair;

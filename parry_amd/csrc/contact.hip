@@ -2168,7 +2168,9 @@ hipError_t launch_contacts(const DeviceShapes &s, const float *poses, const uint
     const TierArgs t0 = tier(0, w.orig_small);
     const RecSink<SmallRec> small_sink{w.small_recs, c + 10, w.small_cap};
     const bool few = m <= kFewPairs;
-    const int lanes = g_epa_schedule == 0 ? (few ? 16 : 8) : g_epa_lanes_per_pair;
+    // 16 lanes with schedule 0, the default, is automatic; any other setting is the caller's
+    const bool automatic = g_epa_schedule == 0 && g_epa_lanes_per_pair == 16;
+    const int lanes = automatic ? (few ? 16 : 8) : g_epa_lanes_per_pair;
     switch (lanes) {
         case 4: e = launch_small<4>(t0, small_sink, m, stream); break;
         case 8: e = launch_small<8>(t0, small_sink, m, stream); break;

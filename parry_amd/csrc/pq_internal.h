@@ -287,10 +287,11 @@ size_t cast_workspace_bytes(uint64_t m);
 hipError_t launch_casts(const DeviceShapes &s, const float *poses, const float *vels, const uint32_t *pairs, uint64_t m,
                         const pq_shape_cast_options &o, pq_shape_cast_hit *out, uint32_t *iters, void *workspace,
                         hipStream_t stream);
-// Lanes that run one pair's EPA together (64, 16 or 8), set by pq_contact_set_tuning.
+// pq_contact_set_tuning: the lanes that run one pair's EPA together in the first tier (64,
+// 32, 16, 8 or 4; by the call's size if 16 with schedule 0).  The polytope has no effect.
 extern int g_epa_lanes_per_pair;
 extern int g_epa_polytope;
-extern int g_epa_schedule;  // first EPA tier: 0 = automatic, 1 or 2 = g_epa_lanes_per_pair
+extern int g_epa_schedule;
 // Phase timing of launch_contacts (pq_contact_set_phase_timing): while on, each
 // call records kContactPhases + 1 events on its stream around its phases.
 constexpr int kContactPhases = 5;  // GJK/dispatch, the two small EPA tiers, 768-face, 2048-face, global-memory tier

@@ -82,9 +82,8 @@ def test_icosphere_shapes_match_oracle(orc):
 
 
 def test_non_default_epa_tunings(orc):
-    """The mesh contact's EPA pairs (a triangle against a shape) under first-tier
-    settings other than the default: wave batches with 8 lanes per pair and the
-    64-face polytope, and the per-group refill with 32 lanes per pair."""
+    """The mesh contact's EPA pairs (a triangle against a shape) with 8 and with 32
+    lanes per pair in the first tier instead of the automatic number."""
     from parry_amd import _native
 
     v, f = scenes.noisy_icosphere(4, seed=2, radius=2.0)

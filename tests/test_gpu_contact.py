@@ -207,26 +207,27 @@ def test_ball_convex_pairs(orc):
 
 
 def test_every_epa_tuning_matches_oracle(orc):
-    """Each first-tier EPA mapping (lanes per pair x polytope buffers x schedule) gives the
-    oracle's contacts and byte-identical records, on mixed broadphase pairs and
-    on the deep-penetration set (whose long runs reach the wave-per-pair tiers)."""
+    """Each number of lanes per pair in the first EPA tier, and the automatic choice, gives the
+    oracle's contacts and byte-identical records, on more and on fewer mixed broadphase pairs
+    than the 16,384 where the automatic choice changes, and on the deep-penetration set
+    (whose long runs reach the wave-per-pair tiers)."""
     from parry_amd import _native
 
     sc = scenes.mixed_scene(40000, seed=21)
     descs, verts, poses = sc["descs"], sc["vertices"], sc["poses"]
     pairs, _ = orc.OracleBvh(orc.shape_aabbs(descs, verts, poses)).self_pairs()
     dd, dposes, dpairs = _deep_case()
-    cases = [("mixed", ShapeSet(descs, verts), descs, verts, poses, pairs, 0.01),
+    shapes = ShapeSet(descs, verts)
+    assert pairs.shape[0] > 16384 > dpairs.shape[0]
+    cases = [("mixed", shapes, descs, verts, poses, pairs, 0.01),
+             ("mixed, few", shapes, descs, verts, poses, pairs[:16384], 0.01),
              ("deep", ShapeSet(dd, np.zeros((0, 3), np.float32)), dd, np.zeros((0, 3), np.float32), dposes,
               dpairs, 10.0)]
     refs = [orc.contact_pairs(c[2], c[3], c[4], c[5], c[6]) for c in cases]
     saved = _native.get_contact_tuning()
-    first = [None, None]
+    first = [None] * len(cases)
     try:
-        settings = [(64, poly, 0) for poly in range(5)]
-        for g in (32, 16, 8, 4):
-            settings += [(g, poly, 0) for poly in range(5)] + [(g, poly, 1) for poly in range(5)] + [(g, 1, 2)]
-        settings += [(16, poly, 2) for poly in (0, 2, 3, 4)]
+        settings = [(16, 1, 0)] + [(g, 1, 1) for g in (64, 32, 16, 8, 4)] + [(g, 0, 0) for g in (64, 8)] + [(32, 4, 2)]
         for g, poly, sched in settings:
             _native.set_contact_tuning(g, poly, sched)
             for k, (label, shapes, _, _, p, pr, pred) in enumerate(cases):
