@@ -1,6 +1,7 @@
 """Small calls of the static and binned ray mappings put fewer rays in a wave: at the
 sizes where their number changes, the hits and node counts are those of a call large
-enough for full waves (cast_local_ray_and_get_normal, ray_trimesh.rs:12-130)."""
+enough for full waves, and those are the oracle's (cast_local_ray_and_get_normal,
+ray_trimesh.rs:12-130; cast_local_ray_with_culling, :152-178)."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("mapping,block", [("static", 256), ("static", 64), ("binned", 128)])
 @pytest.mark.parametrize("level", [0, 4])
-def test_few_rays_per_wave(mapping, block, level):
+def test_few_rays_per_wave(orc, mapping, block, level):
     import torch
 
     v, f = scenes.noisy_icosphere(level, 1)
@@ -22,11 +23,27 @@ def test_few_rays_per_wave(mapping, block, level):
     mesh.set_tuning("static")
     want = mesh.cast_local_rays_and_get_normal(rays, 10.0, True).view(torch.int32)
     culled = mesh.cast_local_rays_with_culling(rays, 10.0, "ignore_backfaces").view(torch.int32)
+    _, counts = mesh.cast_local_rays_counted(rays, 10.0)
+    culled_counts = torch.empty(70000, 2, dtype=torch.int32, device="cuda")
+    mesh.cast_local_rays_with_culling(rays, 10.0, "ignore_backfaces", counts=culled_counts)
+    om = orc.OracleTriMesh(v, f)
+    ref = om.cast_rays(many, 10.0, per_ray_counts=True)
+    assert np.array_equal(want[:, 4].cpu().numpy().view(np.uint32), ref["feature"])
+    assert np.array_equal(want.view(torch.float32)[:, 0].cpu().numpy(), ref["toi"])
+    assert np.array_equal(counts.cpu().numpy(), np.stack([ref["w"], ref["k"]], 1))
+    ref = om.cast_rays_with_culling(many, 10.0, 1)
+    assert np.array_equal(culled[:, 4].cpu().numpy().view(np.uint32), ref["feature"])
+    assert np.array_equal(culled_counts.sum(0).cpu().numpy(), [ref["W"], ref["K"]])
     mesh.set_tuning(mapping, block_size=block)
     for n in (1, 2, 3, 63, 1023, 1024, 1025, 8192, 8193, 20480, 20481, 32768, 32769, 65536, 65537):
         print(f"case: {mapping} {block}, level {level}, {n} rays", flush=True)
-        got = mesh.cast_local_rays_and_get_normal(rays[:n].contiguous(), 10.0, True).view(torch.int32)
+        few = rays[:n].contiguous()
+        got = mesh.cast_local_rays_and_get_normal(few, 10.0, True).view(torch.int32)
         assert torch.equal(got, want[:n])
-        got = mesh.cast_local_rays_with_culling(rays[:n].contiguous(), 10.0, "ignore_backfaces").view(torch.int32)
+        got = mesh.cast_local_rays_with_culling(few, 10.0, "ignore_backfaces").view(torch.int32)
         assert torch.equal(got, culled[:n])
+        got, c = mesh.cast_local_rays_counted(few, 10.0)
+        assert torch.equal(got.view(torch.int32), want[:n]) and torch.equal(c, counts[:n])
+        got = mesh.cast_local_rays_with_culling(few, 10.0, "ignore_backfaces", counts=c).view(torch.int32)
+        assert torch.equal(got, culled[:n]) and torch.equal(c, culled_counts[:n])
     assert np.isfinite(want.view(torch.float32).cpu().numpy()[:, 0]).any()
