@@ -319,9 +319,9 @@ __global__ void zero_count_kernel(unsigned long long *c) {
 // From this many pairs on, and with several shape types, the casts are taken class
 // by class (contact.hip's pair order): the ray cast's support functions and
 // iteration counts differ by class, and in the caller's order 13% of a wave's lanes
-// were enabled on average.  Measured, ordered and not, us a call: 8,000 pairs 866 and
-// 1,026, 64,000 1,538 and 1,603, 128,000 1,370 and 1,341, 262,144 1,665 and 1,922,
-// 1,000,000 2,594 and 3,372; 1,000 pairs 758 either way.
+// were enabled on average.  Measured, ordered and not, us a call: 64,000 pairs 1,420 and
+// 1,486, 128,000 1,290 and 1,262, 262,144 1,580 and 1,862, 1,000,000 2,500 and 3,291.
+// Below the line too (1,000 pairs 652 and 695, 8,000 760 and 878), so it could lie lower.
 constexpr uint64_t kOrderMinCasts = 8192;
 
 struct CastWorkspace {

@@ -1400,16 +1400,16 @@ struct TierArgs {
 // and the cross-lane operations of the EPA code stay within a group.
 //
 // The first tier is bound by instruction issue (counters on 2^20 mixed pairs: VALU
-// busy 87% of the kernel's SIMD cycles, 1,900 VALU instructions per trip of eight
-// pairs, nine waves per CU), the third by its longest pairs' chains of about 17,000
-// cycles per iteration.  4 lanes per pair in the first tier measured 4.18 ms on
+// busy 80% of the kernel's SIMD cycles, half of the lanes enabled, ten waves per CU; the
+// second 53%), the third by its longest pairs' chains of about 17,000
+// cycles per iteration (12%).  4 lanes per pair in the first tier measured 4.18 ms on
 // the mixed pairs against 3.37 with 8 and 3.9 with 16 (the lanes of a wave take
 // the longest walk of its pairs); the second tier with 8 lanes 3.56 against 3.32
 // with 16.
 template <int G, class W, class RI, class RO, int MINW>
 __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI *recs, RecSink<RO> sink) {
     constexpr uint32_t kGroups = 64 / G;
-        constexpr uint32_t kTurnover = kGroups > 2 ? kGroups / 2 : 1;
+    constexpr uint32_t kTurnover = kGroups > 2 ? kGroups / 2 : 1;
     __shared__ W w[kGroups];
     const uint32_t group = threadIdx.x / G;
     const uint32_t sub = __lane_id() % G;
@@ -1481,7 +1481,7 @@ __global__ __launch_bounds__(64, MINW) void epa_lazy_kernel(TierArgs t, const RI
 // First tier: LDS for ten waves per CU, deleted flags in registers.  1,888 bytes per
 // polytope: an odd multiple of 32 puts a wave's eight polytopes on different LDS banks
 // (with 1,920 bytes 2^20 mixed pairs took 3.07 ms, with 1,888 3.05).  Its polytopes move on to the second tier (four pairs per wave,
-// ten waves per CU), those to the third (one wave per pair, seven waves per CU, room
+// eight waves per CU: kWideGroups), those to the third (one wave per pair, seven waves per CU, room
 // for parry's 100 iterations).  A closed polytope of V vertices has 2 V - 4 faces:
 // that many places and a few more; one that needs more moves on as well.
 using LazySmall = LazyState<20, 60, 16, 20, uint8_t, 0, 37>;
@@ -2033,10 +2033,10 @@ constexpr uint64_t kBigWaves = 256ull * 2;
 
 // Calls of at most this many pairs are bound by the longest chain of iterations, not
 // by instruction issue: more lanes per pair make an iteration shorter.  First tier
-// with 8 lanes and second with 16, against 16 and 64: 100 mixed pairs 212 and 188 us,
-// 500 497 and 433, 2,000 633 and 602, 10,000 857 and 818, 20,000 768 and 734, 80,000
-// 1,076 and 1,149; polyhedra 500 262 and 247, 10,000 380 and 381, 20,000 419 and 427,
-// 40,000 465 and 512.
+// with 8 lanes and second with 16, against 16 and 64: 100 mixed pairs 205 and 194 us,
+// 500 493 and 435, 2,000 602 and 560, 10,000 805 and 775, 20,000 731 and 688, 32,000
+// 1,126 and 1,108, 80,000 1,048 and 1,136; polyhedra 500 251 and 233, 10,000 332 and 340,
+// 20,000 371 and 368, 32,000 384 and 398, 40,000 431 and 467.
 constexpr uint64_t kFewPairs = 16384;
 
 int g_epa_lanes_per_pair = 16;
@@ -2065,10 +2065,10 @@ struct ContactWorkspace {
 // Whether the pairs are ordered by class: where there are enough of them to fill
 // the GPU several times over (below that a call lasts as long as its longest
 // pairs, in any order) and the shapes are of several types.  Measured, ordered
-// and not, us a call: mixed types 1,313 and 1,318 at 32,000 pairs, 1,450 and 1,460
-// at 128,000, 3,770 and 4,444 at 2^20; polyhedra alone 480 and 443 at 32,000, 780
-// and 734 at 128,000 (the two ordering kernels take 20 us, and the broadphase's
-// order has its own locality).
+// and not, us a call: mixed types 1,124 and 1,126 at 32,000 pairs, 1,070 and 1,048 at
+// 80,000, 1,260 and 1,272 at 128,000, 3,028 and 3,676 at 2^20; polyhedra alone 422 and
+// 384 at 32,000, 704 and 648 at 128,000 (the two ordering kernels take 22 us at 131,072
+// pairs and 54 at 2^20, and the broadphase's order has its own locality).
 constexpr uint64_t kOrderMinPairs = 1u << 17;
 bool takes_order(const DeviceShapes &s, uint64_t m) {
     return m >= kOrderMinPairs && (s.types & (s.types - 1u)) != 0u;

@@ -294,7 +294,7 @@ extern int g_epa_polytope;
 extern int g_epa_schedule;
 // Phase timing of launch_contacts (pq_contact_set_phase_timing): while on, each
 // call records kContactPhases + 1 events on its stream around its phases.
-constexpr int kContactPhases = 5;  // GJK/dispatch, the two small EPA tiers, 768-face, 2048-face, global-memory tier
+constexpr int kContactPhases = 5;  // GJK/dispatch, the two small EPA tiers, 760-face, 2048-face, global-memory tier
 extern bool g_contact_phase_timing;
 extern hipEvent_t g_contact_phase_events[kContactPhases + 1];
 // Per-(device, stream) workspace owned by the library, grown on demand.
