@@ -174,9 +174,10 @@ __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, 
 // node in ten, so some lane of a wave did at nearly every node, and each node cost
 // the wave two projections (2.2 us per node, two thirds of it for them).  Up to four
 // leaves wait in registers, and the wave projects the first of every lane when one
-// lane has more than two.  After `limit` nodes, or four times as many where `far`, a
-// lane that may leaves its point to the wave kernel: `leave` puts it in the list (and
-// returns its argument).
+// lane has more than two.  After `limit` nodes a lane that may leaves its point to the
+// wave kernel: `leave` puts it in the list (and returns its argument).  Where `far` it
+// does so only once `few` lanes of its wave or less still walk, or after four times
+// `limit`.
 //
 // The nodes are taken in find_best's order with a best cost that is late, so this
 // walk sees find_best's leaves and a few more, in its order, as long as the
@@ -188,9 +189,9 @@ __device__ __forceinline__ bool point_in_box(const float4 *tri4, uint32_t leaf, 
 enum : uint32_t { WALK_DONE, WALK_UNKNOWN, WALK_LEFT };  // unknown: the answer may not be find_best's
 template <class Leave>
 __device__ __forceinline__ uint32_t walk_deferred(const float4 *node4, const float4 *tri4, f3 pt, bool solid,
-                                                  uint32_t *stk, uint32_t stride, uint32_t limit, bool may, bool far,
-                                                  const Leave &leave, PtBest &b) {
-    uint32_t curr = 0, sp = 0, n = 0, steps = 0;
+                                                  uint32_t *stk, uint32_t stride, uint32_t limit, int few, bool may,
+                                                  bool far, const Leave &leave, PtBest &b) {
+    uint32_t curr = 0, sp = 0, n = 0, steps = 0, check = limit;
     uint32_t l0 = 0, l1 = 0, l2 = 0, l3 = 0;
     bool walking = true, known = true;
     auto put = [&](bool add, uint32_t leaf) {
@@ -203,8 +204,10 @@ __device__ __forceinline__ uint32_t walk_deferred(const float4 *node4, const flo
     for (;;) {
         // A node adds two leaves at most: wave-uniform, so that the lanes keep step.
         const bool leaves = __any(n > 2u) || !__any(walking);
-        if (!leaves && (steps == limit || steps == 4u * limit)) {  // all walking lanes at once: they keep step
-            if (leave(walking && may && (!far || steps != limit))) return WALK_LEFT;
+        if (!leaves && steps == check) {  // all walking lanes at once: they keep step
+            check += limit / 2u;
+            const bool late = __popcll(__ballot(walking)) <= few || steps >= 4u * limit;
+            if (leave(walking && may && (!far || late))) return WALK_LEFT;
         }
         steps += leaves ? 0u : 1u;
         if (!leaves && walking) {
@@ -296,6 +299,9 @@ __device__ __forceinline__ bool in_root_box(const float4 *node4, f3 p) {
 // lanes 34 / 16.2 / 10.9; 260,000 by waves 63 / 22.4 / 12.3, by lanes 34.6 / 16.3 / 11.4; 10^6
 // 244 / 86 / 47 and 94 / 39 / 22.
 constexpr uint32_t kHeavyMax = 131072;
+// Farther out than this share of the bound's reach the slack keeps a wave from pruning:
+// 260,000 points at 120 radii of that sphere 1,830 us, 720 if they stay with their lanes.
+constexpr float kWaveReach = 0.25f;
 struct HeavyList {
     uint32_t *at;
     uint32_t *count;
@@ -313,7 +319,7 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
                                                                   pq_point_projection *__restrict__ out,
                                                                   uint32_t *__restrict__ counts,
                                                                   const uint32_t *order, uint32_t limit,
-                                                                  MeshBounds bounds, HeavyList heavy) {
+                                                                  int few, MeshBounds bounds, HeavyList heavy) {
     extern __shared__ uint32_t lds_stack[];
     const uint64_t j = (uint64_t)blockIdx.x * kPtBlock + threadIdx.x;
     if (!LIMIT && heavy.at) {
@@ -345,8 +351,8 @@ __global__ __launch_bounds__(kPtBlock) void project_points_kernel(const pq_bvh_n
                         (uint32_t)i;
                 return left;
             };
-            const bool may = bound_dist(bounds, pt) <= bounds.reach;  // a wave's lane 0 is no faster
-            const uint32_t r = walk_deferred(node4, tri4, pt, solid, stk, kPtBlock, limit, may,
+            const bool may = bound_dist(bounds, pt) <= kWaveReach * bounds.reach;
+            const uint32_t r = walk_deferred(node4, tri4, pt, solid, stk, kPtBlock, limit, few, may,
                                              !in_root_box(node4, pt), leave, b);
             if (r == WALK_LEFT || leave(r == WALK_UNKNOWN)) return;
         }
@@ -569,12 +575,15 @@ constexpr uint64_t kWavePoints = 16384;
 // the larger calls hide better.  Measured (limit 192 / 256 / 384): 32,000 points
 // 480 / 553 / 736 us, 65,536 534 / 587 / 763, 262,147 815 / 801 / 936, 2^20
 // 2,553 / 2,203 / 1,927.
-// Points outside the mesh's box have walks of even lengths that no wave needs to cut
-// short (463 nodes at most on that sphere, from any distance): with one limit for all,
-// 260,000 points at 20 radii took 6,240 us, with four times the limit outside 704 (1,290
-// before there were waves).  Above rough ground the even limit is better: 260,000 points
-// up to ten widths high 576 and 746 (843 before).
 uint32_t lane_nodes(uint64_t n) { return n < 49152 ? 192u : (n < 524288 ? 256u : 384u); }
+// Points outside the mesh's box often have walks of even lengths, which no wave needs to
+// cut short (463 nodes at most on that sphere, from any distance): they leave when this
+// many lanes of their wave or less still walk.  Measured, us a call, with no such points
+// kept back / with 8 / 24 / 40 / only after four times the limit: 260,000 points at 3
+// radii 1,158 / 596 / 909 / 1,141 / 507, at 20 6,250 / 931 / 997 / 1,731 / 702, up to ten widths
+// above rough ground 576 / 562 / 559 / 559 / 745; 20,000 at 3 radii 579 / 425 / 417 / 454 / 387,
+// up to ten widths high 356 / 400 / 357 / 351 / 531, up to one 390 / 692 / 497 / 478 / 696.
+int few_lanes(uint64_t n) { return n <= 131072 ? 24 : 8; }
 constexpr uint32_t kWaveGrid = 256 * 10;  // resident waves (LDS: ten per CU)
 // Points out of reach that share a wave in a small call (0: a wave each; so many fit the
 // GPU at once).  16,000 points at 200 radii: 1,376 us with a wave each, 657 with eight to
@@ -597,7 +606,7 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
     const HeavyList no_list{nullptr, nullptr};
     if (counts) {
         hipLaunchKernelGGL((project_points_kernel<true, false>), grid(n), dim3(kPtBlock), lds, stream, m.nodes, m.tris,
-                           points, n, solid, out, counts, none, 0u, m.bounds, no_list);
+                           points, n, solid, out, counts, none, 0u, 0, m.bounds, no_list);
         return hipGetLastError();
     }
     // Waves need the mesh's bound on projections, a tree their keys can hold and two leaves.
@@ -624,16 +633,16 @@ hipError_t launch_project_points(const DeviceMesh &m, const float *points, uint6
             const HeavyList heavy{ws.keyrank, ws.count};  // keyrank: the sort's last kernel has read it
             hipLaunchKernelGGL((project_points_kernel<false, true>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
                                m.tris, pts, part, solid, out + at, nullptr, ws.order, lane_nodes(part),
-                               m.bounds, heavy);
+                               few_lanes(part), m.bounds, heavy);
             hipLaunchKernelGGL(project_points_wave_kernel, dim3(kWaveGrid), dim3(64), 0, stream, m.nodes, m.tris, pts,
                                0u, heavy, 0u, solid, m.bounds, out + at);
             if (part > kHeavyMax)
                 hipLaunchKernelGGL((project_points_kernel<false, false>), grid(part), dim3(kPtBlock), lds, stream,
-                                   m.nodes, m.tris, pts, 0ull, solid, out + at, nullptr, none, 0u, m.bounds, heavy);
+                                   m.nodes, m.tris, pts, 0ull, solid, out + at, nullptr, none, 0u, 0, m.bounds, heavy);
         } else {
             if (sorted) (void)hipGetLastError();  // no room for the buffers: the plain walk needs none
             hipLaunchKernelGGL((project_points_kernel<false, false>), grid(part), dim3(kPtBlock), lds, stream, m.nodes,
-                               m.tris, pts, part, solid, out + at, nullptr, none, 0u, m.bounds, no_list);
+                               m.tris, pts, part, solid, out + at, nullptr, none, 0u, 0, m.bounds, no_list);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (!sorted) break;
